@@ -17,13 +17,13 @@
 //    instead of 8-byte gathers with stride lda;
 //  * Toledo-style recursion on column halves puts the flops into large MFMA
 //    GEMMs (At22 -= At21*At12) and one right-side unit-upper TRSM;
-//  * leaves of 32 columns are factored by one cooperative kernel: each
-//    workgroup keeps 512 rows x 32 columns of the panel in registers, the
-//    per-column pivot search is a wavefront max-reduction (ties -> lowest
-//    row), then one grid barrier per column exchanges the per-workgroup
-//    candidates (value, row index and the whole 32-wide candidate row), so
-//    every workgroup applies the interchange, scaling and rank-1 update to
-//    its own rows without a second barrier;
+//  * leaves of 32 columns are factored by one cooperative kernel
+//    (lu_panel3.h; the two kernels below for taller panels): each workgroup
+//    keeps 512 rows x 32 columns of the panel in registers, the per-column
+//    pivot search is a wavefront max-reduction (ties -> lowest row), then one
+//    exchange per column hands the per-workgroup candidates (value, row index
+//    and the whole candidate row) to every workgroup, which applies the
+//    interchange, scaling and rank-1 update to its own rows;
 //  * an extra row of At carries the original row numbers through every
 //    interchange, which yields the composed permutation for the solves.
 #include "kernels.h"
@@ -963,6 +963,8 @@ __global__ __launch_bounds__(L2_NT) void lu_panel2_kernel(T* __restrict__ At, lo
   }
 }
 
+#include "lu_panel3.h"
+
 // Apply a panel's interchanges to the columns of A in [lo, hi) outside
 // [ex_lo, ex_hi), i.e. to those rows of At: the moves (destination position,
 // source row, both relative to the panel's first row j0) form a permutation
@@ -1082,6 +1084,8 @@ struct LuCtx {
   int* moves;          // LU_MV ints per panel: a count and up to 2*LU_W pairs
   long panel_no = 0;
   unsigned long long* rec;   // candidate records (LuRec)
+  unsigned long long* rec3;  // two areas of L3Rec records, used in turn
+  long panel3_no = 0;
   unsigned base = 0;
   unsigned* err;
   long sw_lo = 0, sw_hi = 0;     // At rows (columns of A) the leaf interchanges go to at once
@@ -1092,12 +1096,12 @@ struct LuCtx {
 // rows per thread of lu_panel2_kernel
 constexpr int L2_RPT = 2;
 
-// Which panel kernel factors a leaf.  The first form (512-thread workgroups,
-// one row per thread) is the faster one up to its LU_PMAX workgroups (65536
-// rows): measured at N=16384 the FP32 factorization takes ~4.5 us per
-// column with it against ~6.2 us with the second form.  Taller panels take
-// the second form (256-thread workgroups, two rows per thread, up to
-// L2_PMAX workgroups).  OPENBLAS_AMD_LU_PANEL=2 forces the second form.
+// Which panel kernel factors a leaf: lu_panel3_kernel up to L3_PMAX
+// workgroups (16384 rows), then lu_panel_kernel (512-thread workgroups, one
+// row per thread, up to LU_PMAX of them: 65536 rows; ~4.5 us per column at
+// 16384 rows against ~6.2 us of lu_panel2_kernel and ~2.8 of
+// lu_panel3_kernel, FP32), then lu_panel2_kernel (two rows per thread, up to
+// L2_PMAX workgroups).  OPENBLAS_AMD_LU_PANEL=2 forces the last.
 static bool lu_force_panel2() {
   static const bool v = [] {
     const char* e = getenv("OPENBLAS_AMD_LU_PANEL");
@@ -1118,7 +1122,7 @@ static long lu_capacity(K kernel, int threads) {
   return (long)std::max(per_cu, 0) * rt().num_cu;
 }
 
-// The panel kernel for a leaf of mp rows (1: first form, 2: second form, 0:
+// The panel kernel for a leaf of mp rows (1, 2, 3: lu_panel[23]_kernel, 0:
 // none can hold it resident) and its workgroup count *P.
 template <typename T>
 static int lu_panel_form(long mp, long* P) {
@@ -1127,7 +1131,9 @@ static int lu_panel_form(long mp, long* P) {
   constexpr long ROWS1 = (long)NT * RPT, ROWS2 = (long)L2_NT * L2_RPT;
   static const long cap1 = std::min<long>(LU_PMAX, lu_capacity(lu_panel_kernel<T, LU_W, RPT, NT>, NT));
   static const long cap2 = std::min<long>(L2_PMAX, lu_capacity(lu_panel2_kernel<T, LU_W, L2_RPT>, L2_NT));
-  const long P1 = (mp + ROWS1 - 1) / ROWS1, P2 = (mp + ROWS2 - 1) / ROWS2;
+  static const long cap3 = std::min<long>(L3_PMAX, lu_capacity(lu_panel3_kernel<T, LU_W, true>, L3_NT));
+  const long P1 = (mp + ROWS1 - 1) / ROWS1, P2 = (mp + ROWS2 - 1) / ROWS2, P3 = (mp + L3_ROWS - 1) / L3_ROWS;
+  if (!lu_force_panel2() && P3 <= cap3) { *P = P3; return 3; }
   if (!lu_force_panel2() && P1 <= cap1) { *P = P1; return 1; }
   if (P2 <= cap2) { *P = P2; return 2; }
   *P = 0;
@@ -1139,6 +1145,7 @@ static void lu_panel(LuCtx<T>& c, long j0, int w, bool pre = false) {
   const long mp = c.m - j0;
   int* mv = c.moves + c.panel_no * LU_MV;
   long P;
+  int form;
   // algorithmic work of the leaf: per column j, (mp-1-j) multipliers and a
   // rank-1 update of (mp-1-j) x (w-1-j); with `pre`, the node's W x w solve
   // and the mp x w x W update; bytes: the panel read and written once
@@ -1148,8 +1155,18 @@ static void lu_panel(LuCtx<T>& c, long j0, int w, bool pre = false) {
   if (pre) lf += (double)LU_W * LU_W * w + 2.0 * mp * LU_W * w;
   {
   KTimer kt("lu_panel", c.s, lf, (double)sizeof(T) * mp * (2.0 * w + (pre ? LU_W : 0)));
-  const int form = lu_panel_form<T>(mp, &P);
-  if (form == 1) {
+  form = lu_panel_form<T>(mp, &P);
+  if (form == 3) {
+    unsigned long long* r0 = c.rec3 + (c.panel3_no & 1) * L3Rec<T>::AREA;
+    unsigned long long* r1 = c.rec3 + (~c.panel3_no & 1) * L3Rec<T>::AREA;
+    if (P > 1)
+      lu_panel3_kernel<T, LU_W, true><<<(unsigned)P, L3_NT, 0, c.s>>>(c.At, c.ldt, c.m, j0, w, c.ipiv, c.info, mv, r0,
+                                                                      r1, c.err, pre ? 1 : 0);
+    else
+      lu_panel3_kernel<T, LU_W, false><<<1, L3_NT, 0, c.s>>>(c.At, c.ldt, c.m, j0, w, c.ipiv, c.info, mv, r0, r1,
+                                                             c.err, pre ? 1 : 0);
+    c.panel3_no++;
+  } else if (form == 1) {
     lu_panel_kernel<T, LU_W, LuRpt<T>::v, LuNt<T>::v><<<(unsigned)P, LuNt<T>::v, 0, c.s>>>(
         c.At, c.ldt, c.m, j0, w, c.ipiv, c.info, mv, c.rec, c.base, c.err, pre ? 1 : 0);
   } else if (form == 2) {
@@ -1160,7 +1177,7 @@ static void lu_panel(LuCtx<T>& c, long j0, int w, bool pre = false) {
   }
   OBA_HIP(hipGetLastError());
   }
-  if (P > 1) c.base += (unsigned)w;   // record tags of this panel: base+1 .. base+w
+  if (form != 3 && P > 1) c.base += (unsigned)w;   // record tags of this panel: base+1 .. base+w
   c.panel_no++;
   c.leaves.push_back(LuLeaf{j0, mv});
   lu_swap<T>(c.At, c.ldt, c.sw_lo, c.sw_hi, j0, j0 + w, j0, mp, mv, c.s);
@@ -1291,7 +1308,8 @@ int getrf_t(long m, long n, T* At, long ldt, int* ipiv_dev, bool track_perm, hip
   const long npanels = (mn + LU_W - 1) / LU_W + 1;
   const size_t rec_bytes = sizeof(unsigned long long) * LuRec<T, LU_W>::RW * 2 * std::max(LU_PMAX, L2_PMAX);
   const size_t mv_bytes = sizeof(int) * npanels * LU_MV;
-  DevBuf ws(4096 + rec_bytes + mv_bytes);
+  const size_t rec3_bytes = sizeof(unsigned long long) * 2 * L3Rec<T>::AREA;
+  DevBuf ws(4096 + rec_bytes + mv_bytes + 256 + rec3_bytes);
   char* p = ws.as<char>();
   LuCtx<T> c;
   c.At = At; c.ldt = ldt; c.m = m; c.nrows_t = n + (track_perm ? 1 : 0); c.ipiv = ipiv_dev; c.s = s;
@@ -1299,7 +1317,9 @@ int getrf_t(long m, long n, T* At, long ldt, int* ipiv_dev, bool track_perm, hip
   c.err = (unsigned*)(p + 64);
   c.rec = (unsigned long long*)(p + 4096);
   c.moves = (int*)(p + 4096 + rec_bytes);
+  c.rec3 = (unsigned long long*)(p + 4096 + rec_bytes + (mv_bytes + 255) / 256 * 256);
   OBA_HIP(hipMemsetAsync(p, 0, 4096 + rec_bytes + mv_bytes, s));
+  OBA_HIP(hipMemsetAsync(c.rec3, 0xff, rec3_bytes, s));   // L3_EMPTY
   if (track_perm) {
     iota_row_kernel<T><<<(unsigned)((m + 255) / 256), 256, 0, s>>>(At + n, m, ldt);
     OBA_HIP(hipGetLastError());
