@@ -9,10 +9,9 @@
 // Design (MI355X, not the GotoBLAS 5-loop): one workgroup of 4 wavefronts
 // owns a BM x BN tile of C held in MFMA accumulators; K advances in BK slabs
 // that are loaded from HBM with 16-byte vector loads into registers one slab
-// ahead and staged through a double-buffered k-major LDS tile (padded so the
-// fragment reads are bank-conflict free).  The MFMA is issued with op(B) as
-// its first operand so that the 16 consecutive lanes of an output row map to
-// 16 consecutive rows of column-major C (128-byte coalesced stores).  Tiles
+// ahead and staged through a double-buffered k-major LDS tile.  The MFMA is
+// issued with op(B) as its first operand, and a lane's fragments are
+// consecutive rows, so 16 lanes store 16 x 16 bytes of one column of C.  Tiles
 // are mapped XCD-aware: the 8 XCDs each get a contiguous, grouped block of C
 // tiles so that the panels of A and B they share stay in their own L2.
 #include "kernels.h"
@@ -41,34 +40,34 @@ template <> struct MF<float> {
   __device__ static inline int orow(int l, int r) { return 4 * (l >> 4) + r; }
 };
 
-template <typename T> struct Vec16;
-template <> struct Vec16<double> { typedef double2 type; static constexpr int n = 2; };
-template <> struct Vec16<float> { typedef float4 type; static constexpr int n = 4; };
+// A vector of V elements at an element-aligned (not 16-byte-aligned) address:
+// global loads and stores of 16 bytes only need 4-byte alignment, so odd
+// leading dimensions and tiles that start anywhere use the same wide accesses
+// (with per-element loads 2047 x 3001 x 1501 FP64 took 606 us).
+template <typename T, int V> struct UVec { typedef T type __attribute__((ext_vector_type(V), aligned(sizeof(T)))); };
+template <typename T, int V> struct AVec { typedef T type __attribute__((ext_vector_type(V))); };
 
 // Loads one BK-deep slab of an operand tile (TILE along m or n) into
 // registers.  KC: the operand is contiguous along k in memory (Trans A /
-// NoTrans B).  VEC: 16-byte vector loads are legal (aligned base and ld).
-// The slab is staged k-major in LDS, s[BK][TILE + PAD] (PAD: 128 bytes of
-// doubles, 64 of floats, so that the four 16-lane rows of one fragment read
-// do not start in the same bank).
-template <typename T, int TILE, int BK, bool KC, bool VEC>
+// NoTrans B).  The slab is staged k-major in LDS, s[BK][TILE + 4]: a lane
+// reads V consecutive m (n) of one k with one 16-byte read, and the padding
+// spreads the k-strided writes of a KC operand over the banks.
+template <typename T, int TILE, int BK, bool KC>
 struct TileLoader {
-  static constexpr int V = VEC ? Vec16<T>::n : 1;
+  static constexpr int V = 16 / sizeof(T);
   static constexpr int NV = TILE * BK / V / 256;  // vectors per thread
   static_assert(NV * V * 256 == TILE * BK, "tile must divide over 256 threads");
-  static constexpr int PAD = 64 / sizeof(T) * (sizeof(T) == 8 ? 2 : 1);  // 16 doubles / 16 floats
-  static constexpr int LD = TILE + PAD;
+  static constexpr int LD = TILE + 4;
   static constexpr int SIZE = BK * LD;   // elements per buffer
-  __device__ static inline int at(int k, int mn) { return k * LD + mn; }
-  T r[NV * V];
+  typedef typename AVec<T, V>::type vec;
+  vec r[NV];
 
-  // GUARD: per-element bounds checks (edge tiles, K tail); otherwise the
-  // caller guarantees the whole slab is in range and the loads are
-  // unconditional 16-byte vector loads.
-  template <bool GUARD>
+  // FULL: the whole slab is in range.  Otherwise rows past MN repeat the last
+  // one (their results are never stored) and k past K gives zeros; the
+  // addresses are clamped, so no load is predicated.
+  template <bool FULL>
   __device__ inline void load(const T* __restrict__ g, long ld, long mn0, long k0, long MN, long K) {
     const int tid = threadIdx.x & 255;   // thread within its 256-thread group
-    constexpr bool full = !GUARD;
 #pragma unroll
     for (int i = 0; i < NV; i++) {
       const int v = tid + i * 256;
@@ -76,25 +75,21 @@ struct TileLoader {
       if (!KC) { k = v / (TILE / V); mn = (v % (TILE / V)) * V; }
       else { mn = v / (BK / V); k = (v % (BK / V)) * V; }
       mn += mn0; k += k0;
-      if (full) {
-        if constexpr (V > 1) {
-          const T* p = KC ? g + k + mn * ld : g + mn + k * ld;
-          typedef typename Vec16<T>::type vt;
-          vt x = *(const vt*)p;
-          const T* xs = (const T*)&x;
-#pragma unroll
-          for (int e = 0; e < V; e++) r[i * V + e] = xs[e];
-        } else {
-          r[i] = KC ? g[k + mn * ld] : g[mn + k * ld];
-        }
+      if constexpr (FULL) {
+        r[i] = *(const typename UVec<T, V>::type*)(KC ? g + k + mn * ld : g + mn + k * ld);
       } else {
 #pragma unroll
         for (int e = 0; e < V; e++) {
-          long mm = KC ? mn : mn + e, kk = KC ? k + e : k;
-          r[i * V + e] = (mm < MN && kk < K) ? g[KC ? kk + mm * ld : mm + kk * ld] : T(0);
+          const long mm = min(KC ? mn : mn + e, MN - 1), kk = KC ? k + e : k, kc = min(kk, K - 1);
+          const T x = g[KC ? kc + mm * ld : mm + kc * ld];
+          r[i][e] = kk < K ? x : T(0);
         }
       }
     }
+  }
+  __device__ inline void zero() {
+#pragma unroll
+    for (int i = 0; i < NV; i++) r[i] = vec{};
   }
   // writes the slab into its LDS buffer (layout above)
   __device__ inline void store(T* s) const {
@@ -103,21 +98,12 @@ struct TileLoader {
     for (int i = 0; i < NV; i++) {
       const int v = tid + i * 256;
       if (!KC) {
-        int k = v / (TILE / V), mn = (v % (TILE / V)) * V;
-        if constexpr (V > 1) {
-          typedef typename Vec16<T>::type vt;
-          vt x;
-          T* xs = (T*)&x;
-#pragma unroll
-          for (int e = 0; e < V; e++) xs[e] = r[i * V + e];
-          *(vt*)(s + at(k, mn)) = x;
-        } else {
-          s[at(k, mn)] = r[i];
-        }
+        const int k = v / (TILE / V), mn = (v % (TILE / V)) * V;
+        *(vec*)(s + k * LD + mn) = r[i];
       } else {
-        int mn = v / (BK / V), k = (v % (BK / V)) * V;
+        const int mn = v / (BK / V), k = (v % (BK / V)) * V;
 #pragma unroll
-        for (int e = 0; e < V; e++) s[at(k + e, mn)] = r[i * V + e];
+        for (int e = 0; e < V; e++) s[(k + e) * LD + mn] = r[i][e];
       }
     }
   }
@@ -129,8 +115,8 @@ struct TileLoader {
 // order 0..KS-1 before the epilogue (one launch, no workspace, the same
 // result on every run).  It fills a CU with one workgroup when there are
 // only about as many tiles as CUs.
-template <typename T, int BM, int BN, int BK, bool TA, bool TB, bool VEC, int KS = 1>
-__global__ __launch_bounds__(256 * KS, KS == 1 ? 2 : 1) void gemm_kernel(long M, long N, long K, T alpha,
+template <typename T, int BM, int BN, int BK, bool TA, bool TB, int KS, int OCC>
+__global__ __launch_bounds__(256 * KS, OCC) void gemm_kernel(long M, long N, long K, T alpha,
                                                       const T* __restrict__ A, long lda,
                                                       const T* __restrict__ B, long ldb, T beta,
                                                       T* __restrict__ C, long ldc, int tiles_m,
@@ -145,23 +131,27 @@ __global__ __launch_bounds__(256 * KS, KS == 1 ? 2 : 1) void gemm_kernel(long M,
     K = min(kc, K - y * kc);
     C += y * cstride;
   }
-  typedef TileLoader<T, BM, BK, TA, VEC> LA;
-  typedef TileLoader<T, BN, BK, !TB, VEC> LB;
+  typedef TileLoader<T, BM, BK, TA> LA;
+  typedef TileLoader<T, BN, BK, !TB> LB;
+  constexpr int V = LA::V;
   constexpr int WTM = BM / 2, WTN = BN / 2;  // 2x2 waves
   constexpr int FM = WTM / 16, FN = WTN / 16;
+  // fragment i of a wave's tile holds rows PM*(lane%16) + i%PM of the
+  // i/PM-th group of 16*PM rows, so one LDS read feeds PM fragments and a
+  // lane's outputs are PM consecutive rows of C (likewise PN columns of B)
+  constexpr int PM = FM < V ? FM : V, PN = FN < V ? FN : V;
   typedef MF<T> mf;
   typedef typename mf::acc acc_t;
 
   constexpr int STAGE = 2 * (LA::SIZE + LB::SIZE);   // one group's double-buffered slabs
   constexpr int SMEM = KS == 1 ? STAGE : (KS * STAGE > KS * BM * BN ? KS * STAGE : KS * BM * BN);
-  __shared__ T smem[SMEM];
+  __shared__ __attribute__((aligned(16))) T smem[SMEM];
   const int grp = KS == 1 ? 0 : (int)(threadIdx.x >> 8);
   // buffer b of the A slab at st + b*LA::SIZE, of the B slab after both A's
   T* const st = smem + grp * STAGE;
 #define OBA_AS(b) (st + (b) * LA::SIZE)
 #define OBA_BS(b) (st + 2 * LA::SIZE + (b) * LB::SIZE)
   long kg = 0;   // sliced K: the groups' common k-range length, a multiple of BK
-  const long k_total = K;
   if (KS > 1) {
     kg = ((K + KS - 1) / KS + BK - 1) / BK * BK;
     A += grp * kg * (TA ? 1 : lda);
@@ -181,10 +171,14 @@ __global__ __launch_bounds__(256 * KS, KS == 1 ? 2 : 1) void gemm_kernel(long M,
   const int in_group = lin - group * GM * tiles_n;
   const int tm = first_m + in_group % gsize;
   const int tn = in_group / gsize;
-  const long m0 = (long)tm * BM, n0 = (long)tn * BN;
+  // the tile owns C rows [mt, mt+BM) and columns [nt, nt+BN); an edge tile
+  // reads from m0 = M-BM (n0 = N-BN) instead, where every load is in range,
+  // recomputing rows of its neighbour that it does not store
+  const long mt = (long)tm * BM, nt = (long)tn * BN;
+  const long m0 = M >= BM ? min(mt, M - BM) : 0, n0 = N >= BN ? min(nt, N - BN) : 0;
   // tri: 1 = update only C(i,j) with i >= j (lower), 2 = only i <= j (upper)
-  if (tri == 1 && n0 > m0 + BM - 1) return;
-  if (tri == 2 && m0 > n0 + BN - 1) return;
+  if (tri == 1 && nt > mt + BM - 1) return;
+  if (tri == 2 && mt > nt + BN - 1) return;
   if (abort_flag && *abort_flag) return;
 
   const int lane = threadIdx.x & 63;
@@ -194,81 +188,114 @@ __global__ __launch_bounds__(256 * KS, KS == 1 ? 2 : 1) void gemm_kernel(long M,
   LA la;
   LB lb;
 
-  acc_t acc[FM][FN];
+  // a wave with a single fragment runs its k steps through 4 accumulators in
+  // turn: independent MFMAs instead of one dependent chain, and shorter sums
+  constexpr int NA = FM * FN == 1 ? 4 : 1;
+  acc_t accs[NA][FM][FN];
 #pragma unroll
-  for (int i = 0; i < FM; i++)
+  for (int q = 0; q < NA; q++)
 #pragma unroll
-    for (int j = 0; j < FN; j++) acc[i][j] = acc_t{};
+    for (int i = 0; i < FM; i++)
+#pragma unroll
+      for (int j = 0; j < FN; j++) accs[q][i][j] = acc_t{};
+  auto& acc = accs[0];
 
-  // compute one staged slab: BK/4 MFMA k-steps on the wave's FM x FN tiles
-  auto compute = [&](int buf) __attribute__((always_inline)) {
-    const T* as = OBA_AS(buf);
-    const T* bs = OBA_BS(buf);
+  // A slab's fragments are read from LDS into registers one slab ahead, so
+  // the reads run behind the MFMAs of the slab before instead of in front of
+  // their own.
+  struct Frags {
+    T a[BK / 4][FM], b[BK / 4][FN];
+  };
+  Frags f0, f1;
+  auto read = [&](int buf, Frags& f) __attribute__((always_inline)) {
+    const T* as = OBA_AS(buf) + wm0;
+    const T* bs = OBA_BS(buf) + wn0;
 #pragma unroll
     for (int kk = 0; kk < BK / 4; kk++) {
       const int kr = kk * 4 + (lane >> 4);
-      T fa[FM], fb[FN];
 #pragma unroll
-      for (int i = 0; i < FM; i++) fa[i] = as[LA::at(kr, wm0 + i * 16 + (lane & 15))];
+      for (int i = 0; i < FM; i += PM)
+        *(typename AVec<T, PM>::type*)&f.a[kk][i] =
+            *(const typename AVec<T, PM>::type*)&as[kr * LA::LD + i * 16 + PM * (lane & 15)];
 #pragma unroll
-      for (int j = 0; j < FN; j++) fb[j] = bs[LB::at(kr, wn0 + j * 16 + (lane & 15))];
+      for (int j = 0; j < FN; j += PN)
+        *(typename AVec<T, PN>::type*)&f.b[kk][j] =
+            *(const typename AVec<T, PN>::type*)&bs[kr * LB::LD + j * 16 + PN * (lane & 15)];
+    }
+  };
+  auto mma = [&](const Frags& f) __attribute__((always_inline)) {
+#pragma unroll
+    for (int kk = 0; kk < BK / 4; kk++)
 #pragma unroll
       for (int i = 0; i < FM; i++)
 #pragma unroll
-        for (int j = 0; j < FN; j++) acc[i][j] = mf::mma(fb[j], fa[i], acc[i][j]);
-    }
+        for (int j = 0; j < FN; j++)
+          accs[kk % NA][i][j] = mf::mma(f.b[kk][j], f.a[kk][i], accs[kk % NA][i][j]);
   };
-  // Full slabs run with unconditional loads on interior tiles (no control
-  // flow around the prefetch, so its loads stay in flight across the MFMAs);
-  // the K tail and edge tiles use guarded loads.
-  // With sliced K every group runs the same kg/BK slabs (the same barriers);
-  // a group whose range ends early loads zeros through the guarded loads.
-  auto run = [&](auto guard_tag) __attribute__((always_inline)) {
-    constexpr bool G = decltype(guard_tag)::value;
-    const int nkf = KS > 1 ? (int)(kg / BK) : (int)(K / BK);
-    const bool tail = KS == 1 && (K % BK) != 0;
-    if (nkf == 0) {
-      la.template load<true>(A, lda, m0, 0, M, K);
-      lb.template load<true>(B, ldb, n0, 0, N, K);
-      la.store(OBA_AS(0));
-      lb.store(OBA_BS(0));
-      __syncthreads();
-      compute(0);
+  // A slab that lies in range is loaded unconditionally; the K tail (and
+  // every slab of an operand narrower than the tile) through clamped
+  // addresses; with sliced K a group past its range's end multiplies zeros,
+  // so that all groups meet the same barriers.
+  const bool fit_a = M >= BM, fit_b = N >= BN, fits = fit_a && fit_b;
+  auto fetch = [&](long k0) __attribute__((always_inline)) {
+    if (k0 >= K) {
+      la.zero();
+      lb.zero();
       return;
     }
-    la.template load<G>(A, lda, m0, 0, M, K);
-    lb.template load<G>(B, ldb, n0, 0, N, K);
-    la.store(OBA_AS(0));
-    lb.store(OBA_BS(0));
-    __syncthreads();
-    for (int kt = 0; kt < nkf - 1; kt++) {
-      const int cur = kt & 1;
-      la.template load<G>(A, lda, m0, (long)(kt + 1) * BK, M, K);
-      lb.template load<G>(B, ldb, n0, (long)(kt + 1) * BK, N, K);
-      compute(cur);
-      la.store(OBA_AS(cur ^ 1));
-      lb.store(OBA_BS(cur ^ 1));
-      __syncthreads();
-    }
-    const int last = (nkf - 1) & 1;
-    if (tail) {
-      la.template load<true>(A, lda, m0, (long)nkf * BK, M, K);
-      lb.template load<true>(B, ldb, n0, (long)nkf * BK, N, K);
-    }
-    compute(last);
-    if (tail) {
-      la.store(OBA_AS(last ^ 1));
-      lb.store(OBA_BS(last ^ 1));
-      __syncthreads();
-      compute(last ^ 1);
-    }
+    const bool in = k0 + BK <= K;
+    if (fit_a && in) la.template load<true>(A, lda, m0, k0, M, K);
+    else la.template load<false>(A, lda, m0, k0, M, K);
+    if (fit_b && in) lb.template load<true>(B, ldb, n0, k0, N, K);
+    else lb.template load<false>(B, ldb, n0, k0, N, K);
   };
-  // Unguarded loads on interior tiles; with sliced K also only when every
-  // group's range is full (K_total == KS*kg), so that the choice, and with
-  // it the barrier sequence, is the same for the whole workgroup.
-  const bool interior = (m0 + BM <= M) && (n0 + BN <= N) && (KS == 1 || k_total == KS * kg);
-  if (interior) run(std::false_type{});
-  else run(std::true_type{});
+  auto stage = [&](int buf) __attribute__((always_inline)) {
+    la.store(OBA_AS(buf));
+    lb.store(OBA_BS(buf));
+  };
+  const int nk = KS > 1 ? (int)(kg / BK) : (int)((K + BK - 1) / BK);
+  const int nfull = fits ? (int)(K / BK) : 0;   // leading slabs that lie in range
+  fetch(0);
+  stage(0);
+  fetch(BK);
+  __syncthreads();
+  read(0, f0);
+  int kt = 0;
+  // one step: slab kt+1 from registers to LDS, slab kt+2 from memory to
+  // registers, slab kt+1's fragments read while slab kt is multiplied.  No
+  // control flow around the loads of a slab in range, so that they stay in
+  // flight across the MFMAs.
+  auto step = [&](auto full_tag, int buf, Frags& cur, Frags& next) __attribute__((always_inline)) {
+    stage(buf);
+    if constexpr (decltype(full_tag)::value) {
+      la.template load<true>(A, lda, m0, (long)(kt + 2) * BK, M, K);
+      lb.template load<true>(B, ldb, n0, (long)(kt + 2) * BK, N, K);
+    } else {
+      fetch((long)(kt + 2) * BK);
+    }
+    __syncthreads();
+    read(buf, next);
+    mma(cur);
+    kt++;
+  };
+  while (kt + 3 < nfull) {
+    step(std::true_type{}, 1, f0, f1);
+    step(std::true_type{}, 0, f1, f0);
+  }
+  while (kt + 2 < nk) {
+    step(std::false_type{}, 1, f0, f1);
+    step(std::false_type{}, 0, f1, f0);
+  }
+  if (kt + 1 < nk) {   // kt is even: slab kt in f0, slab kt+1 in registers
+    stage(1);
+    __syncthreads();
+    read(1, f1);
+    mma(f0);
+    mma(f1);
+  } else if (kt < nk) {
+    mma(f0);
+  }
+  if constexpr (NA == 4) acc[0][0] = (acc[0][0] + accs[1][0][0]) + (accs[2][0][0] + accs[3][0][0]);
 
 #undef OBA_AS
 #undef OBA_BS
@@ -279,37 +306,78 @@ __global__ __launch_bounds__(256 * KS, KS == 1 ? 2 : 1) void gemm_kernel(long M,
     __syncthreads();
     T* pt = smem + grp * BM * BN;
 #pragma unroll
-    for (int i = 0; i < FM; i++)
+    for (int i = 0; i < FM; i += PM)
 #pragma unroll
       for (int j = 0; j < FN; j++)
 #pragma unroll
-        for (int r = 0; r < 4; r++)
-          pt[(wn0 + j * 16 + mf::orow(lane, r)) * BM + wm0 + i * 16 + (lane & 15)] = acc[i][j][r];
+        for (int r = 0; r < 4; r++) {
+          typename AVec<T, PM>::type v;
+#pragma unroll
+          for (int e = 0; e < PM; e++) v[e] = acc[i + e][j][r];
+          const int n = wn0 + (j / PN) * 16 * PN + PN * mf::orow(lane, r) + j % PN;
+          *(typename AVec<T, PM>::type*)&pt[n * BM + wm0 + i * 16 + PM * (lane & 15)] = v;
+        }
     __syncthreads();
+    typedef typename AVec<T, V>::type vec;
 #pragma unroll
-    for (int e = threadIdx.x; e < BM * BN; e += 256 * KS) {
-      const long m = m0 + e % BM, n = n0 + e / BM;
-      T sum = smem[e];
+    for (int e0 = threadIdx.x * V; e0 < BM * BN; e0 += 256 * KS * V) {
+      const long m = m0 + e0 % BM, n = n0 + e0 / BM;
+      vec sum = *(const vec*)&smem[e0];
 #pragma unroll
-      for (int g = 1; g < KS; g++) sum += smem[g * BM * BN + e];
-      if (m < M && n < N) {
-        T* p = C + m + n * ldc;
-        T v = alpha * sum;
-        if (!bz) v += beta * *p;
-        *p = v;
+      for (int g = 1; g < KS; g++) sum += *(const vec*)&smem[g * BM * BN + e0];
+      if (n >= N || n < nt) continue;
+      T* p = C + m + n * ldc;
+#pragma unroll
+      for (int e = 0; e < V; e++) {
+        const long i = m + e;
+        if (i < M && i >= mt && !(tri == 1 && n > i) && !(tri == 2 && i > n)) {
+          T v = alpha * sum[e];
+          if (!bz) v += beta * p[e];
+          p[e] = v;
+        }
+      }
+    }
+    return;
+  }
+  // a tile whose every element is its own to write: PM rows per store
+  const bool whole = m0 == mt && n0 == nt && fits && (tri == 0 || (tri == 1 ? m0 >= n0 + BN - 1 : m0 + BM - 1 <= n0));
+  typedef typename UVec<T, PM>::type uvec;
+  if (whole) {
+#pragma unroll
+    for (int i = 0; i < FM; i += PM) {
+      T* const pc = C + m0 + wm0 + i * 16 + PM * (lane & 15) + (n0 + wn0) * ldc;
+#pragma unroll
+      for (int j = 0; j < FN; j++) {
+        uvec old[4];
+        T* p[4];
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          p[r] = pc + ((j / PN) * 16 * PN + PN * mf::orow(lane, r) + j % PN) * ldc;
+          if (!bz) old[r] = *(const uvec*)p[r];
+        }
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          uvec v;
+#pragma unroll
+          for (int e = 0; e < PM; e++) {
+            v[e] = alpha * acc[i + e][j][r];
+            if (!bz) v[e] += beta * old[r][e];
+          }
+          *(uvec*)p[r] = v;
+        }
       }
     }
     return;
   }
 #pragma unroll
   for (int i = 0; i < FM; i++) {
-    const long m = m0 + wm0 + i * 16 + (lane & 15);
+    const long m = m0 + wm0 + (i / PM) * 16 * PM + PM * (lane & 15) + i % PM;
 #pragma unroll
     for (int j = 0; j < FN; j++) {
 #pragma unroll
       for (int r = 0; r < 4; r++) {
-        const long n = n0 + wn0 + j * 16 + mf::orow(lane, r);
-        if (m < M && n < N && !(tri == 1 && n > m) && !(tri == 2 && m > n)) {
+        const long n = n0 + wn0 + (j / PN) * 16 * PN + PN * mf::orow(lane, r) + j % PN;
+        if (m >= mt && n >= nt && m < M && n < N && !(tri == 1 && n > m) && !(tri == 2 && m > n)) {
           T* p = C + m + n * ldc;
           T v = alpha * acc[i][j][r];
           if (!bz) v += beta * *p;
@@ -421,7 +489,7 @@ static void gemm_skinny(long m, long k, T alpha, const T* a, long lda, const T* 
   OBA_HIP(hipGetLastError());
 }
 
-template <typename T, int BM, int BN, int BK, bool VEC, int KS = 1>
+template <typename T, int BM, int BN, int BK, int KS = 1, int OCC = 1>
 static void launch_cfg(bool ta, bool tb, long M, long N, long K, T alpha, const T* A, long lda,
                        const T* B, long ldb, T beta, T* C, long ldc, hipStream_t s, int tri,
                        const int* abort_flag, int ksplit = 1, long kc = 0, long cstride = 0) {
@@ -429,7 +497,7 @@ static void launch_cfg(bool ta, bool tb, long M, long N, long K, T alpha, const 
   if (tm * tn > 0x7fffffffL) fatal("gemm: grid too large", nullptr);
   dim3 grid((unsigned)(tm * tn), (unsigned)ksplit), block(256 * KS);
 #define OBA_GEMM_L(TA_, TB_) \
-  gemm_kernel<T, BM, BN, BK, TA_, TB_, VEC, KS><<<grid, block, 0, s>>>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, (int)tm, (int)tn, tri, abort_flag, kc, cstride)
+  gemm_kernel<T, BM, BN, BK, TA_, TB_, KS, OCC><<<grid, block, 0, s>>>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, (int)tm, (int)tn, tri, abort_flag, kc, cstride)
   if (!ta && !tb) OBA_GEMM_L(false, false);
   else if (!ta && tb) OBA_GEMM_L(false, true);
   else if (ta && !tb) OBA_GEMM_L(true, false);
@@ -475,60 +543,69 @@ void gemm(bool ta, bool tb, long m, long n, long k, T alpha, const T* a, long ld
       default: gemm_skinny<T, 4>(m, k, alpha, a, lda, b, ldb, beta, c, ldc, s); return;
     }
   }
-  constexpr int V = Vec16<T>::n;
-  const bool vec = (lda % V == 0) && (ldb % V == 0) && (((uintptr_t)a & 15) == 0) && (((uintptr_t)b & 15) == 0);
-  const long big_tiles = ((m + 127) / 128) * ((n + 127) / 128);
-  const bool small = big_tiles < rt().num_cu;
-  // k-slab depths from a sweep on MI355X (8192^3): shallow slabs keep the
-  // LDS footprint small and the MFMA pipe fed (FP64 128x128: BK 16 -> 4 is
-  // 60.6 -> 66.0 TF/s; FP32 BK 32 -> 8 is 118.5 -> 134.8 TF/s); the tile
-  // loaders need TILE*BK >= 256 vectors of 16 bytes
-  constexpr int BK_BIG = sizeof(T) == 8 ? 4 : 8;
-  constexpr int BK_SMALL = sizeof(T) == 8 ? 8 : 16;
-  const long tiles64 = ((m + 63) / 64) * ((n + 63) / 64);
-  const bool sliced_deep = k >= 1024 && 8 * tiles64 >= 7 * rt().num_cu && tiles64 <= rt().num_cu;
-  // few tiles and a moderate K (no split-K path below 1024): the four wave
-  // groups per tile hide each other's latencies (the recursive TRSM's
-  // updates, 256..512 x n x 256..512)
-  const bool sliced_mid = k >= 256 && k < 1024 && 2 * tiles64 <= rt().num_cu;
-  if (small && tri == 0 && abort_flag == nullptr && (sliced_deep || sliced_mid)) {
-    // about one 64x64 tile per CU, deep K: one workgroup of 4 wave groups per
-    // tile, each group a quarter of K, partials summed in LDS (4 wavefronts
-    // per SIMD instead of 1; no workspace, so any stream).  MI355X, 1024^3:
-    // DGEMM 68.7 -> 59.5 us, SGEMM 47.4 -> 40.3 us per call against the
-    // split across workgroups; with 192 tiles the split is still ahead.
-    if (vec) launch_cfg<T, 64, 64, BK_SMALL, true, 4>(ta, tb, m, n, k, alpha, a, lda, b, ldb, beta, c, ldc, s, 0, nullptr);
-    else launch_cfg<T, 64, 64, BK_SMALL, false, 4>(ta, tb, m, n, k, alpha, a, lda, b, ldb, beta, c, ldc, s, 0, nullptr);
-    return;
-  }
-  if (ws_ok && small && tri == 0 && abort_flag == nullptr && k >= 1024 && tiles64 <= rt().num_cu) {
-    // fewer tiles than half the CUs, deep K: split K across workgroups so
-    // that ~4 of them per CU hide each other's latencies
-    const int ks = (int)std::min<long>({8L, std::max<long>(1L, 4L * rt().num_cu / tiles64), k / 256});
-    if (ks > 1) {
-      const long kc = ((k + ks - 1) / ks + 15) / 16 * 16;
+  // Tile, slab and K slicing by how many tiles there are per CU.  MI355X, us
+  // per synchronous call (launch and completion about 10 us of it), NN unless
+  // said; the last column is the kernel before this table (128x128 or 64x64
+  // tiles, per-element loads at odd leading dimensions, fragments read in
+  // front of their own MFMAs):
+  //   FP64            64x64x8 KS1  KS2  64x32x16 KS2  32x32x16 KS1  KS2   before
+  //   8192^3                15009  15300        16224         17668  18713  16400
+  //   2047x3001x1501 TN       320    327          370           430    488    617
+  //   4096x1024x4096          496    497          529           588    623    925
+  //   2048x1024x2048          152    138          146           162    171    190
+  //   256x5000x5000           346    303          258           263    258
+  //   1024^3                   59     54           52            57     60     52
+  //   512x1024x512             35     32           24            25     25     33
+  //   512^3                    35     32           24            22     20     33
+  //   64^3                   15.6   16.3         14.8          14.2   14.0   17.7
+  // An FP64 MFMA takes 64 cycles, so a 64x64 tile hides its loads once a CU
+  // holds several workgroups; with two tiles per CU or fewer a second wave
+  // group per tile does that, and fewer tiles than CUs want smaller ones.
+  constexpr bool D = sizeof(T) == 8;
+  const long cu = rt().num_cu;
+  const long m64 = (m + 63) / 64, t64 = m64 * ((n + 63) / 64), t6432 = m64 * ((n + 31) / 32);
+  const long t32 = ((m + 31) / 32) * ((n + 31) / 32);
+  constexpr int BK32 = D ? 16 : 32, BK64 = D ? 8 : 16;
+#define OBA_GEMM_ARGS ta, tb, m, n, k, alpha, a, lda, b, ldb, beta, c, ldc, s, tri, abort_flag
+  if (8 * t64 < 7 * cu) {
+    // a deep K of few tiles is split over workgroups too (256x256x8192 FP64:
+    // 95 us with four groups in one workgroup, 33 in 16 parts)
+    const long parts_w = std::min<long>({8L, cu / std::max(t32, 1L), k / 512});
+    if (ws_ok && tri == 0 && abort_flag == nullptr && k >= 1024 && parts_w > 1) {
+      const long kc = ((k + parts_w - 1) / parts_w + 15) / 16 * 16;
       const int parts = (int)((k + kc - 1) / kc);
       DevBuf w(sizeof(T) * (size_t)parts * m * n);
-      if (vec)
-        launch_cfg<T, 64, 64, BK_SMALL, true>(ta, tb, m, n, k, alpha, a, lda, b, ldb, T(0), w.as<T>(), m, s, 0, nullptr,
-                                              parts, kc, m * n);
-      else
-        launch_cfg<T, 64, 64, BK_SMALL, false>(ta, tb, m, n, k, alpha, a, lda, b, ldb, T(0), w.as<T>(), m, s, 0,
-                                               nullptr, parts, kc, m * n);
+      launch_cfg<T, 32, 32, BK32, 4, 2>(ta, tb, m, n, k, alpha, a, lda, b, ldb, T(0), w.as<T>(), m, s, 0, nullptr,
+                                        parts, kc, m * n);
       const long total = m * n;
       gemm_ksum_kernel<T><<<(unsigned)std::min<long>((total + 255) / 256, 4096), 256, 0, s>>>(m, n, parts, w.as<T>(),
                                                                                              beta, c, ldc);
       OBA_HIP(hipGetLastError());
       return;
     }
+    if (k >= 1024 && t32 <= cu) launch_cfg<T, 32, 32, BK32, 4, 2>(OBA_GEMM_ARGS);
+    else if (k >= 1024 || (D && k >= 256 && t32 <= 2 * cu)) launch_cfg<T, 32, 32, BK32, 2, 2>(OBA_GEMM_ARGS);
+    else launch_cfg<T, 32, 32, BK32, 1, 4>(OBA_GEMM_ARGS);
+    return;
   }
-  if (small) {
-    if (vec) launch_cfg<T, 64, 64, BK_SMALL, true>(ta, tb, m, n, k, alpha, a, lda, b, ldb, beta, c, ldc, s, tri, abort_flag);
-    else launch_cfg<T, 64, 64, BK_SMALL, false>(ta, tb, m, n, k, alpha, a, lda, b, ldb, beta, c, ldc, s, tri, abort_flag);
-  } else {
-    if (vec) launch_cfg<T, 128, 128, BK_BIG, true>(ta, tb, m, n, k, alpha, a, lda, b, ldb, beta, c, ldc, s, tri, abort_flag);
-    else launch_cfg<T, 128, 128, BK_BIG, false>(ta, tb, m, n, k, alpha, a, lda, b, ldb, beta, c, ldc, s, tri, abort_flag);
+  if (D && t64 <= 4 * cu && k >= 256) {
+    // the narrower tile where 64x64 ones would fill their last round of CUs
+    // worse (316 tiles on 256 CUs: 303 us, 632 half tiles: 258), or there is
+    // one per CU
+    auto fill = [cu](long t) { return (double)t / (double)((t + cu - 1) / cu * cu); };
+    if (t64 <= cu || 0.95 * fill(t6432) > fill(t64)) {
+      if (t64 <= 2 * cu) launch_cfg<T, 64, 32, BK32, 2, 2>(OBA_GEMM_ARGS);
+      else launch_cfg<T, 64, 32, BK32, 1, 4>(OBA_GEMM_ARGS);
+      return;
+    }
   }
+  // FP32 (16-cycle steps) needs the LDS reuse of 128x128 tiles once there are
+  // enough of them: 8192^3 7883 us against 8414 with 64x64; 3000^3 574 / 468
+  const long t128 = ((m + 127) / 128) * ((n + 127) / 128);
+  if (t64 <= 2 * cu && k >= 256) launch_cfg<T, 64, 64, BK64, 2, 2>(OBA_GEMM_ARGS);
+  else if (!D && t128 >= 8 * cu) launch_cfg<T, 128, 128, 16, 1, 2>(OBA_GEMM_ARGS);
+  else launch_cfg<T, 64, 64, BK64, 1, 4>(OBA_GEMM_ARGS);
+#undef OBA_GEMM_ARGS
 }
 
 template void gemm<double>(bool, bool, long, long, long, double, const double*, long, const double*, long, double, double*, long, hipStream_t, int, const int*);
