@@ -11,9 +11,8 @@
 // leaves (up to 256 rows) are solved by wavefronts of right-hand-side
 // vectors: lane i owns x_i and row i of the current 64x64 tile of the
 // triangle, and x_k is broadcast with v_readlane after it is final (forward
-// or backward column-oriented substitution).  Right-side leaves multiply by
-// explicit inverses of the 64x64 diagonal blocks, or solve rows of B (the
-// transposed system) one row per lane.
+// or backward column-oriented substitution).  Right-side leaves (up to 256
+// columns) multiply by explicit inverses of the 64x64 diagonal blocks.
 #include "kernels.h"
 
 namespace oba {
@@ -259,62 +258,10 @@ __global__ __launch_bounds__(256) void trsm_leafb_kernel(int nb, long nvec, cons
     }
 }
 
-// Right-side leaves: the vectors are rows of B (contiguous across vectors,
-// stride ldb along a vector), so one lane owns one whole vector in
-// registers and the loads/stores of a wavefront are coalesced; the triangle
-// is read from LDS as broadcasts.
-template <typename T>
-__global__ __launch_bounds__(256) void trsm_leaf_rows_kernel(int nb, long nvec, const T* __restrict__ A, long lda,
-                                                             T* __restrict__ B, long ldb, bool eT, bool elower,
-                                                             bool unit, const int* abort_flag) {
-  constexpr int LDE = TRSM_NB + 2;
-  __shared__ T Ec[TRSM_NB * LDE];      // E(c,k) at Ec[k*LDE + c]: column k contiguous
-  __shared__ T dinv[TRSM_NB];
-  if (abort_flag && *abort_flag) return;
-  for (int idx = threadIdx.x; idx < TRSM_NB * TRSM_NB; idx += blockDim.x) {
-    const int f = idx & 63, s = idx >> 6;   // A(f, s), f contiguous
-    const int c = eT ? s : f, k = eT ? f : s;
-    T v = T(0);
-    if (f < nb && s < nb) v = A[f + (long)s * lda];
-    Ec[k * LDE + c] = v;
-  }
-  __syncthreads();
-  if (threadIdx.x < TRSM_NB) {
-    const int k = threadIdx.x;
-    dinv[k] = (k < nb && !unit) ? T(1) / Ec[k * LDE + k] : T(1);
-  }
-  __syncthreads();
-  const long v = blockIdx.x * (long)blockDim.x + threadIdx.x;
-  if (v >= nvec) return;
-  T x[TRSM_NB];
-#pragma unroll
-  for (int c = 0; c < TRSM_NB; c++) x[c] = (c < nb) ? B[v + c * ldb] : T(0);
-  // column-oriented substitution: x_k is final, then an independent axpy
-  // over the remaining entries (ILP instead of a dependent dot product)
-  if (elower) {
-#pragma unroll
-    for (int k = 0; k < TRSM_NB; k++) {
-      x[k] *= dinv[k];
-#pragma unroll
-      for (int c = k + 1; c < TRSM_NB; c++) x[c] -= Ec[k * LDE + c] * x[k];
-    }
-  } else {
-#pragma unroll
-    for (int k = TRSM_NB - 1; k >= 0; k--) {
-      x[k] *= dinv[k];
-#pragma unroll
-      for (int c = 0; c < k; c++) x[c] -= Ec[k * LDE + c] * x[k];
-    }
-  }
-#pragma unroll
-  for (int c = 0; c < TRSM_NB; c++)
-    if (c < nb) B[v + c * ldb] = x[c];
-}
-
 // Right-side leaves through explicit inverses of the 64x64 diagonal blocks:
 // a fully unrolled per-row substitution is ~4000 straight-line instructions
 // run once per wavefront and measured at 40-65 us per leaf whatever its
-// size (instruction fetch); the two loop-based kernels below replace it.
+// size (instruction fetch); the two kernels below replace it.
 //
 // (1) One workgroup per diagonal block b of M = op(A) (upper or lower,
 //     unit or not) computes M_bb^{-1} by doubling: the four 16x16 diagonal
@@ -433,53 +380,129 @@ __global__ __launch_bounds__(256) void trsm_inv_diag_kernel(long na, const T* __
   }
 }
 
-// (2) X <- X * M_bb^{-1} for the leaf's nb columns of B, in place: a
-//     workgroup stages 64 rows x nb columns of B and the inverse in LDS;
-//     wavefront w computes columns 16w..16w+15 of all 64 rows (the inverse
-//     row is a broadcast read, the B column a contiguous one).
-template <typename T>
-__global__ __launch_bounds__(256) void trsm_right_inv_kernel(int nb, long nvec, const T* __restrict__ inv,
-                                                             T* __restrict__ B, long ldb, const int* abort_flag) {
-  constexpr int LDX = TRSM_NB + 1;
-  __shared__ T Xs[TRSM_NB * LDX];                              // X(r, k) at Xs[k*LDX + r]
-  __shared__ __attribute__((aligned(16))) T Ys[TRSM_NB * TRSM_NB];   // inverse, row-major
+// (2) One launch solves X M = B for up to TRSM_RN columns, in place: a
+//     workgroup owns RB rows of B in LDS and takes the 64-column blocks in
+//     dependency order, X_b = (B_b - sum_k X_k M_kb) M_bb^{-1}, both products
+//     on the matrix cores (wavefront w: columns 16w..16w+15 of the block).
+//     The tiles of M and of the inverses come straight from L2 as fragments,
+//     the next tile's loads in flight behind the current one's MFMAs; step s
+//     of a product takes k = 16*(lane/16) + s, so a lane's 16 elements of M
+//     are consecutive in memory where M's columns are.  Rows never meet, so
+//     there is no exchange between workgroups; the bound is the chain of tile
+//     products (10 of them and 8 barriers at 256 columns).  A call with the
+//     inversion and ~10 us of launch, against the recursion of 64-column
+//     multiplies and GEMMs (2 N/64 - 1 launches) that this replaced: 64 x 256
+//     FP64 90.0 -> 41.6 us, FP32 73.5 -> 35.2; 16000 x 256 116 -> 72, 83 -> 50;
+//     4000 x 2000 1056 -> 461, 739 -> 322.
+constexpr int TRSM_RN = 256;
+
+template <typename T> struct TrMf;
+template <> struct TrMf<double> {
+  typedef double acc __attribute__((ext_vector_type(4)));
+  __device__ static inline acc mma(double a, double b, acc c) { return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0); }
+  __device__ static inline int orow(int l, int r) { return 4 * r + (l >> 4); }
+};
+template <> struct TrMf<float> {
+  typedef float acc __attribute__((ext_vector_type(4)));
+  __device__ static inline acc mma(float a, float b, acc c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+  __device__ static inline int orow(int l, int r) { return 4 * (l >> 4) + r; }
+};
+
+template <typename T, int RB, bool MT>
+__global__ __launch_bounds__(256) void trsm_right_kernel(int n, long nvec, const T* __restrict__ A, long lda,
+                                                         bool upper, const T* __restrict__ inv, T* __restrict__ B,
+                                                         long ldb, const int* abort_flag) {
+  constexpr int LDX = RB + 2, RT = RB / 16, NB = TRSM_NB;
+  typedef TrMf<T> mf;
+  __shared__ T Xs[TRSM_RN * LDX];   // X(r, c) at Xs[c*LDX + r]
+  __shared__ T Ts[NB * LDX];        // B_b less the products of the solved blocks
   if (abort_flag && *abort_flag) return;
-  const long v0 = (long)blockIdx.x * 64;
-  const int t = threadIdx.x, r = t & 63, cg = t >> 6;
-  // staging: every load issued before the first LDS write (unconditional
-  // loads from clamped, in-bounds addresses; the padding is selected after)
-  constexpr int SU = TRSM_NB * TRSM_NB / 256;
-  T xv[SU], yv[SU];
-  const long vmax = nvec - 1 - v0;
+  const long v0 = (long)blockIdx.x * RB;
+  const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6), lr = lane & 15, lg = lane >> 4;
+  const int nblk = (n + NB - 1) / NB, np = nblk * NB;
+  const int rows = (int)min((long)RB, nvec - v0);
+  auto blk_of = [&](int q) { return upper ? q : nblk - 1 - q; };
+  // tile (q, p): p < q: M(block p, block q) of the order of solution; p == q: the inverse of block q
+  auto fetch = [&](int q, int p, T (&f)[16]) __attribute__((always_inline)) {
+    const int b = blk_of(q), c = 16 * w + lr;
+    if (p == q) {
+      const T* src = inv + (long)b * NB * NB + 16 * lg * NB + c;
 #pragma unroll
-  for (int u = 0; u < SU; u++) {
-    const int idx = t + 256 * u, rr = idx & 63, k = idx >> 6;
-    xv[u] = B[(v0 + min((long)rr, vmax)) + (long)min(k, nb - 1) * ldb];
-    yv[u] = inv[idx];
-  }
+      for (int s = 0; s < 16; s++) f[s] = src[s * NB];
+      return;
+    }
+    const int k0 = blk_of(p) * NB + 16 * lg, cc = b * NB + c;
+    if ((b + 1 < nblk && blk_of(p) + 1 < nblk) || np == n) {   // whole tiles
 #pragma unroll
-  for (int u = 0; u < SU; u++) {
-    const int idx = t + 256 * u, rr = idx & 63, k = idx >> 6;
-    Xs[k * LDX + rr] = (k < nb && v0 + rr < nvec) ? xv[u] : T(0);
-    Ys[idx] = yv[u];
+      for (int s = 0; s < 16; s++) f[s] = MT ? A[cc + (long)(k0 + s) * lda] : A[k0 + s + (long)cc * lda];
+    } else {
+#pragma unroll
+      for (int s = 0; s < 16; s++) {
+        const int k = min(k0 + s, n - 1), ce = min(cc, n - 1);
+        const T x = MT ? A[ce + (long)k * lda] : A[k + (long)ce * lda];
+        f[s] = k0 + s < n && cc < n ? x : T(0);
+      }
+    }
+  };
+  T cur[16], next[16];
+  fetch(0, 0, next);
+  for (int i0 = 0; i0 < np * RB; i0 += 256 * 16) {
+    T v[16];
+#pragma unroll
+    for (int u = 0; u < 16; u++) {
+      const int i = i0 + t + 256 * u, r = i % RB, c = i / RB;
+      v[u] = B[v0 + min(r, rows - 1) + (long)min(c, n - 1) * ldb];
+    }
+#pragma unroll
+    for (int u = 0; u < 16; u++) {
+      const int i = i0 + t + 256 * u, r = i % RB, c = i / RB;
+      if (c < np) Xs[c * LDX + r] = c < n && r < rows ? v[u] : T(0);
+    }
   }
   __syncthreads();
-  T acc[16];
+  typename mf::acc acc[RT];
 #pragma unroll
-  for (int c = 0; c < 16; c++) acc[c] = T(0);
-  // a static trip count (X and the inverse are zero past nb) lets each
-  // unrolled group of steps issue its LDS reads together
-#pragma unroll 8
-  for (int k = 0; k < TRSM_NB; k++) {
-    const T xv = Xs[k * LDX + r];
-    const T* yr = Ys + k * TRSM_NB + cg * 16;
+  for (int i = 0; i < RT; i++) acc[i] = typename mf::acc{};
+  int q = 0, p = 0;
+  while (true) {
 #pragma unroll
-    for (int c = 0; c < 16; c++) acc[c] += xv * yr[c];
-  }
-  if (v0 + r < nvec) {
+    for (int s = 0; s < 16; s++) cur[s] = next[s];
+    int nq = q, np2 = p + 1;
+    if (np2 > q) { nq = q + 1; np2 = 0; }
+    if (nq < nblk) fetch(nq, np2, next);
+    const int b = blk_of(q);
+    T* const xb = Xs + b * NB * LDX;
+    if (p == q) {   // T = B_b - products, every wavefront its 16 columns
 #pragma unroll
-    for (int c = 0; c < 16; c++)
-      if (cg * 16 + c < nb) B[(v0 + r) + (long)(cg * 16 + c) * ldb] = acc[c];
+      for (int i = 0; i < RT; i++)
+#pragma unroll
+        for (int x = 0; x < 4; x++) {
+          const int o = (16 * w + mf::orow(lane, x)) * LDX + 16 * i + lr;
+          Ts[o] = xb[o] - acc[i][x];
+          acc[i][x] = T(0);
+        }
+      __syncthreads();
+    }
+    const T* src = (p == q ? Ts : Xs + blk_of(p) * NB * LDX) + 16 * lg * LDX + lr;
+#pragma unroll
+    for (int s = 0; s < 16; s++)
+#pragma unroll
+      for (int i = 0; i < RT; i++) acc[i] = mf::mma(cur[s], src[s * LDX + 16 * i], acc[i]);
+    if (p == q) {   // X_b to LDS and memory
+#pragma unroll
+      for (int i = 0; i < RT; i++)
+#pragma unroll
+        for (int x = 0; x < 4; x++) {
+          const int c = 16 * w + mf::orow(lane, x), r = 16 * i + lr;
+          xb[c * LDX + r] = acc[i][x];
+          if (r < rows && b * NB + c < n) B[v0 + r + (long)(b * NB + c) * ldb] = acc[i][x];
+          acc[i][x] = T(0);
+        }
+      if (nq >= nblk) break;
+      __syncthreads();
+    }
+    q = nq;
+    p = np2;
   }
 }
 
@@ -496,24 +519,26 @@ template <typename T>
 static void leaf(bool right, bool lower, bool trans, bool unit, long nb, long nrhs, const T* a, long lda, T* b,
                  long ldb, hipStream_t s, const int* abort_flag, const InvCtx<T>& ic) {
   if (nb <= 0 || nrhs <= 0) return;
-  // E = op(A) for left, op(A)^T for right
-  const bool eT = trans != right;
-  const bool elower = lower != eT;
-  if (right && ic.inv) {
-    const long blk = (long)(a - ic.a0) / (ic.lda + 1) / TRSM_NB;
-    trsm_right_inv_kernel<T><<<(unsigned)((nrhs + 63) / 64), 256, 0, s>>>(
-        (int)nb, nrhs, ic.inv + blk * TRSM_NB * TRSM_NB, b, ldb, abort_flag);
-    OBA_HIP(hipGetLastError());
-    return;
-  }
+  const bool eT = trans, elower = lower != eT;   // left: E = op(A)
   if (right) {
-    trsm_leaf_rows_kernel<T><<<(unsigned)((nrhs + 63) / 64), 64, 0, s>>>((int)nb, nrhs, a, lda, b, ldb, eT, elower,
-                                                                        unit, abort_flag);
+    const T* inv = ic.inv + (long)(a - ic.a0) / (ic.lda + 1) / TRSM_NB * TRSM_NB * TRSM_NB;
+    const bool upper = lower == trans;   // op(A)
+#define OBA_TR(RB, MT)                                                                                             \
+  trsm_right_kernel<T, RB, MT><<<(unsigned)((nrhs + RB - 1) / RB), 256, 0, s>>>((int)nb, nrhs, a, lda, upper, inv, b, \
+                                                                                ldb, abort_flag)
+    // 32 rows per workgroup halve the reads of M: FP32 from two 16-row
+    // workgroups per CU on (16000 x 256: 54.5 us with 16 rows, 49.9 with 32);
+    // FP64 is bound by its MFMAs (71.9 / 74.8)
+    if (sizeof(T) == 4 && nrhs >= 16 * 2 * (long)rt().num_cu) {
+      if (trans) OBA_TR(32, true); else OBA_TR(32, false);
+    } else {
+      if (trans) OBA_TR(16, true); else OBA_TR(16, false);
+    }
+#undef OBA_TR
     OBA_HIP(hipGetLastError());
     return;
   }
-  const long inc_e = right ? ldb : 1;
-  const long inc_v = right ? 1 : ldb;
+  const long inc_e = 1, inc_v = ldb;
   const int waves = 4;
   const long per_block = (long)waves * TRSM_VPW;
   long blocks = (nrhs + per_block - 1) / per_block;
@@ -531,9 +556,9 @@ template <typename T>
 static void rec(bool right, bool lower, bool trans, bool unit, long m, long n, const T* a, long lda, T* b,
                 long ldb, hipStream_t s, const int* abort_flag, const InvCtx<T>& ic) {
   const long na = right ? n : m;   // order of the triangle
-  // left-side leaves take up to TRSM_LEAF_MAX rows (trsm_leafb_kernel);
-  // right-side leaves stay on the 64-grid of the diagonal inverses
-  if (na <= (right ? TRSM_NB : TRSM_LEAF_MAX)) {
+  // leaves: trsm_leafb_kernel (left), trsm_right_kernel (right; on the 64-grid
+  // of the diagonal inverses)
+  if (na <= (right ? TRSM_RN : TRSM_LEAF_MAX)) {
     leaf<T>(right, lower, trans, unit, na, right ? m : n, a, lda, b, ldb, s, abort_flag, ic);
     return;
   }
