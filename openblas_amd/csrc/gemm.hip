@@ -109,6 +109,35 @@ struct TileLoader {
   }
 };
 
+// the linear tile index of workgroup b: each of the 8 XCDs a contiguous range
+__device__ inline int xcd_range(int b, int total) {
+  const int x = b & 7, base = total >> 3, rem = total & 7;
+  return x * base + min(x, rem) + (b >> 3);
+}
+// tile `lin` of the lower triangle of nt x nt tiles, in groups of 8 tile rows
+// (columns left of a group's square first, down each column), so that equal
+// ranges of lin are equal work: an order over the full square gave the last
+// XCD twice the average share of the triangle (12000 x 448 FP64: 1810 us, and
+// 1374 with the tiles dealt out one by one)
+__device__ inline void tri_tile(int lin, int nt, int& tm, int& tn) {
+  auto row_of = [](int i) {   // largest r with r(r+1)/2 <= i
+    int r = (int)((sqrtf(8.0f * (float)i + 1.0f) - 1.0f) * 0.5f);
+    while ((long)r * (r + 1) / 2 > i) r--;
+    while ((long)(r + 1) * (r + 2) / 2 <= i) r++;
+    return r;
+  };
+  const int g0 = row_of(lin) & ~7, gs = min(nt - g0, 8);
+  const int off = lin - (int)((long)g0 * (g0 + 1) / 2);
+  if (off < g0 * gs) {
+    tm = g0 + off % gs;
+    tn = off / gs;
+  } else {
+    const int o = off - g0 * gs, r = row_of(o);
+    tm = g0 + r;
+    tn = g0 + o - r * (r + 1) / 2;
+  }
+}
+
 // KS > 1 (sliced K): the workgroup is KS groups of 4 wavefronts; group g
 // multiplies the g-th of KS equal, BK-aligned k ranges into its own
 // accumulators, and the KS partial tiles are summed in LDS in the fixed
@@ -161,24 +190,25 @@ __global__ __launch_bounds__(256 * KS, OCC) void gemm_kernel(long M, long N, lon
 
   // XCD-aware tile order: workgroup b runs on XCD b%8; give each XCD a
   // contiguous range of the grouped tile order.
-  const int T_all = tiles_m * tiles_n;
-  int lin = blockIdx.x;
-  if ((T_all & 7) == 0) lin = (blockIdx.x & 7) * (T_all >> 3) + (blockIdx.x >> 3);
-  constexpr int GM = 8;
-  const int group = lin / (GM * tiles_n);
-  const int first_m = group * GM;
-  const int gsize = min(tiles_m - first_m, GM);
-  const int in_group = lin - group * GM * tiles_n;
-  const int tm = first_m + in_group % gsize;
-  const int tn = in_group / gsize;
+  int lin = xcd_range(blockIdx.x, gridDim.x);
+  int tm, tn;
+  if (tri) {   // gridDim.x = the tiles of the triangle
+    tri_tile(lin, tiles_m, tm, tn);
+    if (tri == 2) { const int x = tm; tm = tn; tn = x; }
+  } else {
+    constexpr int GM = 8;
+    const int group = lin / (GM * tiles_n);
+    const int first_m = group * GM;
+    const int gsize = min(tiles_m - first_m, GM);
+    const int in_group = lin - group * GM * tiles_n;
+    tm = first_m + in_group % gsize;
+    tn = in_group / gsize;
+  }
   // the tile owns C rows [mt, mt+BM) and columns [nt, nt+BN); an edge tile
   // reads from m0 = M-BM (n0 = N-BN) instead, where every load is in range,
   // recomputing rows of its neighbour that it does not store
   const long mt = (long)tm * BM, nt = (long)tn * BN;
   const long m0 = M >= BM ? min(mt, M - BM) : 0, n0 = N >= BN ? min(nt, N - BN) : 0;
-  // tri: 1 = update only C(i,j) with i >= j (lower), 2 = only i <= j (upper)
-  if (tri == 1 && nt > mt + BM - 1) return;
-  if (tri == 2 && mt > nt + BN - 1) return;
   if (abort_flag && *abort_flag) return;
 
   const int lane = threadIdx.x & 63;
@@ -495,7 +525,8 @@ static void launch_cfg(bool ta, bool tb, long M, long N, long K, T alpha, const 
                        const int* abort_flag, int ksplit = 1, long kc = 0, long cstride = 0) {
   long tm = (M + BM - 1) / BM, tn = (N + BN - 1) / BN;
   if (tm * tn > 0x7fffffffL) fatal("gemm: grid too large", nullptr);
-  dim3 grid((unsigned)(tm * tn), (unsigned)ksplit), block(256 * KS);
+  if (tri && (BM != BN || M != N)) fatal("gemm: a triangular update is of square tiles of a square C", nullptr);
+  dim3 grid((unsigned)(tri ? tm * (tm + 1) / 2 : tm * tn), (unsigned)ksplit), block(256 * KS);
 #define OBA_GEMM_L(TA_, TB_) \
   gemm_kernel<T, BM, BN, BK, TA_, TB_, KS, OCC><<<grid, block, 0, s>>>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, (int)tm, (int)tn, tri, abort_flag, kc, cstride)
   if (!ta && !tb) OBA_GEMM_L(false, false);
@@ -563,8 +594,9 @@ void gemm(bool ta, bool tb, long m, long n, long k, T alpha, const T* a, long ld
   // group per tile does that, and fewer tiles than CUs want smaller ones.
   constexpr bool D = sizeof(T) == 8;
   const long cu = rt().num_cu;
-  const long m64 = (m + 63) / 64, t64 = m64 * ((n + 63) / 64), t6432 = m64 * ((n + 31) / 32);
-  const long t32 = ((m + 31) / 32) * ((n + 31) / 32);
+  const long m64 = (m + 63) / 64, m32 = (m + 31) / 32;   // tri: only the triangle's tiles run
+  const long t64 = tri ? m64 * (m64 + 1) / 2 : m64 * ((n + 63) / 64), t6432 = m64 * ((n + 31) / 32);
+  const long t32 = tri ? m32 * (m32 + 1) / 2 : m32 * ((n + 31) / 32);
   constexpr int BK32 = D ? 16 : 32, BK64 = D ? 8 : 16;
 #define OBA_GEMM_ARGS ta, tb, m, n, k, alpha, a, lda, b, ldb, beta, c, ldc, s, tri, abort_flag
   if (8 * t64 < 7 * cu) {
@@ -588,7 +620,7 @@ void gemm(bool ta, bool tb, long m, long n, long k, T alpha, const T* a, long ld
     else launch_cfg<T, 32, 32, BK32, 1, 4>(OBA_GEMM_ARGS);
     return;
   }
-  if (D && t64 <= 4 * cu && k >= 256) {
+  if (D && tri == 0 && t64 <= 4 * cu && k >= 256) {
     // the narrower tile where 64x64 ones would fill their last round of CUs
     // worse (316 tiles on 256 CUs: 303 us, 632 half tiles: 258), or there is
     // one per CU
@@ -601,7 +633,7 @@ void gemm(bool ta, bool tb, long m, long n, long k, T alpha, const T* a, long ld
   }
   // FP32 (16-cycle steps) needs the LDS reuse of 128x128 tiles once there are
   // enough of them: 8192^3 7883 us against 8414 with 64x64; 3000^3 574 / 468
-  const long t128 = ((m + 127) / 128) * ((n + 127) / 128);
+  const long m128 = (m + 127) / 128, t128 = tri ? m128 * (m128 + 1) / 2 : m128 * ((n + 127) / 128);
   if (t64 <= 2 * cu && k >= 256) launch_cfg<T, 64, 64, BK64, 2, 2>(OBA_GEMM_ARGS);
   else if (!D && t128 >= 8 * cu) launch_cfg<T, 128, 128, 16, 1, 2>(OBA_GEMM_ARGS);
   else launch_cfg<T, 64, 64, BK64, 1, 4>(OBA_GEMM_ARGS);
