@@ -10,7 +10,7 @@
 // MI355X design: recursion on halves (64-column grid): L21 <- A21*L11^-T is a
 // right-side TRSM, A22 -= L21*L21^T is an MFMA GEMM restricted to the lower
 // triangle (the role of the reference's SYRK kernel); 64x64 diagonal leaves
-// are factored by one wavefront with the rows in registers.  Large lower
+// are factored and inverted by one workgroup.  Large lower
 // factorizations run blocked with look-ahead (potrf_blocked).  A failing leaf raises a device flag
 // that turns every later kernel of the same call into a no-op, so the call
 // stops where the reference stops without a host round trip per leaf.
@@ -28,104 +28,265 @@ __device__ inline double po_rl(double v, int l) {
   return __hiloint2double(hi, lo);
 }
 
-// Factor the nb x nb (nb <= 64) diagonal block at a (lower: E(i,k) =
-// a[i + k*lda]; upper: E(i,k) = a[k + i*lda], i >= k); info and the failure
-// flag take the global column offset j0.  One wavefront, no barrier: lane i
-// loads row i of the block straight into registers (all loads in flight at
-// once; a staging loop through LDS waited for each load in turn, and a
-// four-wavefront form with two barriers per column took ~73 us FP32 per
-// leaf), x[k] holding column 16q + k while the column loop is in its
-// quarter q (the row is shifted down by 16 registers between quarters, so
-// every register index in the unrolled 16-column body is static).  Column
-// j: the diagonal comes from lane j (readlane); ajj <= 0 (not NaN) is
-// stored as it is and stops the leaf; otherwise the column is scaled by
-// 1/l_jj (potf2_L.c's SCAL_K), its multipliers go through LDS (written and
-// read back by the same wavefront) and every lane subtracts l_ij l_kj from
-// its entries right of j (entries above the diagonal take garbage and are
-// never stored; LDS past column 63 reads zeros).  A quarter's 16 columns
-// are final when it ends and are stored then.
+template <typename T> struct PoMf;
+template <> struct PoMf<double> {
+  typedef double acc __attribute__((ext_vector_type(4)));
+  __device__ static inline acc mma(double a, double b, acc c) { return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0); }
+  __device__ static inline int orow(int l, int r) { return 4 * r + (l >> 4); }
+};
+template <> struct PoMf<float> {
+  typedef float acc __attribute__((ext_vector_type(4)));
+  __device__ static inline acc mma(float a, float b, acc c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+  __device__ static inline int orow(int l, int r) { return 4 * (l >> 4) + r; }
+};
+
+// lane K of each row of 16 lanes, to all of the row
+template <int K>
+__device__ inline float po_bcast16(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + K, 0xF, 0xF, false));
+}
+template <int K>
+__device__ inline double po_bcast16(double v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), 0x150 + K, 0xF, 0xF, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), 0x150 + K, 0xF, 0xF, false);
+  return __hiloint2double(hi, lo);
+}
+template <int K, typename T>
+__device__ __attribute__((always_inline)) inline void potrf_inv16_step(T (&y)[4], const T (&l)[16], T r, int i) {
+  if constexpr (K < 15) {
+    const T rk = po_bcast16<K>(r);
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+      const T f = y[c] - l[K] * (po_bcast16<K>(y[c]) * rk);
+      y[c] = i > K ? f : y[c];   // an Inf or NaN of L only meets its own rows
+    }
+    potrf_inv16_step<K + 1>(y, l, r, i);
+  }
+}
+// One wavefront inverts the 16x16 lower triangle at o (diagonal reciprocals
+// in rinv): lane (i, g) = (lane % 16, lane / 16) holds row i of columns g,
+// g+4, g+8, g+12; row k, once final, reaches the rows below by DPP row
+// broadcasts.
 template <typename T>
-__global__ __launch_bounds__(64) void potrf_leaf1_kernel(int nb, T* a, long lda, bool upper, long j0, int* info) {
-  __shared__ T col[2 * PO_NB];
-  if (*info) return;
-  const int lane = threadIdx.x;
-  const int rl = min(lane, nb - 1);   // in-bounds row for the unconditional loads
-  // row `lane` straight into registers: all 64 loads in flight at once
-  // (lower: E(i,k) = a[i + k*lda], coalesced across lanes; upper: a[k + i*lda])
-  T x[PO_NB];
+__device__ __attribute__((always_inline)) inline void potrf_inv16(const T* S, T* Y, const T* rinv, int o) {
+  constexpr int LD = PO_NB + 1;
+  const int i = threadIdx.x & 15, g = (threadIdx.x & 63) >> 4;
+  T l[16], y[4];
 #pragma unroll
-  for (int k = 0; k < PO_NB; k++) {
-    const int kc = min(k, nb - 1);
-    const T v = upper ? a[kc + (long)rl * lda] : a[rl + (long)kc * lda];
-    x[k] = (lane < nb && k < nb && k <= lane) ? v : T(0);
-  }
-  col[PO_NB + lane] = T(0);
-  int fail = 0;
-#pragma unroll 1
-  for (int q = 0; q < 4; q++) {
-    int done = 16;   // columns of this quarter that are final in x[0..15]
+  for (int k = 0; k < 16; k++) l[k] = S[(o + k) * LD + o + i];
+  const T r = rinv[o + i];
 #pragma unroll
-    for (int jj = 0; jj < 16; jj++) {
-      const int j = 16 * q + jj;
-      if (j >= nb || fail) { done = min(done, jj); continue; }   // uniform
-      const T d = po_rl(x[jj], j);
-      if (!(d > T(0)) && !isnan(d)) {   // ajj <= 0: stored as it is, stop
-        fail = j + 1;
-        done = jj + 1;                   // the failing column keeps its diagonal
-        continue;
-      }
-      const T ljj = sqrt(d);
-      const T rinv = T(1) / ljj;
-      const T lij = lane == j ? ljj : x[jj] * rinv;
-      if (lane >= j) x[jj] = lij;
-      const T li = lane > j ? lij : T(0);
-      col[lane] = li;
+  for (int c = 0; c < 4; c++) y[c] = i == g + 4 * c ? T(1) : T(0);
+  potrf_inv16_step<0>(y, l, r, i);
 #pragma unroll
-      for (int k = jj + 1; k < PO_NB; k++) x[k] -= li * col[16 * q + k];
-    }
-    // the quarter's final columns back to memory (of a failing column
-    // only its diagonal)
-#pragma unroll
-    for (int k = 0; k < 16; k++) {
-      const int c = 16 * q + k;
-      const bool st = k < done && lane < nb && c <= lane && !(fail && c == fail - 1 && lane > c);
-      if (st) {
-        if (upper) a[c + (long)lane * lda] = x[k];
-        else a[lane + (long)c * lda] = x[k];
-      }
-    }
-    if (fail || 16 * (q + 1) >= nb) break;
-#pragma unroll
-    for (int k = 0; k < PO_NB - 16; k++) x[k] = x[k + 16];
-#pragma unroll
-    for (int k = PO_NB - 16; k < PO_NB; k++) x[k] = T(0);
-  }
-  if (lane == 0 && fail) *info = (int)(j0 + fail);
+  for (int c = 0; c < 4; c++) Y[(o + g + 4 * c) * LD + o + i] = i >= g + 4 * c ? y[c] * r : T(0);
 }
 
+// one wavefront: tile (ri, ci) of `o` = sign * sum over the 16-deep tiles k0
+// .. k0+NK of x(ri, k) y(k, ci), in 64x64 LDS matrices
+template <int NK, typename T>
+__device__ __attribute__((always_inline)) inline void potrf_prod(T* o, const T* x, const T* y, int ri, int ci, int k0,
+                                                                 T sign) {
+  constexpr int LD = PO_NB + 1;
+  typedef PoMf<T> mf;
+  const int lane = threadIdx.x & 63, lr = lane & 15, lg = lane >> 4;
+  typename mf::acc acc[2] = {};
+#pragma unroll
+  for (int k = 0; k < 16 * NK; k += 4)
+    acc[(k >> 2) & 1] = mf::mma(y[(16 * ci + lr) * LD + 16 * k0 + k + lg], x[(16 * k0 + k + lg) * LD + 16 * ri + lr],
+                                acc[(k >> 2) & 1]);
+  acc[0] += acc[1];
+#pragma unroll
+  for (int r = 0; r < 4; r++) o[(16 * ci + mf::orow(lane, r)) * LD + 16 * ri + lr] = sign * acc[0][r];
+}
+
+// Factor the nb x nb (nb <= 64) diagonal block at a (lower: E(i,k) =
+// a[i + k*lda]; upper: E(i,k) = a[k + i*lda], i >= k) and, when inv is not
+// null, invert the factor for the right-side solve that follows
+// (M = L^T: M^{-1}(i,j) = L^{-1}(j,i) at inv[i*64 + j], as
+// trsm_inv_diag_kernel leaves it); info and the failure flag take the global
+// column offset j0.
+//
+// The bound is the chain of 64 columns (diagonal, square root, reciprocal,
+// multipliers, next column).  The block sits in LDS and is taken in four
+// steps of 16 columns: wavefront 0 factors a step with row i in lane i and the
+// 16 columns in registers, every value another row needs read with
+// v_readlane (no LDS, no barrier inside a step); then all four wavefronts
+// subtract the step's products from the later columns, 16x16 tiles on the
+// matrix cores; wavefronts 1 to 3 invert the finished 16x16 diagonal blocks
+// and join the inverse 16 -> 32 -> 64 by small MFMA products while wavefront 0
+// factors the next step.  22 us FP64 and 16 FP32 with the inverse.  One wavefront
+// with all 64 columns in registers, every column updating all later ones with
+// multipliers read back from LDS, took 62 and 50 us per leaf, and the
+// inversion was a launch of its own (16 and 14 us).
+//
+// Column j: ajj <= 0 (not NaN) is stored as it is and stops the leaf
+// (potf2_L.c:71-75); otherwise the column is scaled by 1/l_jj (its SCAL_K).
+// Rows and columns past nb hold the identity.
 template <typename T>
-static void potrf_rec(bool lower, long j0, long nc, T* a, long lda, int* info, hipStream_t s) {
+__global__ __launch_bounds__(256) void potrf_leaf_kernel(int nb, T* a, long lda, bool upper, long j0, int* info,
+                                                         T* inv) {
+  constexpr int NB = PO_NB, LD = NB + 1;
+  typedef PoMf<T> mf;
+  __shared__ T S[NB * LD];   // E(i, c) at S[c*LD + i]
+  __shared__ T Y[NB * LD];   // L^{-1}(i, c) at Y[c*LD + i]
+  __shared__ T U[NB * LD];   // products of the joins
+  __shared__ T s_rinv[NB];
+  __shared__ int s_fail;
+  if (*info) return;
+  const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6), lr = lane & 15, lg = lane >> 4;
+  {
+    T v[16];
+#pragma unroll
+    for (int u = 0; u < 16; u++) {
+      const int f = (t + 256 * u) & 63, g = (t + 256 * u) >> 6;   // f contiguous in memory
+      v[u] = a[min(f, nb - 1) + (long)min(g, nb - 1) * lda];
+    }
+#pragma unroll
+    for (int u = 0; u < 16; u++) {
+      const int f = (t + 256 * u) & 63, g = (t + 256 * u) >> 6, i = upper ? g : f, c = upper ? f : g;
+      S[c * LD + i] = i >= c && i < nb && c < nb ? v[u] : (i == c ? T(1) : T(0));
+      Y[c * LD + i] = T(0);
+    }
+  }
+  if (t == 0) s_fail = 0;
+  __syncthreads();
+  int fail = 0;
+#pragma unroll 1
+  for (int q = 0; q < 5; q++) {
+    if (w == 0 && q < 4) {
+      // row (lane + 16q) mod 64 in this lane: the step's own 16 rows are in
+      // lanes 0..15 whatever q is, so every v_readlane has a constant lane
+      // (with a lane index from an SGPR they took 25 cycles each, 740 a column)
+      const int row = (lane + 16 * q) & 63;
+      const bool below = lane < 64 - 16 * q;   // rows 16q and later
+      T x[16];
+#pragma unroll
+      for (int k = 0; k < 16; k++) x[k] = S[(16 * q + k) * LD + row];
+      // no branch inside the step: the tail of a column's update runs beside
+      // the next column's square root and reciprocal
+      bool low = false;
+      T rv = T(0);
+#pragma unroll
+      for (int jj = 0; jj < 16; jj++) {
+        const T d = po_rl(x[jj], jj);
+        low |= d <= T(0);
+        const T ljj = sqrt(d);
+        const T rinv = T(1) / ljj;
+        const T li = x[jj] * rinv;
+#pragma unroll
+        for (int k = jj + 1; k < 16; k++) x[k] -= li * po_rl(li, k);
+        x[jj] = lane == jj ? ljj : li;
+        rv = lane == jj ? rinv : rv;
+      }
+      int bad = 0;
+      if (low) {   // the step again, up to the diagonal that is stored as it is
+#pragma unroll
+        for (int k = 0; k < 16; k++) x[k] = S[(16 * q + k) * LD + row];
+#pragma unroll
+        for (int jj = 0; jj < 16; jj++) {
+          const T d = po_rl(x[jj], jj);
+          if (!bad && d <= T(0)) bad = 16 * q + jj + 1;
+          if (bad) continue;
+          const T ljj = sqrt(d);
+          const T li = x[jj] * (T(1) / ljj);
+#pragma unroll
+          for (int k = jj + 1; k < 16; k++) x[k] -= li * po_rl(li, k);
+          x[jj] = lane == jj ? ljj : li;
+        }
+      }
+      if (lane < 16) s_rinv[16 * q + lane] = rv;
+      if (below) {
+#pragma unroll
+        for (int k = 0; k < 16; k++)
+          if (lane >= k) S[(16 * q + k) * LD + row] = x[k];
+      }
+      if (lane == 0 && bad) s_fail = bad;
+    }
+    if (inv) {   // beside the factorization of a step: the inverse, as far as the columns are final
+      if (w == 3 && q > 0) {
+        potrf_inv16(S, Y, s_rinv, 16 * (q - 1));
+        if (!(q & 1)) {   // join with the block before
+          potrf_prod<1>(U, S, Y, q - 1, q - 2, q - 2, T(1));
+          potrf_prod<1>(Y, Y, U, q - 1, q - 2, q - 1, T(-1));
+        }
+      }
+      if (q == 3 && (w == 1 || w == 2)) {   // L21 Y11
+#pragma unroll 1
+        for (int u = 0; u < 2; u++) potrf_prod<2>(U, S, Y, 1 + w, u, 0, T(1));
+      }
+    }
+    if (q == 4) break;
+    __syncthreads();
+    fail = __builtin_amdgcn_readfirstlane(s_fail);
+    if (fail) break;
+    // the step's products leave the later columns, one tile per wavefront at
+    // a time: (1,1) (2,1) (2,2) (3,1) (3,2) (3,3), offset by q
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+      const int tile = w + 4 * u, ti = tile < 1 ? 1 : tile < 3 ? 2 : 3, tj = tile - ti * (ti - 1) / 2 + 1;
+      const int ri = q + ti, ci = q + tj;
+      if (tile < 6 && ri < 4) {
+        const T* l = S + (16 * q + lg) * LD;
+        typename mf::acc acc{};
+#pragma unroll
+        for (int s = 0; s < 4; s++)
+          acc = mf::mma(l[4 * s * LD + 16 * ci + lr], l[4 * s * LD + 16 * ri + lr], acc);
+#pragma unroll
+        for (int r = 0; r < 4; r++) S[(16 * ci + mf::orow(lane, r)) * LD + 16 * ri + lr] -= acc[r];
+      }
+    }
+    __syncthreads();
+  }
+  // the factor back to memory (a failed leaf: the columns before the failing
+  // one, and its diagonal)
+  const int cols = fail ? fail - 1 : nb;
+#pragma unroll
+  for (int u = 0; u < 16; u++) {
+    const int f = (t + 256 * u) & 63, g = (t + 256 * u) >> 6, i = upper ? g : f, c = upper ? f : g;
+    if (i < nb && i >= c && (c < cols || (c == cols && i == c && c < nb))) a[f + (long)g * lda] = S[c * LD + i];
+  }
+  if (fail) {
+    if (t == 0) *info = (int)(j0 + fail);
+    return;
+  }
+  if (!inv) return;
+  __syncthreads();
+  potrf_prod<2>(Y, Y, U, 2 + (w >> 1), w & 1, 2, T(-1));   // Y21 = -Y22 (L21 Y11)
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < 16; u++) {
+    const int idx = t + 256 * u, i = idx >> 6, j = idx & 63;
+    inv[idx] = i < nb && j < nb ? Y[i * LD + j] : T(0);
+  }
+}
+
+// inv (lower): the inverses of the 64x64 diagonal blocks, block b of the
+// matrix at inv + b*64*64, left by the leaves for the right-side solves
+template <typename T>
+static void potrf_rec(bool lower, long j0, long nc, T* a, long lda, int* info, T* inv, hipStream_t s) {
   T* a11 = a + j0 + j0 * lda;
+  T* inv11 = inv ? inv + j0 * PO_NB : nullptr;   // j0 is a multiple of 64
   if (nc <= PO_NB) {
-    potrf_leaf1_kernel<T><<<1, 64, 0, s>>>((int)nc, a11, lda, !lower, j0, info);
+    potrf_leaf_kernel<T><<<1, 256, 0, s>>>((int)nc, a11, lda, !lower, j0, info, inv11);
     OBA_HIP(hipGetLastError());
     return;
   }
   long n1 = ((nc / 2) + PO_NB - 1) / PO_NB * PO_NB;
   if (n1 >= nc) n1 = nc - PO_NB;
   const long n2 = nc - n1;
-  potrf_rec<T>(lower, j0, n1, a, lda, info, s);
+  potrf_rec<T>(lower, j0, n1, a, lda, info, inv, s);
   T* a22 = a + (j0 + n1) + (j0 + n1) * lda;
   if (lower) {
     T* a21 = a + (j0 + n1) + j0 * lda;
-    trsm<T>(true, true, true, false, n2, n1, T(1), a11, lda, a21, lda, s, info);   // A21 L11^-T
+    trsm_right_prepared<T>(true, true, false, n2, n1, a11, lda, a21, lda, inv11, s, info);   // A21 L11^-T
     gemm<T>(false, true, n2, n2, n1, T(-1), a21, lda, a21, lda, T(1), a22, lda, s, 1, info);
   } else {
     T* a12 = a + j0 + (j0 + n1) * lda;
     trsm<T>(false, false, true, false, n1, n2, T(1), a11, lda, a12, lda, s, info);  // U11^-T A12
     gemm<T>(true, false, n2, n2, n1, T(-1), a12, lda, a12, lda, T(1), a22, lda, s, 2, info);
   }
-  potrf_rec<T>(lower, j0 + n1, n2, a, lda, info, s);
+  potrf_rec<T>(lower, j0 + n1, n2, a, lda, info, inv, s);
 }
 
 // Blocked right-looking Cholesky (lower) with look-ahead, for large n, as
@@ -142,14 +303,11 @@ static void potrf_rec(bool lower, long j0, long nc, T* a, long lda, int* info, h
 // recursion.  The trailing sums run over blocks instead of recursion
 // halves: a different association of the same products.
 template <typename T>
-static void potrf_blocked(long n, T* a, long lda, int* info, long nb, hipStream_t s) {
+static void potrf_blocked(long n, T* a, long lda, int* info, long nb, T* inv, hipStream_t s) {
   Runtime& r = rt();
   hipStream_t M = s, X = bulk_stream();
-  DevBuf invb[2] = {DevBuf(trsm_right_inv_bytes<T>(nb)), DevBuf(trsm_right_inv_bytes<T>(nb))};
-  invb[0].use_on(X);   // read by the bulk stream's solves
-  invb[1].use_on(X);
   auto at = [&](long i, long j) { return a + i + j * lda; };
-  potrf_rec<T>(true, 0, std::min(nb, n), a, lda, info, M);
+  potrf_rec<T>(true, 0, std::min(nb, n), a, lda, info, inv, M);
   bool pending = false;
   for (long jb = 0; jb < n; jb += nb) {
     const long w = std::min(nb, n - jb), jn = jb + w;
@@ -159,16 +317,15 @@ static void potrf_blocked(long n, T* a, long lda, int* info, long nb, hipStream_
     }
     if (jn >= n) break;
     const long w1 = std::min(nb, n - jn);
-    T* inv = invb[(jb / nb) & 1].as<T>();
     const T* l11 = at(jb, jb);
-    trsm_right_prepare<T>(true, true, false, w, l11, lda, inv, M);
-    trsm_right_prepared<T>(true, true, false, w1, w, l11, lda, at(jn, jb), lda, inv, M, info);
+    const T* inv11 = inv + jb * PO_NB;
+    trsm_right_prepared<T>(true, true, false, w1, w, l11, lda, at(jn, jb), lda, inv11, M, info);
     gemm<T>(false, true, w1, w1, w, T(-1), at(jn, jb), lda, at(jn, jb), lda, T(1), at(jn, jn), lda, M, 1, info);
     const long rest = n - (jn + w1);
     if (rest > 0) {
       OBA_HIP(hipEventRecord(r.ev_a, M));
       OBA_HIP(hipStreamWaitEvent(X, r.ev_a, 0));
-      trsm_right_prepared<T>(true, true, false, rest, w, l11, lda, at(jn + w1, jb), lda, inv, X, info);
+      trsm_right_prepared<T>(true, true, false, rest, w, l11, lda, at(jn + w1, jb), lda, inv11, X, info);
       gemm<T>(false, true, rest, w1, w, T(-1), at(jn + w1, jb), lda, at(jn, jb), lda, T(1), at(jn + w1, jn), lda, X, 0,
               info);
       gemm<T>(false, true, rest, rest, w, T(-1), at(jn + w1, jb), lda, at(jn + w1, jb), lda, T(1),
@@ -176,7 +333,7 @@ static void potrf_blocked(long n, T* a, long lda, int* info, long nb, hipStream_
       OBA_HIP(hipEventRecord(r.ev_b, X));
       pending = true;
     }
-    potrf_rec<T>(true, jn, w1, a, lda, info, M);
+    potrf_rec<T>(true, jn, w1, a, lda, info, inv, M);
   }
   if (pending) OBA_HIP(hipStreamWaitEvent(M, r.ev_b, 0));
 }
@@ -184,12 +341,13 @@ static void potrf_blocked(long n, T* a, long lda, int* info, long nb, hipStream_
 // block width of the look-ahead driver (OPENBLAS_AMD_PO_NB; 0 turns it off);
 // it is used from 4 blocks on
 template <typename T>
-static long potrf_block_nb() {
-  // swept at n = 16384 with the one-wavefront leaves (the chain no longer
-  // the bound, the trailing updates prefer a deeper K): 256 / 320 / 384 /
-  // 448 / 512 / 640 / 768 gave dpotrf 70.2 / 65.0 / 61.8 / 62.0 / 71.8 /
-  // 60.5 / 64.8 ms, spotrf 41.3 / 39.3 / 38.6 / 38.3 / 43.0 / 39.5 / 41.5
-  long v = 384;
+static long potrf_block_nb(long n) {
+  // swept with the 64x64 leaves inverted in place, ms for widths 256 / 384 /
+  // 512 / 640: dpotrf n = 5000 3.54 / 3.86 / 3.71 / 3.99, 8192 7.25 / 7.43 /
+  // 7.28 / 7.70, 16384 35.0 / 34.3 / 33.0 / 33.5; spotrf 8192 5.37 / 5.39 /
+  // 5.48 / 5.77, 16384 21.2 / 20.4 / 19.8 / 20.3: short chains favour the
+  // narrow block, large trailing updates the deeper K
+  long v = n >= 12288 ? 512 : 256;
   if (const char* e = getenv("OPENBLAS_AMD_PO_NB")) v = atol(e);
   return v;
 }
@@ -200,9 +358,15 @@ int potrf(bool lower, long n, T* a, long lda, hipStream_t s) {
   DevBuf ib(sizeof(int) * 64);
   int* info = ib.as<int>();
   OBA_HIP(hipMemsetAsync(info, 0, sizeof(int), s));
-  const long nb = potrf_block_nb<T>();
-  if (lower && nb > 0 && n >= 4 * nb) potrf_blocked<T>(n, a, lda, info, nb, s);
-  else potrf_rec<T>(lower, 0, n, a, lda, info, s);
+  const long nb = potrf_block_nb<T>(n);
+  const bool blocked = lower && nb >= PO_NB && nb % PO_NB == 0 && n >= 4 * nb;
+  DevBuf invb(lower ? trsm_right_inv_bytes<T>(n) : 0);
+  if (blocked) {
+    invb.use_on(bulk_stream());   // read by the bulk stream's solves
+    potrf_blocked<T>(n, a, lda, info, nb, invb.as<T>(), s);
+  } else {
+    potrf_rec<T>(lower, 0, n, a, lda, info, invb.as<T>(), s);
+  }
   int h = 0;
   OBA_HIP(hipMemcpyAsync(&h, info, sizeof(int), hipMemcpyDeviceToHost, s));
   OBA_HIP(hipStreamSynchronize(s));
