@@ -13,12 +13,7 @@
 //    without one launch per problem;
 //  * GEMM: BT x BT output tiles (BT = 32 or 64) on the FP64/FP32 16x16x4
 //    MFMA, k-slabs staged through LDS;
-//  * LU (m <= 512): one workgroup per problem; each thread owns one or two
-//    rows of the current W-column panel in registers, the pivot search is
-//    a wavefront max-reduction plus one barrier per column, interchanges
-//    are deferred (a position -> row map in LDS; rows are permuted once at
-//    the end), the U12 block is a column-per-thread substitution and the
-//    trailing update a rank-W FMA sweep with U12 broadcast from LDS;
+//  * LU (m <= 512): batched_lu.h, one launch per size class;
 //  * Cholesky (n <= 512): same row-owner panel, one barrier per column,
 //    SYRK-shaped trailing update of the lower triangle;
 //  * LU solve (n <= 512): one wavefront per problem, the right-hand side in
@@ -49,6 +44,12 @@ namespace oba {
 // memory operations too.  They point to device memory: use them as global.
 template <typename T>
 using gptr = __attribute__((address_space(1))) T*;
+
+}  // namespace oba
+
+#include "batched_lu.h"
+
+namespace oba {
 
 // ---- small device helpers ----------------------------------------------------
 __device__ inline double bcast_lane(double v, int l) {
@@ -219,267 +220,6 @@ __global__ __launch_bounds__(256) void bgemm_kernel(const BDesc* __restrict__ de
           }
       }
     }
-    __syncthreads();
-    cur ^= 1;
-    it = s_item[cur];
-  }
-}
-
-// ---- batched LU (m <= 256*RPT) -------------------------------------------------
-template <typename T, int RPT, int W>
-__global__ __launch_bounds__(256) void bgetrf_kernel(const BDesc* __restrict__ desc, int count,
-                                                     unsigned* __restrict__ counter, int* __restrict__ info_out) {
-  constexpr int NT = 256, MAXM = NT * RPT, UB = NT, LDU = W + 1, CH = 8, BU = RPT == 1 ? 32 : 16;
-  typedef typename RowVec<T, W>::type RV;
-  __shared__ int s_perm[MAXM];            // position -> physical row
-  __shared__ T s_row[2][4][W];            // per-wave pivot candidates (by column parity)
-  __shared__ double s_key[2][4];
-  __shared__ int s_pos[2][4];
-  __shared__ T s_l11[W * W];              // strictly lower part of the diagonal block
-  __shared__ T s_u[UB * LDU];             // U12 chunk, one column per thread
-  __shared__ T s_l21[RPT == 1 ? MAXM * LDU : 1];   // multipliers of the trailing rows (MFMA update)
-  __shared__ int s_prow[RPT == 1 ? MAXM : 1];      // their physical rows
-  __shared__ int s_item[2];
-  __shared__ int s_moved;
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-
-  if (t == 0) s_item[0] = (int)atomicAdd(counter, 1u);
-  __syncthreads();
-  int cur = 0;
-  int it = s_item[0];
-  while (it < count) {
-    if (t == 0) { s_item[cur ^ 1] = (int)atomicAdd(counter, 1u); s_moved = 0; }
-    const BDesc& d = desc[it];
-    const int m = d.m, n = d.n, kmax = min(d.m, d.n);
-    const long lda = d.lda;
-    gptr<T> A = (gptr<T>)d.a;
-    gptr<int> ipiv = (gptr<int>)d.ipiv;
-    int info = 0;
-    for (int i = t; i < m; i += NT) s_perm[i] = i;
-    __syncthreads();
-
-    #pragma unroll 1
-    for (int j0 = 0; j0 < kmax; j0 += W) {
-      const int w = min(W, kmax - j0);
-      RV x[RPT];
-      int pos[RPT], phys[RPT];
-      bool live[RPT];
-#pragma unroll
-      for (int q = 0; q < RPT; q++) {
-        pos[q] = j0 + t + NT * q;
-        live[q] = pos[q] < m;
-        phys[q] = live[q] ? s_perm[pos[q]] : 0;
-#pragma unroll
-        for (int c = 0; c < W; c++) x[q][c] = (live[q] && c < w) ? A[phys[q] + (j0 + c) * lda] : T(0);
-      }
-      #pragma unroll 1
-      for (int k = 0; k < w; k++) {
-        const int j = j0 + k, buf = k & 1;
-        double bv = -2.0;
-        int bp = INT_MAX, bq = -1;
-#pragma unroll
-        for (int q = 0; q < RPT; q++) {
-          if (live[q] && pos[q] >= j) {
-            const double v = pivot_key((T)pick<RV, W>(x[q], k), pos[q], j);
-            if (better(v, pos[q], bv, bp)) { bv = v; bp = pos[q]; bq = q; }
-          }
-        }
-        double wv = bv;
-        int wp = bp;
-        lu_wave_best(wv, wp);   // DPP row moves + readlanes (no LDS shuffles)
-        if (lane == 0) { s_key[buf][wave] = wv; s_pos[buf][wave] = wp; }
-        if (bq >= 0 && bp == wp) {
-#pragma unroll
-          for (int q = 0; q < RPT; q++)
-            if (q == bq) {
-#pragma unroll
-              for (int c = 0; c < W; c++) s_row[buf][wave][c] = x[q][c];
-            }
-        }
-        __syncthreads();
-        double gv = s_key[buf][0];
-        int gp = s_pos[buf][0], gw = 0;
-#pragma unroll
-        for (int v = 1; v < 4; v++)
-          if (better(s_key[buf][v], s_pos[buf][v], gv, gp)) { gv = s_key[buf][v]; gp = s_pos[buf][v]; gw = v; }
-        const T* prow = s_row[buf][gw];
-        const T piv = prow[k];
-        const bool nz = piv != T(0);
-        const bool doscale = nz && fabs(piv) >= MinNormal<T>::v;
-        if (t == 0) {
-          ipiv[j] = gp + 1;
-          if (!nz && info == 0) info = j + 1;
-          if (gp != j) { const int tmp = s_perm[j]; s_perm[j] = s_perm[gp]; s_perm[gp] = tmp; s_moved = 1; }
-        }
-        const T rinv = doscale ? T(1) / piv : T(1);
-#pragma unroll
-        for (int q = 0; q < RPT; q++) {
-          if (!live[q]) continue;
-          if (pos[q] == gp) pos[q] = j;
-          else if (pos[q] == j) pos[q] = gp;
-          if (pos[q] > j) {
-            T l = pick<RV, W>(x[q], k);
-            if (doscale) l *= rinv;
-#pragma unroll
-            for (int c = 0; c < W; c++) {
-              if (c == k) x[q][c] = l;
-              else if (c > k && c < w) x[q][c] -= l * prow[c];
-            }
-          }
-        }
-      }
-      // panel back to its physical rows; L11 to LDS
-#pragma unroll
-      for (int q = 0; q < RPT; q++) {
-        if (!live[q]) continue;
-#pragma unroll
-        for (int c = 0; c < W; c++)
-          if (c < w) A[phys[q] + (j0 + c) * lda] = x[q][c];
-        const int rr = pos[q] - j0;
-        if (rr < w) {
-#pragma unroll
-          for (int c = 0; c < W; c++)
-            if (c < rr) s_l11[rr * W + c] = x[q][c];
-        }
-      }
-      __syncthreads();
-      #pragma unroll 1
-      for (int c0 = j0 + w; c0 < n; c0 += UB) {
-        const int cw = min(UB, n - c0);
-        if (t < cw) {   // U12 column c0+t: forward substitution with unit L11
-          auto colp = A + (long)(c0 + t) * lda;
-          T u[W];
-#pragma unroll
-          for (int k = 0; k < W; k++) u[k] = (k < w) ? colp[s_perm[j0 + k]] : T(0);
-#pragma unroll
-          for (int kp = 0; kp < W; kp++) {
-            // keep each step's L11 column reads in that step (bounded registers)
-            asm volatile("" ::: "memory");
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int k = kp + 1; k < W; k++)
-              if (k < w) u[k] -= s_l11[k * W + kp] * u[kp];
-          }
-#pragma unroll
-          for (int k = 0; k < W; k++)
-            if (k < w) { colp[s_perm[j0 + k]] = u[k]; s_u[t * LDU + k] = u[k]; }
-        }
-        __syncthreads();
-        if constexpr (RPT == 1) {
-          // A22 -= L21 U12 on MFMA 16x16 tiles (rows: positions >= j0+w at
-          // their physical rows, staged with their multipliers in LDS;
-          // 4 wavefronts, GT tiles per step with their C elements loaded
-          // before the products)
-          typedef BMF<T> mf;
-          const int r0 = j0 + w, nr = m - r0;
-          if (c0 == j0 + w && live[0] && pos[0] >= r0) {   // once per panel
-            s_prow[pos[0] - r0] = phys[0];
-#pragma unroll
-            for (int k = 0; k < W; k++) s_l21[(pos[0] - r0) * LDU + k] = k < w ? x[0][k] : T(0);
-          }
-          __syncthreads();
-          const int ntr = (nr + 15) / 16, ntc = (cw + 15) / 16, ntiles = ntr * ntc;
-          constexpr int GT = 4;
-          #pragma unroll 1
-          for (int tb = wave * GT; tb < ntiles; tb += 4 * GT) {
-            int ti[GT], tj[GT];
-            T cv[GT][4];
-            typename mf::acc acc[GT];
-#pragma unroll
-            for (int g = 0; g < GT; g++) {
-              const int tile = min(tb + g, ntiles - 1);
-              ti[g] = tile % ntr;
-              tj[g] = tile / ntr;
-              const int ri = ti[g] * 16 + (lane & 15);
-              const int pr = ri < nr ? s_prow[ri] : 0;
-#pragma unroll
-              for (int r = 0; r < 4; r++) {
-                const int cc = tj[g] * 16 + mf::orow(lane, r);
-                cv[g][r] = (tb + g < ntiles && ri < nr && cc < cw) ? A[pr + (long)(c0 + cc) * lda] : T(0);
-              }
-            }
-#pragma unroll
-            for (int g = 0; g < GT; g++) {
-              acc[g] = typename mf::acc{T(0), T(0), T(0), T(0)};
-              const int ra = ti[g] * 16 + (lane & 15), cb = tj[g] * 16 + (lane & 15);
-#pragma unroll
-              for (int kk = 0; kk < W; kk += 4) {
-                const int k = kk + (lane >> 4);
-                const T fa = ra < nr ? s_l21[ra * LDU + k] : T(0);
-                const T fb = (cb < cw && k < w) ? s_u[cb * LDU + k] : T(0);
-                acc[g] = mf::mma(fb, fa, acc[g]);
-              }
-            }
-#pragma unroll
-            for (int g = 0; g < GT; g++) {
-              const int ri = ti[g] * 16 + (lane & 15);
-              const int pr = ri < nr ? s_prow[ri] : 0;
-#pragma unroll
-              for (int r = 0; r < 4; r++) {
-                const int cc = tj[g] * 16 + mf::orow(lane, r);
-                if (tb + g < ntiles && ri < nr && cc < cw) A[pr + (long)(c0 + cc) * lda] = cv[g][r] - acc[g][r];
-              }
-            }
-          }
-        } else {
-#pragma unroll
-        for (int q = 0; q < RPT; q++) {
-          if (!live[q] || pos[q] < j0 + w) continue;
-          auto rowp = A + phys[q];
-          // BU columns per step, their loads issued together (one exposed
-          // memory latency per step instead of per column)
-          #pragma unroll 1
-          for (int cb = 0; cb < cw; cb += BU) {
-            T a[BU];
-#pragma unroll
-            for (int u = 0; u < BU; u++) a[u] = cb + u < cw ? rowp[(long)(c0 + cb + u) * lda] : T(0);
-#pragma unroll
-            for (int u = 0; u < BU; u++) {
-              if (cb + u < cw) {
-                const T* uc = s_u + (cb + u) * LDU;
-                T v = a[u];
-#pragma unroll
-                for (int k = 0; k < W; k++)
-                  if (k < w) v -= x[q][k] * uc[k];
-                rowp[(long)(c0 + cb + u) * lda] = v;
-              }
-            }
-          }
-        }
-        }
-        __syncthreads();
-      }
-    }
-    // rows to their final positions (position i <- physical row s_perm[i])
-    if (s_moved) {
-      #pragma unroll 1
-      for (int c0 = 0; c0 < n; c0 += CH) {
-        T v[RPT][CH];
-#pragma unroll
-        for (int q = 0; q < RPT; q++) {
-          const int i = t + NT * q;
-          const int src = i < m ? s_perm[i] : i;
-          if (i < m && src != i) {
-#pragma unroll
-            for (int cc = 0; cc < CH; cc++)
-              if (c0 + cc < n) v[q][cc] = A[src + (c0 + cc) * lda];
-          }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int q = 0; q < RPT; q++) {
-          const int i = t + NT * q;
-          const int src = i < m ? s_perm[i] : i;
-          if (i < m && src != i) {
-#pragma unroll
-            for (int cc = 0; cc < CH; cc++)
-              if (c0 + cc < n) A[i + (c0 + cc) * lda] = v[q][cc];
-          }
-        }
-        __syncthreads();
-      }
-    }
-    if (t == 0) info_out[it] = info;
     __syncthreads();
     cur ^= 1;
     it = s_item[cur];
@@ -914,7 +654,7 @@ typedef void (*Launcher)(const Cfg& c, const void* ctx, const BDesc* tab, const 
 
 void enqueue(Launcher L, const Cfg& c, const void* ctx, const BDesc* tab, const void* extra, int nitems, int count,
              unsigned* ctr, int* info, hipStream_t s) {
-  bzero_kernel<<<1, 64, 0, s>>>(ctr, 1);
+  bzero_kernel<<<1, 64, 0, s>>>(ctr, 4);
   L(c, ctx, tab, extra, nitems, count, ctr, info, s);
 }
 
@@ -1071,22 +811,29 @@ void launch_gemm(const Cfg& c, const void* ctx, const BDesc* tab, const void* ex
   OBA_HIP(hipGetLastError());
 }
 
-template <typename T>
-void launch_getrf(const Cfg& c, const void* ctx, const BDesc* tab, const void*, int, int count, unsigned* ctr,
-                  int* info, hipStream_t s) {
-  const int rpt = ((const int*)ctx)[0];
-  const int g = grid_of(c);
-  // panel width: 8 or 16 columns for FP64 (wider FP64 panels exceed the
-  // register file), 16 or 32 for FP32
-  constexpr int W0 = sizeof(T) == 8 ? 8 : 16;
-  if (rpt == 1) {
-    if (c.var == 0) bgetrf_kernel<T, 1, W0><<<g, 256, 0, s>>>(tab, count, ctr, info);
-    else bgetrf_kernel<T, 1, 2 * W0><<<g, 256, 0, s>>>(tab, count, ctr, info);
-  } else {
-    if (c.var == 0) bgetrf_kernel<T, 2, W0><<<g, 256, 0, s>>>(tab, count, ctr, info);
-    else bgetrf_kernel<T, 2, 2 * W0><<<g, 256, 0, s>>>(tab, count, ctr, info);
-  }
+// one launch per size class: problems of up to 64, 128, 256 and 512 rows take
+// as many threads as they have rows
+template <typename T, int NWV>
+void launch_getrf_class(const BDesc* tab, int first, int last, unsigned* ctr, int* info, hipStream_t s) {
+  if (first == last) return;
+  static const int per_cu = [] {
+    int n = 0;
+    OBA_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, bgetrf_kernel<T, NWV>, 64 * NWV, 0));
+    return std::max(n, 1);
+  }();
+  const int g = std::min(last - first, rt().num_cu * per_cu);
+  bgetrf_kernel<T, NWV><<<g, 64 * NWV, 0, s>>>(tab + first, last - first, ctr, info + first);
   OBA_HIP(hipGetLastError());
+}
+
+template <typename T>
+void launch_getrf(const Cfg&, const void* ctx, const BDesc* tab, const void*, int, int count, unsigned* ctr,
+                  int* info, hipStream_t s) {
+  const int* end = (const int*)ctx;   // the classes' ends in the table, largest class first
+  launch_getrf_class<T, 8>(tab, 0, end[0], ctr, info, s);
+  launch_getrf_class<T, 4>(tab, end[0], end[1], ctr + 1, info, s);
+  launch_getrf_class<T, 2>(tab, end[1], end[2], ctr + 2, info, s);
+  launch_getrf_class<T, 1>(tab, end[2], count, ctr + 3, info, s);
 }
 
 template <typename T>
@@ -1167,16 +914,13 @@ void getrf_batched(std::vector<BDesc>& probs, int* info_host) {
   std::vector<BDesc> small, big;
   for (auto& d : probs) (d.m <= 512 ? small : big).push_back(d);
   if (!small.empty()) {
-    int mx = 0;
-    for (auto& d : small) mx = std::max(mx, d.m);
-    const int ctx[1] = {mx <= 256 ? 1 : 2};
-    std::vector<Cfg> cands;
-    for (int v = 0; v < 2; v++)
-      for (int g : {1, 2, 4}) cands.push_back(Cfg{v, g});
+    auto cls = [](const BDesc& d) { return d.m > 256 ? 0 : d.m > 128 ? 1 : d.m > 64 ? 2 : 3; };
+    std::stable_sort(small.begin(), small.end(), [&](const BDesc& x, const BDesc& y) { return cls(x) < cls(y); });
+    int ctx[3] = {0, 0, 0};
+    for (auto& d : small)
+      for (int k = cls(d); k < 3; k++) ctx[k]++;
     const std::vector<char> none;
-    Cfg c = tune(signature(BK_GETRF, sizeof(T), ctx[0], small), cands, launch_getrf<T>, ctx, small, none, 0, 0, 0, 1,
-                 sizeof(T));
-    if (const char* e = getenv("OPENBLAS_AMD_BATCH_LU_W")) c.var = atoi(e) == 32 ? 1 : 0;
+    const Cfg c;
     double fl = 0, by = 0;
     for (auto& d : small) {
       const double mm = d.m, nn = d.n, k = std::min(mm, nn);

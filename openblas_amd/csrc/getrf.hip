@@ -29,6 +29,7 @@
 #include "kernels.h"
 #include "lu_internal.h"
 #include "lu_device.h"
+#include "lu_key.h"
 #include <cfloat>
 #include <climits>
 #include <cmath>
