@@ -11,8 +11,8 @@
 //    (GEMM tiles, LU, Cholesky) or wavefronts (solves) pull the next item
 //    from an atomic queue, so 10^4 uneven problems keep all 256 CUs busy
 //    without one launch per problem;
-//  * GEMM: BT x BT output tiles (BT = 32 or 64) on the FP64/FP32 16x16x4
-//    MFMA, k-slabs staged through LDS;
+//  * GEMM: 64- and 32-wide output tiles with the single GEMM's loads and main
+//    loop, one queue per XCD;
 //  * LU (m <= 512): batched_lu.h, one launch per size class;
 //  * Cholesky (n <= 512): same row-owner panel, one barrier per column,
 //    SYRK-shaped trailing update of the lower triangle;
@@ -28,6 +28,7 @@
 #include "kernels.h"
 #include "lu_device.h"
 #include "lu_internal.h"
+#include "gemm_tile.h"
 #include <algorithm>
 #include <climits>
 #include <cstring>
@@ -47,6 +48,7 @@ using gptr = __attribute__((address_space(1))) T*;
 
 }  // namespace oba
 
+#include "batched_gemm.h"
 #include "batched_lu.h"
 
 namespace oba {
@@ -110,121 +112,6 @@ template <> struct BMF<float> {
   }
   __device__ static inline int orow(int l, int r) { return 4 * (l >> 4) + r; }
 };
-
-// work[i] = (problem, 64x64 tile of C) in launch order; per queue item one
-// workgroup computes that tile of C = alpha*op(A)*op(B) + beta*C, as one
-// 64-wide tile (BT = 64) or as its up to four 32-wide quarters that
-// intersect C (BT = 32, less padding for small problems)
-template <typename T, int BT, bool TA, bool TB>
-__global__ __launch_bounds__(256) void bgemm_kernel(const BDesc* __restrict__ desc, const int2* __restrict__ work,
-                                                    int nwork, unsigned* __restrict__ counter) {
-  constexpr int BK = 16, PAD = 16, LDS_ = BT + PAD;
-  constexpr int WT = BT / 2, F = WT / 16, NE = BT * BK / 256;
-  typedef BMF<T> mf;
-  typedef typename mf::acc acc_t;
-  __shared__ T sa[BK * LDS_];
-  __shared__ T sb[BK * LDS_];
-  __shared__ int s_item[2];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm0 = (wave & 1) * WT, wn0 = (wave >> 1) * WT;
-
-  if (tid == 0) s_item[0] = (int)atomicAdd(counter, 1u);
-  __syncthreads();
-  int cur = 0;
-  int it = s_item[0];
-  while (it < nwork) {
-    if (tid == 0) s_item[cur ^ 1] = (int)atomicAdd(counter, 1u);   // next item, read after the last barrier
-    const int2 wk = work[it];
-    const BDesc& d = desc[wk.x];
-    const long M = d.m, N = d.n, K = d.k, lda = d.lda, ldb = d.ldb, ldc = d.ldc;
-    gptr<const T> A = (gptr<const T>)d.a;
-    gptr<const T> B = (gptr<const T>)d.b;
-    gptr<T> C = (gptr<T>)d.c;
-    const T alpha = (T)d.alpha, beta = (T)d.beta;
-    const int st_m = (int)((M + 63) / 64);
-    const long sm0 = (long)(wk.y % st_m) * 64, sn0 = (long)(wk.y / st_m) * 64;
-    for (int sub = 0; sub < (BT == 64 ? 1 : 4); sub++) {
-      const long m0 = sm0 + (BT == 64 ? 0 : (sub & 1) * 32), n0 = sn0 + (BT == 64 ? 0 : (sub >> 1) * 32);
-      if (m0 >= M || n0 >= N) continue;   // uniform
-
-      acc_t acc[F][F];
-#pragma unroll
-      for (int i = 0; i < F; i++)
-#pragma unroll
-        for (int j = 0; j < F; j++) acc[i][j] = acc_t{};
-
-      if (alpha != T(0)) {
-        T ra[NE], rb[NE];
-        auto load = [&](long k0) __attribute__((always_inline)) {
-#pragma unroll
-          for (int e = 0; e < NE; e++) {
-            const int v = tid + e * 256;
-            int i, kk;
-            if (!TA) { i = v % BT; kk = v / BT; } else { kk = v % BK; i = v / BK; }
-            const long gi = m0 + i, gk = k0 + kk;
-            ra[e] = (gi < M && gk < K) ? (TA ? A[gk + gi * lda] : A[gi + gk * lda]) : T(0);
-            int j, kb;
-            if (!TB) { kb = v % BK; j = v / BK; } else { j = v % BT; kb = v / BT; }
-            const long gj = n0 + j, gkb = k0 + kb;
-            rb[e] = (gj < N && gkb < K) ? (TB ? B[gj + gkb * ldb] : B[gkb + gj * ldb]) : T(0);
-          }
-        };
-        auto store = [&]() __attribute__((always_inline)) {
-#pragma unroll
-          for (int e = 0; e < NE; e++) {
-            const int v = tid + e * 256;
-            int i, kk;
-            if (!TA) { i = v % BT; kk = v / BT; } else { kk = v % BK; i = v / BK; }
-            sa[kk * LDS_ + i] = ra[e];
-            int j, kb;
-            if (!TB) { kb = v % BK; j = v / BK; } else { j = v % BT; kb = v / BT; }
-            sb[kb * LDS_ + j] = rb[e];
-          }
-        };
-        load(0);
-        for (long k0 = 0; k0 < K; k0 += BK) {
-          store();
-          __syncthreads();
-          if (k0 + BK < K) load(k0 + BK);   // next slab in flight during the MFMAs
-#pragma unroll
-          for (int kk = 0; kk < BK / 4; kk++) {
-            const int kr = kk * 4 + (lane >> 4);
-            T fa[F], fb[F];
-#pragma unroll
-            for (int i = 0; i < F; i++) fa[i] = sa[kr * LDS_ + wm0 + i * 16 + (lane & 15)];
-#pragma unroll
-            for (int j = 0; j < F; j++) fb[j] = sb[kr * LDS_ + wn0 + j * 16 + (lane & 15)];
-#pragma unroll
-            for (int i = 0; i < F; i++)
-#pragma unroll
-              for (int j = 0; j < F; j++) acc[i][j] = mf::mma(fb[j], fa[i], acc[i][j]);
-          }
-          __syncthreads();
-        }
-      }
-      const bool bz = beta == T(0);
-#pragma unroll
-      for (int i = 0; i < F; i++) {
-        const long m = m0 + wm0 + i * 16 + (lane & 15);
-#pragma unroll
-        for (int j = 0; j < F; j++)
-#pragma unroll
-          for (int r = 0; r < 4; r++) {
-            const long n = n0 + wn0 + j * 16 + mf::orow(lane, r);
-            if (m < M && n < N) {
-              auto p = C + m + n * ldc;
-              T v = alpha * acc[i][j][r];
-              if (!bz) v += beta * *p;
-              *p = v;
-            }
-          }
-      }
-    }
-    __syncthreads();
-    cur ^= 1;
-    it = s_item[cur];
-  }
-}
 
 // ---- batched Cholesky (n <= 256*RPT) -------------------------------------------
 // LOWER: A = L*L^T with L(i,c) = a[i + c*lda]; upper: A = U^T*U, U = L^T,
@@ -654,7 +541,7 @@ typedef void (*Launcher)(const Cfg& c, const void* ctx, const BDesc* tab, const 
 
 void enqueue(Launcher L, const Cfg& c, const void* ctx, const BDesc* tab, const void* extra, int nitems, int count,
              unsigned* ctr, int* info, hipStream_t s) {
-  bzero_kernel<<<1, 64, 0, s>>>(ctr, 4);
+  bzero_kernel<<<1, 64, 0, s>>>(ctr, 8);
   L(c, ctx, tab, extra, nitems, count, ctr, info, s);
 }
 
@@ -789,26 +676,26 @@ std::string signature(int kind, size_t elem, int flags, const std::vector<BDesc>
 int grid_of(const Cfg& c) { return std::max(1, rt().num_cu * c.grid); }
 
 // ---- launchers ---------------------------------------------------------------
+template <typename T, bool TA, bool TB>
+void launch_gemm_form(const BDesc* tab, const void* extra, int nitems, unsigned* ctr, hipStream_t s) {
+  static const int per_cu = [] {
+    int n = 0;
+    OBA_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, bgemm_kernel<T, TA, TB>, 256, 0));
+    return std::max(n, 1);
+  }();
+  const BSeg* seg = (const BSeg*)extra;
+  bgemm_kernel<T, TA, TB><<<std::min(nitems, rt().num_cu * per_cu), 256, 0, s>>>(tab, seg, (const int2*)(seg + 1), ctr);
+  OBA_HIP(hipGetLastError());
+}
+
 template <typename T>
-void launch_gemm(const Cfg& c, const void* ctx, const BDesc* tab, const void* extra, int nitems, int, unsigned* ctr,
+void launch_gemm(const Cfg&, const void* ctx, const BDesc* tab, const void* extra, int nitems, int, unsigned* ctr,
                  int*, hipStream_t s) {
   const int ta = ((const int*)ctx)[0], tb = ((const int*)ctx)[1];
-  const int2* work = (const int2*)extra;
-  const int g = grid_of(c);
-#define OBA_BG(BT, TA, TB) bgemm_kernel<T, BT, TA, TB><<<g, 256, 0, s>>>(tab, work, nitems, ctr)
-  if (c.var == 0) {
-    if (!ta && !tb) OBA_BG(32, false, false);
-    else if (!ta && tb) OBA_BG(32, false, true);
-    else if (ta && !tb) OBA_BG(32, true, false);
-    else OBA_BG(32, true, true);
-  } else {
-    if (!ta && !tb) OBA_BG(64, false, false);
-    else if (!ta && tb) OBA_BG(64, false, true);
-    else if (ta && !tb) OBA_BG(64, true, false);
-    else OBA_BG(64, true, true);
-  }
-#undef OBA_BG
-  OBA_HIP(hipGetLastError());
+  if (!ta && !tb) launch_gemm_form<T, false, false>(tab, extra, nitems, ctr, s);
+  else if (!ta && tb) launch_gemm_form<T, false, true>(tab, extra, nitems, ctr, s);
+  else if (ta && !tb) launch_gemm_form<T, true, false>(tab, extra, nitems, ctr, s);
+  else launch_gemm_form<T, true, true>(tab, extra, nitems, ctr, s);
 }
 
 // one launch per size class: problems of up to 64, 128, 256 and 512 rows take
@@ -884,22 +771,21 @@ void collect_info(const int* dinfo, const std::vector<BDesc>& probs, int* info_h
 template <typename T>
 void gemm_batched(int ta, int tb, std::vector<BDesc>& probs) {
   if (probs.empty()) return;
-  // work list: every 64x64 tile of every C, problems in the given order
-  std::vector<int> v;
-  for (size_t p = 0; p < probs.size(); p++) {
-    const long tm = (probs[p].m + 63) / 64, tn = (probs[p].n + 63) / 64;
-    for (long t = 0; t < tm * tn; t++) { v.push_back((int)p); v.push_back((int)t); }
-  }
-  std::vector<char> wl(v.size() * sizeof(int));
-  memcpy(wl.data(), v.data(), wl.size());
-  const int nw = (int)(v.size() / 2);
+  // work list: the tiles of every C, problem p's in segment p % 8
+  BSeg seg{};
+  std::vector<int> tiles(probs.size());
+  int len[8] = {};
+  for (size_t p = 0; p < probs.size(); p++) len[p & 7] += tiles[p] = bgemm_tiles(probs[p].m) * bgemm_tiles(probs[p].n);
+  for (int x = 0; x < 8; x++) seg.begin[x + 1] = seg.begin[x] + len[x];
+  const int nw = seg.begin[8];
+  std::vector<char> wl(sizeof(BSeg) + sizeof(int2) * (size_t)nw);
+  memcpy(wl.data(), &seg, sizeof seg);
+  int2* at[8];
+  for (int x = 0; x < 8; x++) at[x] = (int2*)(wl.data() + sizeof(BSeg)) + seg.begin[x];
+  for (size_t p = 0; p < probs.size(); p++)
+    for (int t = 0; t < tiles[p]; t++) *at[p & 7]++ = make_int2((int)p, t);
   const int ctx[2] = {ta, tb};
-  std::vector<Cfg> cands;
-  for (int var = 0; var < 2; var++)
-    for (int g : {2, 4, 8}) cands.push_back(Cfg{var, g});
-  Cfg c = tune(signature(BK_GEMM, sizeof(T), ta | (tb << 1), probs), cands, launch_gemm<T>, ctx, probs, wl, nw, 2, 0,
-               1, sizeof(T));
-  if (const char* e = getenv("OPENBLAS_AMD_BATCH_GEMM_TILE")) c.var = atoi(e) == 64 ? 1 : 0;
+  const Cfg c;
   double fl = 0, by = 0;
   for (auto& d : probs) {
     fl += 2.0 * d.m * d.n * d.k;
