@@ -513,7 +513,9 @@ struct Cfg {
 };
 
 struct Plan {
-  std::vector<char> key;
+  Cfg cfg;
+  std::vector<char> ctx;
+  std::vector<BDesc> probs;   // the table on the device; empty: none
   DevBuf tab;       // BDesc table (+ GEMM work list)
   DevBuf ctr;       // queue counter
   DevBuf info;      // per-problem info
@@ -545,30 +547,31 @@ void enqueue(Launcher L, const Cfg& c, const void* ctx, const BDesc* tab, const 
   L(c, ctx, tab, extra, nitems, count, ctr, info, s);
 }
 
-// Runs the batch described by host bytes `tab` (BDesc[count], then `extra`
-// bytes) through the cached graph of plan slot `slot`, re-capturing only
-// when the table or config changed.  Returns the device info array.
+// Runs the batch `probs` through the cached graph of plan slot `slot`,
+// re-capturing only when the table or config changed; `extra` makes the bytes
+// that follow the table on the device and is only called then (the comparison
+// and the work list took most of a call's 1 ms on the host at 10^4 problems).
+// Returns the device info array.
+template <typename Extra>
 int* run_plan(int slot, Launcher L, const Cfg& c, const void* ctx, size_t ctx_bytes, const std::vector<BDesc>& probs,
-              const std::vector<char>& extra, int nitems) {
+              int nitems, const Extra& make_extra) {
   Runtime& r = rt();
   Plan& P = plans()[slot];
   const int count = (int)probs.size();
   const size_t tb = sizeof(BDesc) * probs.size();
-  std::vector<char> key(sizeof(Cfg) + ctx_bytes + tb + extra.size());
-  memcpy(key.data(), &c, sizeof(Cfg));
-  if (ctx_bytes) memcpy(key.data() + sizeof(Cfg), ctx, ctx_bytes);
-  memcpy(key.data() + sizeof(Cfg) + ctx_bytes, probs.data(), tb);
-  if (!extra.empty()) memcpy(key.data() + sizeof(Cfg) + ctx_bytes + tb, extra.data(), extra.size());
   const bool use_graph = env_flag("OPENBLAS_AMD_BATCH_GRAPH", true);
-  if (P.exec && use_graph && key == P.key) {
+  if (P.exec && use_graph && P.cfg.var == c.var && P.cfg.grid == c.grid && P.ctx.size() == ctx_bytes &&
+      memcmp(P.ctx.data(), ctx, ctx_bytes) == 0 && P.probs.size() == probs.size() &&
+      memcmp(P.probs.data(), probs.data(), tb) == 0) {
     OBA_HIP(hipGraphLaunch(P.exec, r.stream));
     return P.info.as<int>();
   }
+  const std::vector<char> extra = make_extra();
   // the previous graph may still run from the last call: let it finish
   // before its table goes back to the pool
   OBA_HIP(hipStreamSynchronize(r.stream));
   if (P.exec) { OBA_HIP(hipGraphExecDestroy(P.exec)); P.exec = nullptr; }
-  P.key.clear();
+  P.probs.clear();
   P.tab = DevBuf(tb + extra.size() + 16);
   P.ctr = DevBuf(256);
   P.info = DevBuf(sizeof(int) * (size_t)std::max(count, 1));
@@ -587,7 +590,9 @@ int* run_plan(int slot, Launcher L, const Cfg& c, const void* ctx, size_t ctx_by
   OBA_HIP(hipStreamEndCapture(r.stream, &g));
   OBA_HIP(hipGraphInstantiate(&P.exec, g, nullptr, nullptr, 0));
   OBA_HIP(hipGraphDestroy(g));
-  P.key.swap(key);
+  P.cfg = c;
+  P.ctx.assign((const char*)ctx, (const char*)ctx + ctx_bytes);
+  P.probs = probs;
   OBA_HIP(hipGraphLaunch(P.exec, r.stream));
   return P.info.as<int>();
 }
@@ -672,6 +677,8 @@ std::string signature(int kind, size_t elem, int flags, const std::vector<BDesc>
   snprintf(b, sizeof b, "%d/%zu/%d/%d/%ld/%d", kind, elem, flags, lc, (mx + 31) / 32, lw);
   return b;
 }
+
+std::vector<char> no_extra() { return {}; }
 
 int grid_of(const Cfg& c) { return std::max(1, rt().num_cu * c.grid); }
 
@@ -773,17 +780,21 @@ void gemm_batched(int ta, int tb, std::vector<BDesc>& probs) {
   if (probs.empty()) return;
   // work list: the tiles of every C, problem p's in segment p % 8
   BSeg seg{};
-  std::vector<int> tiles(probs.size());
   int len[8] = {};
-  for (size_t p = 0; p < probs.size(); p++) len[p & 7] += tiles[p] = bgemm_tiles(probs[p].m) * bgemm_tiles(probs[p].n);
+  for (size_t p = 0; p < probs.size(); p++) len[p & 7] += bgemm_tiles(probs[p].m) * bgemm_tiles(probs[p].n);
   for (int x = 0; x < 8; x++) seg.begin[x + 1] = seg.begin[x] + len[x];
   const int nw = seg.begin[8];
-  std::vector<char> wl(sizeof(BSeg) + sizeof(int2) * (size_t)nw);
-  memcpy(wl.data(), &seg, sizeof seg);
-  int2* at[8];
-  for (int x = 0; x < 8; x++) at[x] = (int2*)(wl.data() + sizeof(BSeg)) + seg.begin[x];
-  for (size_t p = 0; p < probs.size(); p++)
-    for (int t = 0; t < tiles[p]; t++) *at[p & 7]++ = make_int2((int)p, t);
+  auto work = [&]() {
+    std::vector<char> wl(sizeof(BSeg) + sizeof(int2) * (size_t)nw);
+    memcpy(wl.data(), &seg, sizeof seg);
+    int2* at[8];
+    for (int x = 0; x < 8; x++) at[x] = (int2*)(wl.data() + sizeof(BSeg)) + seg.begin[x];
+    for (size_t p = 0; p < probs.size(); p++) {
+      const int tiles = bgemm_tiles(probs[p].m) * bgemm_tiles(probs[p].n);
+      for (int t = 0; t < tiles; t++) *at[p & 7]++ = make_int2((int)p, t);
+    }
+    return wl;
+  };
   const int ctx[2] = {ta, tb};
   const Cfg c;
   double fl = 0, by = 0;
@@ -792,20 +803,22 @@ void gemm_batched(int ta, int tb, std::vector<BDesc>& probs) {
     by += sizeof(T) * ((double)d.m * d.k + (double)d.k * d.n + (d.beta != 0.0 ? 2.0 : 1.0) * d.m * d.n);
   }
   KTimer kt("batched_gemm", rt().stream, fl, by);
-  run_plan(tslot<T>(BK_GEMM), launch_gemm<T>, c, ctx, sizeof ctx, probs, wl, nw);
+  run_plan(tslot<T>(BK_GEMM), launch_gemm<T>, c, ctx, sizeof ctx, probs, nw, work);
 }
 
 template <typename T>
 void getrf_batched(std::vector<BDesc>& probs, int* info_host) {
+  // the kernel's size classes, largest first, each in the order given
+  auto cls = [](const BDesc& d) { return d.m > 512 ? 4 : d.m > 256 ? 0 : d.m > 128 ? 1 : d.m > 64 ? 2 : 3; };
   std::vector<BDesc> small, big;
-  for (auto& d : probs) (d.m <= 512 ? small : big).push_back(d);
+  small.reserve(probs.size());
+  int ctx[3] = {0, 0, 0};
+  for (int k = 0; k <= 4; k++) {
+    for (auto& d : probs)
+      if (cls(d) == k) (k < 4 ? small : big).push_back(d);
+    if (k < 3) ctx[k] = (int)small.size();
+  }
   if (!small.empty()) {
-    auto cls = [](const BDesc& d) { return d.m > 256 ? 0 : d.m > 128 ? 1 : d.m > 64 ? 2 : 3; };
-    std::stable_sort(small.begin(), small.end(), [&](const BDesc& x, const BDesc& y) { return cls(x) < cls(y); });
-    int ctx[3] = {0, 0, 0};
-    for (auto& d : small)
-      for (int k = cls(d); k < 3; k++) ctx[k]++;
-    const std::vector<char> none;
     const Cfg c;
     double fl = 0, by = 0;
     for (auto& d : small) {
@@ -816,7 +829,7 @@ void getrf_batched(std::vector<BDesc>& probs, int* info_host) {
     const int* di;
     {
       KTimer kt("batched_getrf", rt().stream, fl, by);
-      di = run_plan(tslot<T>(BK_GETRF), launch_getrf<T>, c, ctx, sizeof ctx, small, none, 0);
+      di = run_plan(tslot<T>(BK_GETRF), launch_getrf<T>, c, ctx, sizeof ctx, small, 0, no_extra);
     }
     collect_info(di, small, info_host);
   }
@@ -846,7 +859,7 @@ void potrf_batched(bool lower, std::vector<BDesc>& probs, int* info_host) {
     const int* di;
     {
       KTimer kt("batched_potrf", rt().stream, fl, by);
-      di = run_plan(tslot<T>(BK_POTRF), launch_potrf<T>, c, ctx, sizeof ctx, small, none, 0);
+      di = run_plan(tslot<T>(BK_POTRF), launch_potrf<T>, c, ctx, sizeof ctx, small, 0, no_extra);
     }
     collect_info(di, small, info_host);
   }
@@ -874,7 +887,7 @@ void getrs_batched(bool trans, std::vector<BDesc>& probs, int* info_host) {
       by += sizeof(T) * ((double)d.n * d.n + 2.0 * d.n * std::max(d.k, 0));
     }
     KTimer kt("batched_getrs", rt().stream, fl, by);
-    run_plan(tslot<T>(BK_GETRS), launch_getrs<T>, c, ctx, sizeof ctx, small, none, 0);
+    run_plan(tslot<T>(BK_GETRS), launch_getrs<T>, c, ctx, sizeof ctx, small, 0, no_extra);
   }
   for (auto& d : big) {   // large problems: the single-problem solve
     Runtime& r = rt();
