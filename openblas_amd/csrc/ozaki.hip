@@ -30,6 +30,7 @@
 namespace oba {
 
 typedef int i4v __attribute__((ext_vector_type(4)));
+typedef unsigned u4v __attribute__((ext_vector_type(4)));
 constexpr int OZ_SMAX = 12;     // slices supported by the fused kernel
 constexpr int OZ_NONFINITE = -2;   // return code: NaN/Inf operand, native GEMM used
 constexpr int OZ_BK = 64;       // k per slab (one i8 MFMA k-depth)
@@ -479,7 +480,7 @@ int ozaki_dgemm(bool ta, bool tb, long M, long N, long K, double alpha, const do
 constexpr int CRT_NMAX = 30;    // moduli in the table
 constexpr int CRT_LIMBS = 8;    // 32-bit limbs of the sums: S < NM * 256 * P < 2^256
 constexpr int CRT_T = 256;      // operand padding: a multiple of every GEMM tile edge
-constexpr long CRT_KCHUNK = 131008;   // k per GEMM launch: 131008 * 128^2 < 2^31
+constexpr long CRT_KCHUNK = 16384;    // k per GEMM launch: sums up to 16384 * 128^2 = 2^28 (crt_mod)
 constexpr double CRT_KEEP = 53.0;     // bits kept below the typical entry of each operand
 // pairwise coprime, largest first (greedy from 256 down)
 static const int kCrtModuli[CRT_NMAX] = {256, 255, 253, 251, 247, 241, 239, 233, 229, 227, 223, 217, 211, 199, 197,
@@ -491,7 +492,7 @@ struct CrtTab {
   int p[CRT_NMAX];
   double invp[CRT_NMAX];
   float invpf[CRT_NMAX];
-  int c18[CRT_NMAX][CRT_PIECES];                     // 2^(18 i) mod p
+  int c18[CRT_NMAX][CRT_PIECES];                     // 2^(18 i) mod p, balanced
   unsigned q[CRT_NMAX + 1][CRT_NMAX][CRT_LIMBS];     // Q_m for the first NM moduli (32-bit limbs)
   unsigned short q16[CRT_NMAX + 1][CRT_NMAX][CRT_L16];   // the same in 16-bit limbs
   unsigned short P16[CRT_NMAX + 1][CRT_L16];         // product of the first NM moduli
@@ -534,7 +535,7 @@ static const CrtTab& crt_host_tab() {
     T.invp[m] = 1.0 / p;
     T.invpf[m] = 1.0f / (float)p;
     long v = 1 % p;
-    for (int i = 0; i < CRT_PIECES; i++) { T.c18[m][i] = (int)v; v = (v * (1L << 18)) % p; }
+    for (int i = 0; i < CRT_PIECES; i++) { T.c18[m][i] = (int)(v > p / 2 ? v - p : v); v = (v * (1L << 18)) % p; }
   }
   for (int nm = 1; nm <= CRT_NMAX; nm++) {
     Big P{1u};
@@ -581,15 +582,36 @@ static const CrtTab* crt_dev_tab(hipStream_t s) {
   return (const CrtTab*)d;
 }
 
+// x mod p in [0, p) for |x| <= 2^28 + 2^9 and 113 <= p <= 256.  The FP32
+// quotient y is off by less than 0.34 (x rounded to 24 bits: 8/p; 1/p: 2^-24 of
+// up to 2^21.2; its own rounding: 1/8), so q = round(y - 0.9) lies between
+// y - 1.74 and y - 0.06 and x - q p in (0, 2p): one conditional step.  Rounding
+// is the addition of 1.5 * 2^23; the sum's low 24 bits are 2^22 + q, which the
+// 24-bit product takes as they are, and k = 2^22 p takes the offset out again.
+struct CrtMod {
+  int p, k;
+  float ip;
+  __device__ inline CrtMod(const CrtTab* tab, int m) : p(tab->p[m]), k(tab->p[m] << 22), ip(tab->invpf[m]) {}
+};
+__device__ __attribute__((always_inline)) inline unsigned crt_mod(int x, const CrtMod& m) {
+  const float q = __builtin_fmaf((float)x, m.ip, -0.9f) + 12582912.0f;
+  const unsigned t = (unsigned)x - (__float_as_uint(q) & 0xFFFFFFu) * ((unsigned)m.p & 0x1FFu);
+  return min(t + (unsigned)m.k, t + (unsigned)(m.k - m.p));
+}
+// product of two integers that fit in 24 bits
+__device__ __attribute__((always_inline)) inline int crt_mul24(int a, int b) { return ((a << 8) >> 8) * ((b << 8) >> 8); }
+
 // Residues of the scaled operand: a 64(v) x 64(k) tile through LDS, then
 // every thread takes 16 consecutive k of one vector and writes their
 // balanced residues for each of the NM moduli (R[m][v][k], k contiguous).
 // x' = trunc(|x| 2^(t-e_v)) < 2^t is cut into 18-bit pieces x_i (exact FP64
 // steps: the scaled double is exact, floor of it exact, and the difference
-// of two doubles within 2^18 of each other exact), once per element; per
-// modulus x' mod p = (sum_i x_i (2^(18 i) mod p)) mod p, a sum of 24-bit
-// integer products below 2^30, reduced with an FP32 quotient estimate and
-// one correction step each way.
+// of two doubles within 2^18 of each other exact), once per element, the
+// pieces taking its sign; per modulus the balanced residue of
+// sum_i x_i (2^(18 i) mod p), a sum of 24-bit integer products (eight stay below
+// 2^28, a longer sum is reduced in between).  Bound by these integer steps, 13
+// per residue: 8192^2 and 17 moduli 540 us, 938 with unsigned
+// pieces, a quotient estimate good to 2 and five correction steps.
 template <int NP>
 __global__ __launch_bounds__(256) void crt_split_kernel(long V, long K, const double* __restrict__ X, long sv, long sk,
                                                         const double* __restrict__ vmax, int t, int NM,
@@ -617,25 +639,23 @@ __global__ __launch_bounds__(256) void crt_split_kernel(long V, long K, const do
   const int vv = threadIdx.x >> 2, kq = (threadIdx.x & 3) * 16;
   const long v = v0 + vv;
   const int e = (v < V) ? oz_exp(vmax[v]) : 0;
-  unsigned pc[16][NP];   // 18-bit pieces, least significant first
-  unsigned neg = 0;
+  int pc[16][NP];   // 18-bit pieces, least significant first
 #pragma unroll
   for (int c = 0; c < 16; c++) {
-    double y = ldexp(tile[vv][kq + c], t - e);
-    if (y < 0.0) { neg |= 1u << c; y = -y; }
-    y = trunc(y);
+    const double x = ldexp(tile[vv][kq + c], t - e);
+    const double y = trunc(fabs(x));
     // from the top piece down: hi = floor(y / 2^(18 i)), piece = hi - 2^18 floor(hi / 2^18)
 #pragma unroll
     for (int i = NP - 1; i >= 0; i--) {
       const double hi = floor(ldexp(y, -18 * i));
       const double up = floor(hi * 0x1p-18);
-      pc[c][i] = (unsigned)(hi - up * 0x1p18);
+      const int v = (int)(hi - up * 0x1p18);
+      pc[c][i] = x < 0.0 ? -v : v;
     }
   }
   for (int m = 0; m < NM; m++) {
-    const int p = tab->p[m];
-    const float ipf = tab->invpf[m];
-    const int half = (p + 1) / 2;
+    const CrtMod md(tab, m);
+    const int half = (md.p - 1) / 2;
     int cm[NP];
 #pragma unroll
     for (int i = 0; i < NP; i++) cm[i] = tab->c18[m][i];
@@ -646,19 +666,14 @@ __global__ __launch_bounds__(256) void crt_split_kernel(long V, long K, const do
 #pragma unroll
       for (int b = 0; b < 4; b++) {
         const int c = q4 * 4 + b;
-        unsigned a = 0;
+        int a = half;
 #pragma unroll
-        for (int i = 0; i < NP; i++) a = __umul24(pc[c][i], (unsigned)cm[i]) + a;   // < NP 2^26
-        // the FP32 quotient is within 2 of the true one for a < 2^30
-        int r = (int)a - (int)floorf((float)a * ipf) * p;
-        if (r < 0) r += p;
-        if (r < 0) r += p;
-        if (r >= p) r -= p;
-        if (r >= p) r -= p;
-        if (r >= half) r -= p;   // balanced: [-(p-1)/2, (p-1)/2], [-128, 127] for 256
-        if ((neg >> c) & 1u) r = -r;
-        if (r == 128) r = -128;   // p = 256: 128 = -128 (mod 256)
-        word |= ((unsigned)r & 0xFFu) << (8 * b);
+        for (int i = 0; i < NP; i++) {
+          if (i == 8) a = (int)crt_mod(a, md);
+          a += crt_mul24(pc[c][i], cm[i]);
+        }
+        // balanced: [-(p-1)/2, (p-1)/2], for 256 [-127, 128] whose 128 the byte takes as -128
+        word |= ((crt_mod(a, md) - (unsigned)half) & 0xFFu) << (8 * b);
       }
       w[q4] = (int)word;
     }
@@ -666,18 +681,30 @@ __global__ __launch_bounds__(256) void crt_split_kernel(long V, long K, const do
   }
 }
 
+// LDS byte offset of chunk c of row r of an A slab whose fragments take 4 rows
+// out of every GAP: rows of one fragment read differ in bits 0, 1 and r / GAP
+template <int GAP>
+__device__ __attribute__((always_inline)) inline int crt_lds_off(int r, int c) {
+  return r * 64 + ((c ^ (((r >> 1) ^ (r / GAP)) & 3)) << 4);
+}
+
 // One INT8 GEMM per modulus (blockIdx.y): a (32 FA) x (32 FB) tile of the
 // residue product, four wavefronts of (16 FA) x (16 FB) (FA x FB MFMA
-// blocks each), 64-deep k slabs double-buffered in LDS (the slice kernel's
-// swizzled layout), the next slab's loads in flight during the MFMAs.  The
-// exact int32 sums are reduced mod p_m and stored as balanced int8
-// residues of C (RC[m][j][i], i contiguous); with `accumulate` the launch
-// adds to the residues of the previous k chunk.
+// blocks each).  64-deep k slabs double-buffered in LDS; the fragments of a
+// slab are read into registers while the slab before is multiplied, and the
+// slab after the next is on its way from memory, so a step has one barrier
+// and nothing in front of its MFMAs.  The exact int32 sums are reduced mod p_m
+// and stored as residues in [0, p_m) (RC[m][j][i], i contiguous); a lane's
+// fragment rows are spaced so that it ends with 4 FA consecutive rows of a
+// column, stored 16 bytes at a time.  With `accumulate` the launch adds to the
+// residues of the previous k chunk.  8192^3, 17 moduli: 10.9 ms (1.72 POP/s);
+// 12.05 with the fragments read in front of their own MFMAs, an FP64 remainder
+// and single-byte stores.  One wavefront per SIMD (256 accumulators a lane).
 template <int FA, int FB>
-__global__ __launch_bounds__(256) void crt_gemm_kernel(long M, long N, long Kc, long Kp, long k_off,
+__global__ __launch_bounds__(256) void crt_gemm_kernel(long N, long Kc, long Kp, long k_off,
                                                        const signed char* __restrict__ RA, long Mp,
                                                        const signed char* __restrict__ RB, long Np,
-                                                       const CrtTab* __restrict__ tab, signed char* __restrict__ RC,
+                                                       const CrtTab* __restrict__ tab, unsigned char* __restrict__ RC,
                                                        long ldrc, long plane, int accumulate) {
   constexpr int BM = 32 * FA, BN = 32 * FB;
   constexpr int LA = BM / 64, LB = BN / 64;   // 16-byte loads per thread and slab
@@ -695,7 +722,7 @@ __global__ __launch_bounds__(256) void crt_gemm_kernel(long M, long N, long Kc, 
   const long gsize = min(tiles_m - first_m, GM), in_group = lin - group * GM * tiles_n;
   const long tm = first_m + in_group % gsize, tn = in_group / gsize;
   const long m0 = tm * BM, n0 = tn * BN;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, lr = lane & 15, lg = lane >> 4;
   const int wm = (wave & 1) * (BM / 2), wn = (wave >> 1) * (BN / 2);
 
   i4v acc[FA][FB];
@@ -709,68 +736,88 @@ __global__ __launch_bounds__(256) void crt_gemm_kernel(long M, long N, long Kc, 
   const signed char* gb = RB + ((size_t)n0 + frow) * Kp + fq;
   const size_t step = (size_t)64 * Kp;
   i4v pa[LA], pb[LB];
+  struct Frags {
+    i4v a[FA], b[FB];
+  };
+  Frags f0, f1;
+  auto fetch = [&](long k0) __attribute__((always_inline)) {
 #pragma unroll
-  for (int q = 0; q < LA; q++) pa[q] = *(const i4v*)(ga + q * step);
+    for (int q = 0; q < LA; q++) pa[q] = *(const i4v*)(ga + q * step + k0);
 #pragma unroll
-  for (int q = 0; q < LB; q++) pb[q] = *(const i4v*)(gb + q * step);
+    for (int q = 0; q < LB; q++) pb[q] = *(const i4v*)(gb + q * step + k0);
+  };
+  auto stage = [&](int buf) __attribute__((always_inline)) {
 #pragma unroll
-  for (int q = 0; q < LA; q++) *(i4v*)(&la[0][oz_lds_off<true>(frow + 64 * q, fq >> 4)]) = pa[q];
+    for (int q = 0; q < LA; q++) *(i4v*)(&la[buf][crt_lds_off<4 * FA>(frow + 64 * q, fq >> 4)]) = pa[q];
 #pragma unroll
-  for (int q = 0; q < LB; q++) *(i4v*)(&lb[0][oz_lds_off<true>(frow + 64 * q, fq >> 4)]) = pb[q];
+    for (int q = 0; q < LB; q++) *(i4v*)(&lb[buf][oz_lds_off<true>(frow + 64 * q, fq >> 4)]) = pb[q];
+  };
+  // lane l holds row l%16 of a 16-row fragment, k bytes (l/16)*16..+15; row x
+  // of A fragment a is row (x/4) * 4 FA + 4 a + x%4 of the wavefront's
+  auto read = [&](int buf, Frags& f) __attribute__((always_inline)) {
+#pragma unroll
+    for (int a = 0; a < FA; a++)
+      f.a[a] = *(const i4v*)(&la[buf][crt_lds_off<4 * FA>(wm + (lr >> 2) * 4 * FA + 4 * a + (lr & 3), lg)]);
+#pragma unroll
+    for (int b = 0; b < FB; b++) f.b[b] = *(const i4v*)(&lb[buf][oz_lds_off<true>(wn + b * 16 + lr, lg)]);
+  };
+  auto mma = [&](const Frags& f) __attribute__((always_inline)) {
+#pragma unroll
+    for (int a = 0; a < FA; a++)
+#pragma unroll
+      for (int b = 0; b < FB; b++) acc[a][b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(f.a[a], f.b[b], acc[a][b], 0, 0, 0);
+  };
+  const long last = Kc - OZ_BK;   // Kc > 0, a multiple of OZ_BK
+  fetch(0);
+  stage(0);
+  fetch(min((long)OZ_BK, last));
   __syncthreads();
-  int buf = 0;
-  for (long k0 = 0; k0 < Kc; k0 += OZ_BK) {
-    const bool more = k0 + OZ_BK < Kc;
-    if (more) {
-#pragma unroll
-      for (int q = 0; q < LA; q++) pa[q] = *(const i4v*)(ga + q * step + k0 + OZ_BK);
-#pragma unroll
-      for (int q = 0; q < LB; q++) pb[q] = *(const i4v*)(gb + q * step + k0 + OZ_BK);
-    }
-    // lane l holds row (l%16) of a 16-row block, k bytes (l/16)*16..+15
-    i4v fb[FB];
-#pragma unroll
-    for (int b = 0; b < FB; b++) fb[b] = *(const i4v*)(&lb[buf][oz_lds_off<true>(wn + b * 16 + (lane & 15), lane >> 4)]);
-#pragma unroll
-    for (int a = 0; a < FA; a++) {
-      const i4v fa = *(const i4v*)(&la[buf][oz_lds_off<true>(wm + a * 16 + (lane & 15), lane >> 4)]);
-#pragma unroll
-      for (int b = 0; b < FB; b++) acc[a][b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fb[b], fa, acc[a][b], 0, 0, 0);
-    }
-    if (more) {
-      // the other buffer was last read before the previous barrier
-#pragma unroll
-      for (int q = 0; q < LA; q++) *(i4v*)(&la[buf ^ 1][oz_lds_off<true>(frow + 64 * q, fq >> 4)]) = pa[q];
-#pragma unroll
-      for (int q = 0; q < LB; q++) *(i4v*)(&lb[buf ^ 1][oz_lds_off<true>(frow + 64 * q, fq >> 4)]) = pb[q];
-    }
-    buf ^= 1;
+  read(0, f0);
+  // slab kt is multiplied from cur; slab kt+1 goes to LDS and its fragments to
+  // next; slab kt+2 is fetched (past the end the last one again, unused)
+  long k0 = 0;
+  auto advance = [&](int buf, Frags& cur, Frags& next) __attribute__((always_inline)) {
+    stage(buf);
+    fetch(min(k0 + 2 * OZ_BK, last));
     __syncthreads();
+    read(buf, next);
+    mma(cur);
+    k0 += OZ_BK;
+  };
+  while (k0 + 2 * OZ_BK < Kc) {
+    advance(1, f0, f1);
+    advance(0, f1, f0);
   }
-  // lane l, element r -> row i = l%16 of block a, column j = 4*(l/16)+r of block b
-  const int p = tab->p[mod], hp = (p + 1) / 2;
-  const double ip = tab->invp[mod];
-  signed char* rc = RC + (size_t)mod * plane;
+  if (k0 + OZ_BK < Kc) {   // slab k0 in f0, the last one in registers
+    stage(1);
+    __syncthreads();
+    read(1, f1);
+    mma(f0);
+    mma(f1);
+  } else {
+    mma(f0);
+  }
+  // lane l, element r of block (a, b): row 4 FA * (l/16) + 4 a + r, column b*16 + l%16
+  const CrtMod m(tab, mod);
+  const long i = m0 + wm + 4 * FA * lg;
 #pragma unroll
-  for (int a = 0; a < FA; a++) {
-    const long i = m0 + wm + a * 16 + (lane & 15);
-    if (i >= M) continue;
+  for (int b = 0; b < FB; b++) {
+    const long j = n0 + wn + b * 16 + lr;
+    unsigned* pc = (unsigned*)(RC + (size_t)mod * plane + j * ldrc + i);
 #pragma unroll
-    for (int b = 0; b < FB; b++)
+    for (int a = 0; a < FA; a += 4) {
+      if (j >= N || i + 4 * a >= ldrc) continue;   // 16 rows at a time; ldrc is a multiple of 16
+      u4v old = {0, 0, 0, 0}, w;
+      if (accumulate) old = *(const u4v*)(pc + a);
 #pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const long j = n0 + wn + b * 16 + 4 * (lane >> 4) + r;
-        if (j >= N) continue;
-        signed char* pc = rc + j * ldrc + i;
-        double x = (double)acc[a][b][r];
-        if (accumulate) x += (double)*pc;
-        x -= (double)p * floor(x * ip);
-        if (x < 0.0) x += p;
-        if (x >= p) x -= p;
-        int v = (int)x;
-        if (v >= hp) v -= p;
-        *pc = (signed char)v;
+      for (int c = 0; c < 4; c++) {
+        unsigned v = 0;
+#pragma unroll
+        for (int r = 0; r < 4; r++) v |= crt_mod(acc[a + c][b][r] + (int)((old[c] >> (8 * r)) & 255u), m) << (8 * r);
+        w[c] = v;
       }
+      *(u4v*)(pc + a) = w;
+    }
   }
 }
 
@@ -783,7 +830,7 @@ __global__ __launch_bounds__(256) void crt_gemm_kernel(long M, long N, long Kc, 
 // through the top four limbs.
 template <int L16>
 __global__ __launch_bounds__(256) void crt_combine_kernel(long M, long N, int NM, const CrtTab* __restrict__ tab,
-                                                          const signed char* __restrict__ RC, long ldrc, long plane,
+                                                          const unsigned char* __restrict__ RC, long ldrc, long plane,
                                                           const double* __restrict__ amax,
                                                           const double* __restrict__ bmax, int tsum, double alpha,
                                                           double beta, double* __restrict__ C, long ldc) {
@@ -791,7 +838,6 @@ __global__ __launch_bounds__(256) void crt_combine_kernel(long M, long N, int NM
   const long idx = blockIdx.x * 256L + threadIdx.x;
   if (idx >= quads * N) return;
   const long i0 = (idx % quads) * 4, j = idx / quads;
-  const bool full = i0 + 4 <= M && (ldrc & 3) == 0;
   unsigned acc[4][L16];
 #pragma unroll
   for (int e = 0; e < 4; e++)
@@ -799,21 +845,12 @@ __global__ __launch_bounds__(256) void crt_combine_kernel(long M, long N, int NM
     for (int l = 0; l < L16; l++) acc[e][l] = 0;
   const unsigned short* q = &tab->q16[NM][0][0];
   for (int m = 0; m < NM; m++) {
-    const signed char* src = RC + (size_t)m * plane + j * ldrc + i0;
-    unsigned word;
-    if (full) word = *(const unsigned*)src;
-    else {
-      word = 0;
-      for (int e = 0; e < 4; e++)
-        if (i0 + e < M) word |= ((unsigned)(unsigned char)src[e]) << (8 * e);
-    }
-    const int p = tab->p[m];
+    const unsigned word = *(const unsigned*)(RC + (size_t)m * plane + j * ldrc + i0);   // ldrc: a multiple of 16
 #pragma unroll
     for (int e = 0; e < 4; e++) {
-      int c = (int)(signed char)(word >> (8 * e));
-      if (c < 0) c += p;
+      const unsigned c = (word >> (8 * e)) & 255u;
 #pragma unroll
-      for (int l = 0; l < L16; l++) acc[e][l] = __umul24((unsigned)c, (unsigned)q[m * CRT_L16 + l]) + acc[e][l];
+      for (int l = 0; l < L16; l++) acc[e][l] = __umul24(c, (unsigned)q[m * CRT_L16 + l]) + acc[e][l];
     }
   }
   const unsigned short* P = tab->P16[NM];
@@ -982,7 +1019,8 @@ int ozaki2_dgemm(bool ta, bool tb, long M, long N, long K, double alpha, const d
   const CrtTab* dt = crt_dev_tab(s);
   const long Kp = (K + OZ_BK - 1) / OZ_BK * OZ_BK;
   const long Mp = (M + CRT_T - 1) / CRT_T * CRT_T, Np = (N + CRT_T - 1) / CRT_T * CRT_T;
-  DevBuf ra((size_t)nm * Mp * Kp), rb((size_t)nm * Np * Kp), rc((size_t)nm * M * N);
+  const long ldrc = (M + 15) / 16 * 16;   // the residues of C are written and read in 16-byte pieces of a column
+  DevBuf ra((size_t)nm * Mp * Kp), rb((size_t)nm * Np * Kp), rc((size_t)nm * ldrc * N);
   {
     dim3 ga((unsigned)(Mp / 64), (unsigned)(Kp / 64)), gb((unsigned)(Np / 64), (unsigned)(Kp / 64));
     auto split = [&](dim3 g, long V, const double* X, long sv, long sk, const double* vmx, int t, signed char* R,
@@ -1007,17 +1045,18 @@ int ozaki2_dgemm(bool ta, bool tb, long M, long N, long K, double alpha, const d
     KTimer kt("ozaki_gemm", s, (double)nm * 2.0 * M * N * K, (double)nm * (M * K + K * N + M * N));
     // 256x256 tiles (a 128x128 register tile per wavefront: half the
     // operand traffic per product of the 128x128 tiles) when they still
-    // give every CU a tile per modulus; 8192^3, 17 moduli: 15.1 vs 15.5 ms
+    // give every CU a tile per modulus; 8192^3, 17 moduli: 15.1 against 15.5 ms
+    // for the whole call when it was chosen
     const bool big = (Mp / 256) * (Np / 256) >= rt().num_cu;
     for (long k0 = 0; k0 < Kp; k0 += CRT_KCHUNK) {
       const long kc = std::min(CRT_KCHUNK, Kp - k0);
       if (big)
         crt_gemm_kernel<8, 8><<<dim3((unsigned)((Mp / 256) * (Np / 256)), (unsigned)nm), 256, 0, s>>>(
-            M, N, kc, Kp, k0, ra.as<signed char>(), Mp, rb.as<signed char>(), Np, dt, rc.as<signed char>(), M, M * N,
+            N, kc, Kp, k0, ra.as<signed char>(), Mp, rb.as<signed char>(), Np, dt, rc.as<unsigned char>(), ldrc, ldrc * N,
             k0 > 0 ? 1 : 0);
       else
         crt_gemm_kernel<4, 4><<<dim3((unsigned)((Mp / 128) * (Np / 128)), (unsigned)nm), 256, 0, s>>>(
-            M, N, kc, Kp, k0, ra.as<signed char>(), Mp, rb.as<signed char>(), Np, dt, rc.as<signed char>(), M, M * N,
+            N, kc, Kp, k0, ra.as<signed char>(), Mp, rb.as<signed char>(), Np, dt, rc.as<unsigned char>(), ldrc, ldrc * N,
             k0 > 0 ? 1 : 0);
       OBA_HIP(hipGetLastError());
     }
@@ -1027,7 +1066,7 @@ int ozaki2_dgemm(bool ta, bool tb, long M, long N, long K, double alpha, const d
   const unsigned blocks = (unsigned)(((M + 3) / 4 * N + 255) / 256);
 #define CRT_C(L)                                                                                                    \
   case L:                                                                                                           \
-    crt_combine_kernel<L><<<blocks, 256, 0, s>>>(M, N, nm, dt, rc.as<signed char>(), M, M * N, amax, bmax, tA + tB, \
+    crt_combine_kernel<L><<<blocks, 256, 0, s>>>(M, N, nm, dt, rc.as<unsigned char>(), ldrc, ldrc * N, amax, bmax, tA + tB, \
                                                  alpha, beta, C, ldc);                                              \
     break;
   switch (std::max(l16, 4)) {
