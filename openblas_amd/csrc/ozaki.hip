@@ -688,28 +688,32 @@ __device__ __attribute__((always_inline)) inline int crt_lds_off(int r, int c) {
   return r * 64 + ((c ^ (((r >> 1) ^ (r / GAP)) & 3)) << 4);
 }
 
-// One INT8 GEMM per modulus (blockIdx.y): a (32 FA) x (32 FB) tile of the
-// residue product, four wavefronts of (16 FA) x (16 FB) (FA x FB MFMA
-// blocks each).  64-deep k slabs double-buffered in LDS; the fragments of a
-// slab are read into registers while the slab before is multiplied, and the
-// slab after the next is on its way from memory, so a step has one barrier
-// and nothing in front of its MFMAs.  The exact int32 sums are reduced mod p_m
-// and stored as residues in [0, p_m) (RC[m][j][i], i contiguous); a lane's
-// fragment rows are spaced so that it ends with 4 FA consecutive rows of a
-// column, stored 16 bytes at a time.  With `accumulate` the launch adds to the
-// residues of the previous k chunk.  8192^3, 17 moduli: 10.9 ms (1.72 POP/s);
-// 12.05 with the fragments read in front of their own MFMAs, an FP64 remainder
-// and single-byte stores.  One wavefront per SIMD (256 accumulators a lane).
+// One INT8 GEMM per modulus (blockIdx.y): a (32 FA) x (64 FB) tile of the
+// residue product by eight wavefronts of (16 FA) x (16 FB) (FA x FB MFMA
+// blocks each), two per SIMD, so that one's MFMAs run while the other reads
+// fragments or waits at the barrier.  128-deep k slabs, double-buffered in LDS
+// as two 64-deep halves, the next slab on its way from memory.  The exact int32
+// sums are reduced mod p_m and stored as residues in [0, p_m) (RC[m][j][i], i
+// contiguous); a lane's fragment rows are spaced so that it ends with 4 FA
+// consecutive rows of a column, stored 16 bytes at a time.  With `accumulate`
+// the launch adds to the residues of the previous k chunk.
+// Bound by the matrix cores and the reads around them: 8192^3, 17 moduli 9.1 ms
+// in a call, 8.28 ms (2.26 POP/s) when repeated alone, which the following
+// figures are too.  Four wavefronts of 128x128 with all 256
+// accumulators took 10.2 (register copies between the MFMAs; slabs loaded
+// straight into LDS gave no more), 64-deep slabs take 8.52.  In a
+// call, four wavefronts with an FP64 remainder and single-byte stores took 12.05.
+constexpr int CRT_BK = 128;
 template <int FA, int FB>
-__global__ __launch_bounds__(256) void crt_gemm_kernel(long N, long Kc, long Kp, long k_off,
+__global__ __launch_bounds__(512) void crt_gemm_kernel(long N, long Kc, long Kp, long k_off,
                                                        const signed char* __restrict__ RA, long Mp,
                                                        const signed char* __restrict__ RB, long Np,
                                                        const CrtTab* __restrict__ tab, unsigned char* __restrict__ RC,
                                                        long ldrc, long plane, int accumulate) {
-  constexpr int BM = 32 * FA, BN = 32 * FB;
-  constexpr int LA = BM / 64, LB = BN / 64;   // 16-byte loads per thread and slab
-  __shared__ __attribute__((aligned(16))) signed char la[2][BM * 64];
-  __shared__ __attribute__((aligned(16))) signed char lb[2][BN * 64];
+  constexpr int BM = 32 * FA, BN = 64 * FB;
+  constexpr int LA = BM / 128, LB = BN / 128;   // 16-byte loads per thread and half slab
+  __shared__ __attribute__((aligned(16))) signed char la[2][2][BM * 64];
+  __shared__ __attribute__((aligned(16))) signed char lb[2][2][BN * 64];
   const int mod = blockIdx.y;
   RA += (size_t)mod * Mp * Kp + k_off;
   RB += (size_t)mod * Np * Kp + k_off;
@@ -723,79 +727,64 @@ __global__ __launch_bounds__(256) void crt_gemm_kernel(long N, long Kc, long Kp,
   const long tm = first_m + in_group % gsize, tn = in_group / gsize;
   const long m0 = tm * BM, n0 = tn * BN;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, lr = lane & 15, lg = lane >> 4;
-  const int wm = (wave & 1) * (BM / 2), wn = (wave >> 1) * (BN / 2);
+  const int wm = (wave & 1) * (BM / 2), wn = (wave >> 1) * (BN / 4);
 
   i4v acc[FA][FB];
 #pragma unroll
   for (int a = 0; a < FA; a++)
 #pragma unroll
     for (int b = 0; b < FB; b++) acc[a][b] = i4v{0, 0, 0, 0};
-  // thread's share of a slab: rows frow + 64 q, bytes fq..fq+15
+  // thread's share of a half slab: rows frow + 128 q, bytes fq..fq+15
   const int frow = threadIdx.x >> 2, fq = (threadIdx.x & 3) * 16;
   const signed char* ga = RA + ((size_t)m0 + frow) * Kp + fq;
   const signed char* gb = RB + ((size_t)n0 + frow) * Kp + fq;
-  const size_t step = (size_t)64 * Kp;
-  i4v pa[LA], pb[LB];
-  struct Frags {
-    i4v a[FA], b[FB];
-  };
-  Frags f0, f1;
+  const size_t step = (size_t)128 * Kp;
+  i4v pa[2][LA], pb[2][LB];
   auto fetch = [&](long k0) __attribute__((always_inline)) {
 #pragma unroll
-    for (int q = 0; q < LA; q++) pa[q] = *(const i4v*)(ga + q * step + k0);
+    for (int h = 0; h < 2; h++) {
 #pragma unroll
-    for (int q = 0; q < LB; q++) pb[q] = *(const i4v*)(gb + q * step + k0);
+      for (int q = 0; q < LA; q++) pa[h][q] = *(const i4v*)(ga + q * step + k0 + 64 * h);
+#pragma unroll
+      for (int q = 0; q < LB; q++) pb[h][q] = *(const i4v*)(gb + q * step + k0 + 64 * h);
+    }
   };
   auto stage = [&](int buf) __attribute__((always_inline)) {
 #pragma unroll
-    for (int q = 0; q < LA; q++) *(i4v*)(&la[buf][crt_lds_off<4 * FA>(frow + 64 * q, fq >> 4)]) = pa[q];
+    for (int h = 0; h < 2; h++) {
 #pragma unroll
-    for (int q = 0; q < LB; q++) *(i4v*)(&lb[buf][oz_lds_off<true>(frow + 64 * q, fq >> 4)]) = pb[q];
+      for (int q = 0; q < LA; q++) *(i4v*)(&la[buf][h][crt_lds_off<4 * FA>(frow + 128 * q, fq >> 4)]) = pa[h][q];
+#pragma unroll
+      for (int q = 0; q < LB; q++) *(i4v*)(&lb[buf][h][oz_lds_off<true>(frow + 128 * q, fq >> 4)]) = pb[h][q];
+    }
   };
   // lane l holds row l%16 of a 16-row fragment, k bytes (l/16)*16..+15; row x
   // of A fragment a is row (x/4) * 4 FA + 4 a + x%4 of the wavefront's
-  auto read = [&](int buf, Frags& f) __attribute__((always_inline)) {
+  auto mma = [&](int buf, int h) __attribute__((always_inline)) {
+    i4v fb[FB];
 #pragma unroll
-    for (int a = 0; a < FA; a++)
-      f.a[a] = *(const i4v*)(&la[buf][crt_lds_off<4 * FA>(wm + (lr >> 2) * 4 * FA + 4 * a + (lr & 3), lg)]);
+    for (int b = 0; b < FB; b++) fb[b] = *(const i4v*)(&lb[buf][h][oz_lds_off<true>(wn + b * 16 + lr, lg)]);
 #pragma unroll
-    for (int b = 0; b < FB; b++) f.b[b] = *(const i4v*)(&lb[buf][oz_lds_off<true>(wn + b * 16 + lr, lg)]);
+    for (int a = 0; a < FA; a++) {
+      const i4v fa = *(const i4v*)(&la[buf][h][crt_lds_off<4 * FA>(wm + (lr >> 2) * 4 * FA + 4 * a + (lr & 3), lg)]);
+#pragma unroll
+      for (int b = 0; b < FB; b++) acc[a][b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fa, fb[b], acc[a][b], 0, 0, 0);
+    }
   };
-  auto mma = [&](const Frags& f) __attribute__((always_inline)) {
-#pragma unroll
-    for (int a = 0; a < FA; a++)
-#pragma unroll
-      for (int b = 0; b < FB; b++) acc[a][b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(f.a[a], f.b[b], acc[a][b], 0, 0, 0);
-  };
-  const long last = Kc - OZ_BK;   // Kc > 0, a multiple of OZ_BK
+  const long last = Kc - CRT_BK;   // Kc > 0, a multiple of CRT_BK
   fetch(0);
   stage(0);
-  fetch(min((long)OZ_BK, last));
+  fetch(min((long)CRT_BK, last));
   __syncthreads();
-  read(0, f0);
-  // slab kt is multiplied from cur; slab kt+1 goes to LDS and its fragments to
-  // next; slab kt+2 is fetched (past the end the last one again, unused)
-  long k0 = 0;
-  auto advance = [&](int buf, Frags& cur, Frags& next) __attribute__((always_inline)) {
+  int buf = 0;
+#pragma unroll 1
+  for (long k0 = 0; k0 < Kc; k0 += CRT_BK) {
+    mma(buf, 0);
+    mma(buf, 1);
+    buf ^= 1;   // last read before the previous barrier
     stage(buf);
-    fetch(min(k0 + 2 * OZ_BK, last));
+    fetch(min(k0 + 2 * CRT_BK, last));   // past the end the last slab again, unused
     __syncthreads();
-    read(buf, next);
-    mma(cur);
-    k0 += OZ_BK;
-  };
-  while (k0 + 2 * OZ_BK < Kc) {
-    advance(1, f0, f1);
-    advance(0, f1, f0);
-  }
-  if (k0 + OZ_BK < Kc) {   // slab k0 in f0, the last one in registers
-    stage(1);
-    __syncthreads();
-    read(1, f1);
-    mma(f0);
-    mma(f1);
-  } else {
-    mma(f0);
   }
   // lane l, element r of block (a, b): row 4 FA * (l/16) + 4 a + r, column b*16 + l%16
   const CrtMod m(tab, mod);
@@ -1017,7 +1006,7 @@ int ozaki2_dgemm(bool ta, bool tb, long M, long N, long K, double alpha, const d
   const int tB = total - tA;
   if (tB < 1) fatal("ozaki2: too few moduli for this K", nullptr);
   const CrtTab* dt = crt_dev_tab(s);
-  const long Kp = (K + OZ_BK - 1) / OZ_BK * OZ_BK;
+  const long Kp = (K + CRT_BK - 1) / CRT_BK * CRT_BK;
   const long Mp = (M + CRT_T - 1) / CRT_T * CRT_T, Np = (N + CRT_T - 1) / CRT_T * CRT_T;
   const long ldrc = (M + 15) / 16 * 16;   // the residues of C are written and read in 16-byte pieces of a column
   DevBuf ra((size_t)nm * Mp * Kp), rb((size_t)nm * Np * Kp), rc((size_t)nm * ldrc * N);
@@ -1043,19 +1032,19 @@ int ozaki2_dgemm(bool ta, bool tb, long M, long N, long K, double alpha, const d
     // algorithmic work: nm INT8 GEMMs of 2MNK ops; bytes: the residues of
     // both operands once per modulus and the residues of C written
     KTimer kt("ozaki_gemm", s, (double)nm * 2.0 * M * N * K, (double)nm * (M * K + K * N + M * N));
-    // 256x256 tiles (a 128x128 register tile per wavefront: half the
-    // operand traffic per product of the 128x128 tiles) when they still
+    // 256x256 tiles (a 128x64 register tile per wavefront: half the operand
+    // traffic per product of the 128x128 tiles) when they still
     // give every CU a tile per modulus; 8192^3, 17 moduli: 15.1 against 15.5 ms
     // for the whole call when it was chosen
     const bool big = (Mp / 256) * (Np / 256) >= rt().num_cu;
     for (long k0 = 0; k0 < Kp; k0 += CRT_KCHUNK) {
       const long kc = std::min(CRT_KCHUNK, Kp - k0);
       if (big)
-        crt_gemm_kernel<8, 8><<<dim3((unsigned)((Mp / 256) * (Np / 256)), (unsigned)nm), 256, 0, s>>>(
+        crt_gemm_kernel<8, 4><<<dim3((unsigned)((Mp / 256) * (Np / 256)), (unsigned)nm), 512, 0, s>>>(
             N, kc, Kp, k0, ra.as<signed char>(), Mp, rb.as<signed char>(), Np, dt, rc.as<unsigned char>(), ldrc, ldrc * N,
             k0 > 0 ? 1 : 0);
       else
-        crt_gemm_kernel<4, 4><<<dim3((unsigned)((Mp / 128) * (Np / 128)), (unsigned)nm), 256, 0, s>>>(
+        crt_gemm_kernel<4, 2><<<dim3((unsigned)((Mp / 128) * (Np / 128)), (unsigned)nm), 512, 0, s>>>(
             N, kc, Kp, k0, ra.as<signed char>(), Mp, rb.as<signed char>(), Np, dt, rc.as<unsigned char>(), ldrc, ldrc * N,
             k0 > 0 ? 1 : 0);
       OBA_HIP(hipGetLastError());
