@@ -15,6 +15,7 @@
 // that turns every later kernel of the same call into a no-op, so the call
 // stops where the reference stops without a host round trip per leaf.
 #include "kernels.h"
+#include "tri_inv.h"
 #include <cmath>
 
 namespace oba {
@@ -26,78 +27,6 @@ __device__ inline double po_rl(double v, int l) {
   const int lo = __builtin_amdgcn_readlane(__double2loint(v), l);
   const int hi = __builtin_amdgcn_readlane(__double2hiint(v), l);
   return __hiloint2double(hi, lo);
-}
-
-template <typename T> struct PoMf;
-template <> struct PoMf<double> {
-  typedef double acc __attribute__((ext_vector_type(4)));
-  __device__ static inline acc mma(double a, double b, acc c) { return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0); }
-  __device__ static inline int orow(int l, int r) { return 4 * r + (l >> 4); }
-};
-template <> struct PoMf<float> {
-  typedef float acc __attribute__((ext_vector_type(4)));
-  __device__ static inline acc mma(float a, float b, acc c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
-  __device__ static inline int orow(int l, int r) { return 4 * (l >> 4) + r; }
-};
-
-// lane K of each row of 16 lanes, to all of the row
-template <int K>
-__device__ inline float po_bcast16(float v) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + K, 0xF, 0xF, false));
-}
-template <int K>
-__device__ inline double po_bcast16(double v) {
-  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), 0x150 + K, 0xF, 0xF, false);
-  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), 0x150 + K, 0xF, 0xF, false);
-  return __hiloint2double(hi, lo);
-}
-template <int K, typename T>
-__device__ __attribute__((always_inline)) inline void potrf_inv16_step(T (&y)[4], const T (&l)[16], T r, int i) {
-  if constexpr (K < 15) {
-    const T rk = po_bcast16<K>(r);
-#pragma unroll
-    for (int c = 0; c < 4; c++) {
-      const T f = y[c] - l[K] * (po_bcast16<K>(y[c]) * rk);
-      y[c] = i > K ? f : y[c];   // an Inf or NaN of L only meets its own rows
-    }
-    potrf_inv16_step<K + 1>(y, l, r, i);
-  }
-}
-// One wavefront inverts the 16x16 lower triangle at o (diagonal reciprocals
-// in rinv): lane (i, g) = (lane % 16, lane / 16) holds row i of columns g,
-// g+4, g+8, g+12; row k, once final, reaches the rows below by DPP row
-// broadcasts.
-template <typename T>
-__device__ __attribute__((always_inline)) inline void potrf_inv16(const T* S, T* Y, const T* rinv, int o) {
-  constexpr int LD = PO_NB + 1;
-  const int i = threadIdx.x & 15, g = (threadIdx.x & 63) >> 4;
-  T l[16], y[4];
-#pragma unroll
-  for (int k = 0; k < 16; k++) l[k] = S[(o + k) * LD + o + i];
-  const T r = rinv[o + i];
-#pragma unroll
-  for (int c = 0; c < 4; c++) y[c] = i == g + 4 * c ? T(1) : T(0);
-  potrf_inv16_step<0>(y, l, r, i);
-#pragma unroll
-  for (int c = 0; c < 4; c++) Y[(o + g + 4 * c) * LD + o + i] = i >= g + 4 * c ? y[c] * r : T(0);
-}
-
-// one wavefront: tile (ri, ci) of `o` = sign * sum over the 16-deep tiles k0
-// .. k0+NK of x(ri, k) y(k, ci), in 64x64 LDS matrices
-template <int NK, typename T>
-__device__ __attribute__((always_inline)) inline void potrf_prod(T* o, const T* x, const T* y, int ri, int ci, int k0,
-                                                                 T sign) {
-  constexpr int LD = PO_NB + 1;
-  typedef PoMf<T> mf;
-  const int lane = threadIdx.x & 63, lr = lane & 15, lg = lane >> 4;
-  typename mf::acc acc[2] = {};
-#pragma unroll
-  for (int k = 0; k < 16 * NK; k += 4)
-    acc[(k >> 2) & 1] = mf::mma(y[(16 * ci + lr) * LD + 16 * k0 + k + lg], x[(16 * k0 + k + lg) * LD + 16 * ri + lr],
-                                acc[(k >> 2) & 1]);
-  acc[0] += acc[1];
-#pragma unroll
-  for (int r = 0; r < 4; r++) o[(16 * ci + mf::orow(lane, r)) * LD + 16 * ri + lr] = sign * acc[0][r];
 }
 
 // Factor the nb x nb (nb <= 64) diagonal block at a (lower: E(i,k) =
@@ -127,7 +56,7 @@ template <typename T>
 __global__ __launch_bounds__(256) void potrf_leaf_kernel(int nb, T* a, long lda, bool upper, long j0, int* info,
                                                          T* inv) {
   constexpr int NB = PO_NB, LD = NB + 1;
-  typedef PoMf<T> mf;
+  typedef TriMf<T> mf;
   __shared__ T S[NB * LD];   // E(i, c) at S[c*LD + i]
   __shared__ T Y[NB * LD];   // L^{-1}(i, c) at Y[c*LD + i]
   __shared__ T U[NB * LD];   // products of the joins
@@ -205,15 +134,15 @@ __global__ __launch_bounds__(256) void potrf_leaf_kernel(int nb, T* a, long lda,
     }
     if (inv) {   // beside the factorization of a step: the inverse, as far as the columns are final
       if (w == 3 && q > 0) {
-        potrf_inv16(S, Y, s_rinv, 16 * (q - 1));
+        tri_inv16(S, Y, s_rinv, 16 * (q - 1));
         if (!(q & 1)) {   // join with the block before
-          potrf_prod<1>(U, S, Y, q - 1, q - 2, q - 2, T(1));
-          potrf_prod<1>(Y, Y, U, q - 1, q - 2, q - 1, T(-1));
+          tri_prod<1>(U, S, Y, q - 1, q - 2, q - 2, T(1));
+          tri_prod<1>(Y, Y, U, q - 1, q - 2, q - 1, T(-1));
         }
       }
       if (q == 3 && (w == 1 || w == 2)) {   // L21 Y11
 #pragma unroll 1
-        for (int u = 0; u < 2; u++) potrf_prod<2>(U, S, Y, 1 + w, u, 0, T(1));
+        for (int u = 0; u < 2; u++) tri_prod<2>(U, S, Y, 1 + w, u, 0, T(1));
       }
     }
     if (q == 4) break;
@@ -252,7 +181,7 @@ __global__ __launch_bounds__(256) void potrf_leaf_kernel(int nb, T* a, long lda,
   }
   if (!inv) return;
   __syncthreads();
-  potrf_prod<2>(Y, Y, U, 2 + (w >> 1), w & 1, 2, T(-1));   // Y21 = -Y22 (L21 Y11)
+  tri_prod<2>(Y, Y, U, 2 + (w >> 1), w & 1, 2, T(-1));   // Y21 = -Y22 (L21 Y11)
   __syncthreads();
 #pragma unroll
   for (int u = 0; u < 16; u++) {

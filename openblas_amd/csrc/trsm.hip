@@ -14,6 +14,7 @@
 // or backward column-oriented substitution).  Right-side leaves (up to 256
 // columns) multiply by explicit inverses of the 64x64 diagonal blocks.
 #include "kernels.h"
+#include "tri_inv.h"
 
 namespace oba {
 
@@ -264,24 +265,28 @@ __global__ __launch_bounds__(256) void trsm_leafb_kernel(int nb, long nvec, cons
 // size (instruction fetch); the two kernels below replace it.
 //
 // (1) One workgroup per diagonal block b of M = op(A) (upper or lower,
-//     unit or not) computes M_bb^{-1} by doubling: the four 16x16 diagonal
-//     blocks are inverted by substitution (one thread per column, the
-//     diagonal applied as a multiplication by its reciprocal as
-//     trsm_kernel_LT.c:95), then pairs are joined with two small products
-//     each (upper: Y12 = -Y11 M12 Y22; lower: Y21 = -Y22 M21 Y11), 16 -> 32
-//     -> 64.  Stored row-major at inv[b*64*64 + i*64 + j].
+//     unit or not) computes M_bb^{-1} by doubling, as the lower triangle L =
+//     M or M^T: the four 16x16 diagonal blocks by substitution, one per
+//     wavefront (tri_inv.h; the diagonal applied as a multiplication by its
+//     reciprocal as trsm_kernel_LT.c:95), then pairs joined with two products
+//     each on the matrix cores, Y21 = -Y22 (L21 Y11), 16 -> 32 -> 64.  Stored
+//     row-major at inv[b*64*64 + i*64 + j].  The bound is the chain of 16
+//     substitution steps and four products: 7.8 us FP64 with its launch; 12.9 with a thread per
+//     column reading L from LDS and the joins on the vector unit.
 template <typename T>
 __global__ __launch_bounds__(256) void trsm_inv_diag_kernel(long na, const T* __restrict__ A, long lda, bool mT,
                                                             bool mupper, bool unit, T* __restrict__ inv,
                                                             const int* abort_flag) {
-  constexpr int LD = TRSM_NB + 1;
-  __shared__ T Ms[TRSM_NB * LD];   // M(i,k) at Ms[i*LD + k]
-  __shared__ T Ys[TRSM_NB * LD];   // M^{-1}(i,j) at Ys[i*LD + j]
-  __shared__ T Ts[TRSM_NB * LD];   // products of the joins
+  constexpr int LD = TRI_NB + 1;
+  __shared__ T S[TRSM_NB * LD];   // L, the other triangle zero
+  __shared__ T Y[TRSM_NB * LD];   // its inverse
+  __shared__ T U[TRSM_NB * LD];   // products of the joins
+  __shared__ T s_rinv[TRSM_NB];
   if (abort_flag && *abort_flag) return;
   const long o = (long)blockIdx.x * TRSM_NB;
   const int nb = (int)min((long)TRSM_NB, na - o);
-  const int t = threadIdx.x;
+  const int t = threadIdx.x, w = __builtin_amdgcn_readfirstlane(t >> 6);
+  const bool flip = mT != mupper;   // L(i,k) = A(k,i)
   // staging: every load issued before the first LDS write (unconditional
   // loads from clamped, in-bounds addresses; the padding is selected after)
   constexpr int SU = TRSM_NB * TRSM_NB / 256;
@@ -294,89 +299,28 @@ __global__ __launch_bounds__(256) void trsm_inv_diag_kernel(long na, const T* __
 #pragma unroll
   for (int u = 0; u < SU; u++) {
     const int idx = t + 256 * u, f = idx & 63, g = idx >> 6;
-    const T v = (f < nb && g < nb) ? sv[u] : (f == g ? T(1) : T(0));   // pad with the identity
-    if (mT) Ms[g * LD + f] = v;  // M(g,f) = A(f,g)
-    else Ms[f * LD + g] = v;
-    Ys[f * LD + g] = T(0);
+    const int i = flip ? g : f, k = flip ? f : g;
+    const bool in = i < nb && k < nb;
+    S[k * LD + i] = i > k && in ? sv[u] : T(0);
+    Y[k * LD + i] = T(0);
+    if (i == k) s_rinv[i] = in && !unit ? T(1) / sv[u] : T(1);   // padded with the identity
   }
   __syncthreads();
-  // 16x16 diagonal blocks: lane j < 16 of wavefront blk computes column j
-  // of block blk in registers, every step unrolled with static indices; the
-  // terms outside the column's support are skipped by selects (so an
-  // unreferenced Inf/NaN never meets a zero), the sums run in the order of
-  // the substitution: k upward from the column (lower) or from i+1 (upper).
-  if ((t & 63) < 16) {
-    const int blk = t >> 6, j = t & 15, o16 = blk * 16;
-    auto dinv = [&](int i) { return unit ? T(1) : T(1) / Ms[(o16 + i) * LD + o16 + i]; };
-    T y[16];
-    if (mupper) {
-#pragma unroll
-      for (int i = 15; i >= 0; i--) {
-        T acc = T(0);
-#pragma unroll
-        for (int k = i + 1; k < 16; k++) {
-          const T f = acc + Ms[(o16 + i) * LD + o16 + k] * y[k];
-          acc = k <= j ? f : acc;
-        }
-        y[i] = i > j ? T(0) : (i == j ? dinv(i) : -acc * dinv(i));
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < 16; i++) {
-        T acc = T(0);
-#pragma unroll
-        for (int k = 0; k < i; k++) {
-          const T f = acc + Ms[(o16 + i) * LD + o16 + k] * y[k];
-          acc = k >= j ? f : acc;
-        }
-        y[i] = i < j ? T(0) : (i == j ? dinv(i) : -acc * dinv(i));
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < 16; i++) Ys[(o16 + i) * LD + o16 + j] = y[i];
+  tri_inv16(S, Y, s_rinv, 16 * w);
+  __syncthreads();
+  if (w < 2) {
+    tri_prod<1>(U, S, Y, 2 * w + 1, 2 * w, 2 * w, T(1));
+    tri_prod<1>(Y, Y, U, 2 * w + 1, 2 * w, 2 * w + 1, T(-1));
   }
   __syncthreads();
-  // joins 16 -> 32 -> 64 with the block size a compile-time constant, so
-  // every loop is unrolled and a thread's LDS reads issue together (same
-  // operations, same order)
-  auto join = [&](auto hc) __attribute__((always_inline)) {
-    constexpr int h = decltype(hc)::value;
-    constexpr int npair = TRSM_NB / (2 * h);
-    constexpr int PER = npair * h * h / 256;   // outputs per thread
-    static_assert(PER * 256 == npair * h * h, "whole rounds");
-    // T = M_off * Y_near   (upper: M12 Y22; lower: M21 Y11)
-#pragma unroll
-    for (int u = 0; u < PER; u++) {
-      const int idx = t + 256 * u;
-      const int p = idx / (h * h), r = (idx / h) % h, c = idx % h, po = p * 2 * h;
-      const int mr = mupper ? po + r : po + h + r, mc0 = mupper ? po + h : po;   // M rows / first column
-      const int yc = mupper ? po + h + c : po + c;                                  // Y column
-      T acc = T(0);
-#pragma unroll
-      for (int k = 0; k < h; k++) acc += Ms[mr * LD + mc0 + k] * Ys[(mc0 + k) * LD + yc];
-      Ts[(po + r) * LD + c] = acc;
-    }
-    __syncthreads();
-    // Y_off = -Y_far * T   (upper: Y12 = -Y11 T; lower: Y21 = -Y22 T)
-#pragma unroll
-    for (int u = 0; u < PER; u++) {
-      const int idx = t + 256 * u;
-      const int p = idx / (h * h), r = (idx / h) % h, c = idx % h, po = p * 2 * h;
-      const int yr = mupper ? po + r : po + h + r, yk0 = mupper ? po : po + h;
-      T acc = T(0);
-#pragma unroll
-      for (int k = 0; k < h; k++) acc += Ys[yr * LD + yk0 + k] * Ts[(po + k) * LD + c];
-      const int oc = mupper ? po + h + c : po + c;
-      Ys[yr * LD + oc] = -acc;
-    }
-    __syncthreads();
-  };
-  join(std::integral_constant<int, 16>{});
-  join(std::integral_constant<int, 32>{});
+  tri_prod<2>(U, S, Y, 2 + (w >> 1), w & 1, 0, T(1));
+  __syncthreads();
+  tri_prod<2>(Y, Y, U, 2 + (w >> 1), w & 1, 2, T(-1));
+  __syncthreads();
   T* out = inv + (long)blockIdx.x * TRSM_NB * TRSM_NB;
   for (int idx = t; idx < TRSM_NB * TRSM_NB; idx += 256) {
     const int i = idx >> 6, j = idx & 63;
-    out[idx] = (i < nb && j < nb) ? Ys[i * LD + j] : T(0);
+    out[idx] = (i < nb && j < nb) ? (mupper ? Y[i * LD + j] : Y[j * LD + i]) : T(0);
   }
 }
 
