@@ -7,12 +7,12 @@
 // (kernel/generic/trsm_ltcopy_2.c:43 INV(a) = 1/a, trsm_kernel_LT.c:95).
 //
 // Design: recursive blocking on the triangle (split in halves on a 64-row
-// grid) so that almost all flops land in large MFMA GEMM updates.  Left-side
-// leaves (up to 256 rows) are solved by wavefronts of right-hand-side
-// vectors: lane i owns x_i and row i of the current 64x64 tile of the
-// triangle, and x_k is broadcast with v_readlane after it is final (forward
-// or backward column-oriented substitution).  Right-side leaves (up to 256
-// columns) multiply by explicit inverses of the 64x64 diagonal blocks.
+// grid) so that almost all flops land in large MFMA GEMM updates.  Leaves (up
+// to 256 rows or columns of the triangle) multiply by explicit inverses of the
+// 64x64 diagonal blocks; a left-side triangle of a single block is solved by
+// wavefronts of right-hand-side vectors: lane i owns x_i and row i of the
+// triangle, and x_k is broadcast with v_readlane after it is final (forward or
+// backward column-oriented substitution).
 #include "kernels.h"
 #include "tri_inv.h"
 
@@ -121,148 +121,13 @@ __global__ __launch_bounds__(256) void trsm_leaf_kernel(int nb, long nvec, const
   }
 }
 
-// Left-side leaves of up to TRSM_LEAF_BLKS x 64 rows in one launch: the
-// 64-row blocks are solved in dependency order (forward for lower E,
-// backward for upper), each solved block's terms subtracted from the later
-// blocks of the leaf in registers (x_k broadcast by v_readlane), so the
-// recursion's two lowest GEMM levels (64 x n x 64 and 128 x n x 128 products
-// with few output tiles) and their launches disappear.  The 64x64 tiles of
-// the triangle pass through double-buffered LDS (one barrier per tile, the
-// next tile's loads in flight during the current tile's work); each lane
-// takes its row of the tile into registers.  Vectors as in trsm_leaf_kernel.
-constexpr int TRSM_LEAF_BLKS = 4;
-constexpr int TRSM_LEAF_MAX = TRSM_LEAF_BLKS * TRSM_NB;
-
-template <typename T>
-__global__ __launch_bounds__(256) void trsm_leafb_kernel(int nb, long nvec, const T* __restrict__ A, long lda,
-                                                         T* __restrict__ B, long inc_e, long inc_v, bool eT,
-                                                         bool elower, bool unit, const int* abort_flag) {
-  constexpr int LDE = TRSM_NB + 1;
-  constexpr int MB = TRSM_LEAF_BLKS;
-  constexpr int PF = TRSM_NB * TRSM_NB / 256;   // tile elements per thread
-  __shared__ T E[2][TRSM_NB * LDE];             // tile element (i, k) at E[par][k*LDE + i]
-  // per wavefront: its vectors' x, block by block (written and read back by
-  // the same wavefront only, no barrier; a register array indexed by the
-  // run-time block number was placed in scratch memory)
-  __shared__ T Xb[4][MB][TRSM_VPW][TRSM_NB];
-  if (abort_flag && *abort_flag) return;
-  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-  const int nblk = (nb + TRSM_NB - 1) / TRSM_NB;
-  const long v0 = ((long)blockIdx.x * (blockDim.x >> 6) + (t >> 6)) * TRSM_VPW;
-  // block b of the leaf in processing order q: b = q (lower) or nblk-1-q
-  auto blk_of = [&](int q) { return elower ? q : nblk - 1 - q; };
-  // the tile (i-block bi, k-block bj) of E = op(A) into registers
-  auto fetch = [&](int bi, int bj, T (&r)[PF]) {
-#pragma unroll
-    for (int u = 0; u < PF; u++) {
-      const int idx = t + u * 256, f = idx & 63, s = idx >> 6;   // f: contiguous index of A
-      const int ra = (eT ? bj : bi) * TRSM_NB + f, ca = (eT ? bi : bj) * TRSM_NB + s;
-      r[u] = (ra < nb && ca < nb) ? A[ra + (long)ca * lda] : T(0);
-    }
-  };
-  auto store = [&](int par, const T (&r)[PF]) {
-#pragma unroll
-    for (int u = 0; u < PF; u++) {
-      const int idx = t + u * 256, f = idx & 63, s = idx >> 6;
-      const int i = eT ? s : f, k = eT ? f : s;
-      E[par][k * LDE + i] = r[u];
-    }
-  };
-#pragma unroll
-  for (int b = 0; b < MB; b++)
-#pragma unroll
-    for (int vv = 0; vv < TRSM_VPW; vv++) {
-      const long v = v0 + vv;
-      const int row = b * TRSM_NB + lane;
-      Xb[w][b][vv][lane] = (b < nblk && v < nvec && row < nb) ? B[v * inc_v + (long)row * inc_e] : T(0);
-    }
-  // tiles in order: for each block row qi, the solved blocks qj < qi, then the diagonal
-  int qi = 0, qj = 0, par = 0;
-  T pf[PF];
-  fetch(blk_of(0), blk_of(0), pf);
-  T xt[TRSM_VPW];
-#pragma unroll
-  for (int vv = 0; vv < TRSM_VPW; vv++) xt[vv] = Xb[w][blk_of(0)][vv][lane];
-  while (true) {
-    store(par, pf);
-    __syncthreads();
-    const int bi = blk_of(qi), bj = blk_of(qj);
-    int ni = qi, nj = qj + 1;   // the next tile
-    if (nj > qi) { ni = qi + 1; nj = 0; }
-    const bool more = ni < nblk;
-    if (more) fetch(blk_of(ni), blk_of(nj), pf);
-    // Every step is straight-line code (a branch per step kept each step's
-    // loads from being issued early): rows of a partial block beyond its
-    // end hold exact zeros in x (the diagonal solve never updates them) and
-    // in the tile (the fetch pads with zeros), so steps past the end change
-    // nothing, whatever Inf or NaN the real values hold.
-    const T* el = &E[par][lane];
-    if (qj < qi) {   // xt -= E(bi, bj) x(bj): the tile row and x(bj) read from LDS
-#pragma unroll
-      for (int k = 0; k < TRSM_NB; k++) {
-#pragma unroll
-        for (int vv = 0; vv < TRSM_VPW; vv++) xt[vv] -= el[k * LDE] * Xb[w][bj][vv][k];
-      }
-    } else {         // the diagonal block, as trsm_leaf_kernel, the tile row in registers
-      const int nk = min(TRSM_NB, nb - bi * TRSM_NB);
-      const bool live = lane < nk;
-      const T di = (live && !unit) ? T(1) / el[lane * LDE] : T(1);
-      T e[TRSM_NB];
-#pragma unroll
-      for (int k = 0; k < TRSM_NB; k++) e[k] = el[k * LDE];
-      if (elower) {
-#pragma unroll
-        for (int k = 0; k < TRSM_NB; k++) {
-          T xk[TRSM_VPW];
-#pragma unroll
-          for (int vv = 0; vv < TRSM_VPW; vv++) {
-            if (lane == k) xt[vv] *= di;
-            xk[vv] = bcast_lane(xt[vv], k);
-          }
-#pragma unroll
-          for (int vv = 0; vv < TRSM_VPW; vv++)
-            if (lane > k && live) xt[vv] -= e[k] * xk[vv];
-        }
-      } else {
-#pragma unroll
-        for (int k = TRSM_NB - 1; k >= 0; k--) {
-          T xk[TRSM_VPW];
-#pragma unroll
-          for (int vv = 0; vv < TRSM_VPW; vv++) {
-            if (lane == k) xt[vv] *= di;
-            xk[vv] = bcast_lane(xt[vv], k);
-          }
-#pragma unroll
-          for (int vv = 0; vv < TRSM_VPW; vv++)
-            if (lane < k && live) xt[vv] -= e[k] * xk[vv];
-        }
-      }
-#pragma unroll
-      for (int vv = 0; vv < TRSM_VPW; vv++) Xb[w][bi][vv][lane] = xt[vv];
-      if (more) {
-#pragma unroll
-        for (int vv = 0; vv < TRSM_VPW; vv++) xt[vv] = Xb[w][blk_of(ni)][vv][lane];
-      }
-    }
-    if (!more) break;
-    qi = ni;
-    qj = nj;
-    par ^= 1;
-  }
-#pragma unroll
-  for (int b = 0; b < MB; b++)
-#pragma unroll
-    for (int vv = 0; vv < TRSM_VPW; vv++) {
-      const long v = v0 + vv;
-      const int row = b * TRSM_NB + lane;
-      if (b < nblk && v < nvec && row < nb) B[v * inc_v + (long)row * inc_e] = Xb[w][b][vv][lane];
-    }
-}
-
-// Right-side leaves through explicit inverses of the 64x64 diagonal blocks:
-// a fully unrolled per-row substitution is ~4000 straight-line instructions
-// run once per wavefront and measured at 40-65 us per leaf whatever its
-// size (instruction fetch); the two kernels below replace it.
+// Leaves through explicit inverses of the 64x64 diagonal blocks, on either
+// side: a left-side solve op(A) X = B is X^T op(A)^T = B^T, the right-side
+// kernel with M = op(A)^T and B's two strides exchanged.  A fully unrolled
+// per-row substitution is ~4000 straight-line instructions run once per
+// wavefront and measured at 40-65 us per right-side leaf whatever its size
+// (instruction fetch); the left side's, a wavefront per vector with 64x64 tiles
+// of the triangle through LDS, took 32.3 us per 256 x 1024 FP64 leaf.
 //
 // (1) One workgroup per diagonal block b of M = op(A) (upper or lower,
 //     unit or not) computes M_bb^{-1} by doubling, as the lower triangle L =
@@ -352,8 +217,9 @@ template <> struct TrMf<float> {
   __device__ static inline int orow(int l, int r) { return 4 * (l >> 4) + r; }
 };
 
-template <typename T, int RB, bool MT>
-__global__ __launch_bounds__(256) void trsm_right_kernel(int n, long nvec, const T* __restrict__ A, long lda,
+// LEFT: element (r, c) of the solve's B lies at B[c + r*ldb].
+template <typename T, int RB, bool MT, bool LEFT>
+__global__ __launch_bounds__(256) void trsm_block_kernel(int n, long nvec, const T* __restrict__ A, long lda,
                                                          bool upper, const T* __restrict__ inv, T* __restrict__ B,
                                                          long ldb, const int* abort_flag) {
   constexpr int LDX = RB + 2, RT = RB / 16, NB = TRSM_NB;
@@ -394,13 +260,13 @@ __global__ __launch_bounds__(256) void trsm_right_kernel(int n, long nvec, const
     T v[16];
 #pragma unroll
     for (int u = 0; u < 16; u++) {
-      const int i = i0 + t + 256 * u, r = i % RB, c = i / RB;
-      v[u] = B[v0 + min(r, rows - 1) + (long)min(c, n - 1) * ldb];
+      const int i = i0 + t + 256 * u, r = LEFT ? i / np : i % RB, c = LEFT ? i % np : i / RB;
+      v[u] = LEFT ? B[min(c, n - 1) + (v0 + min(r, rows - 1)) * ldb] : B[v0 + min(r, rows - 1) + (long)min(c, n - 1) * ldb];
     }
 #pragma unroll
     for (int u = 0; u < 16; u++) {
-      const int i = i0 + t + 256 * u, r = i % RB, c = i / RB;
-      if (c < np) Xs[c * LDX + r] = c < n && r < rows ? v[u] : T(0);
+      const int i = i0 + t + 256 * u, r = LEFT ? i / np : i % RB, c = LEFT ? i % np : i / RB;
+      if (LEFT ? r < RB : c < np) Xs[c * LDX + r] = c < n && r < rows ? v[u] : T(0);
     }
   }
   __syncthreads();
@@ -439,7 +305,7 @@ __global__ __launch_bounds__(256) void trsm_right_kernel(int n, long nvec, const
         for (int x = 0; x < 4; x++) {
           const int c = 16 * w + mf::orow(lane, x), r = 16 * i + lr;
           xb[c * LDX + r] = acc[i][x];
-          if (r < rows && b * NB + c < n) B[v0 + r + (long)(b * NB + c) * ldb] = acc[i][x];
+          if (!LEFT && r < rows && b * NB + c < n) B[v0 + r + (long)(b * NB + c) * ldb] = acc[i][x];
           acc[i][x] = T(0);
         }
       if (nq >= nblk) break;
@@ -448,10 +314,18 @@ __global__ __launch_bounds__(256) void trsm_right_kernel(int n, long nvec, const
     q = nq;
     p = np2;
   }
+  if constexpr (LEFT) {   // consecutive elements of a column of B to consecutive lanes
+    __syncthreads();
+    for (int i = t; i < np * RB; i += 256) {
+      const int r = i / np, c = i % np;
+      if (c < n && r < rows) B[c + (v0 + r) * ldb] = Xs[c * LDX + r];
+    }
+  }
 }
 
-// inverses of op(A)'s diagonal blocks for a right-side solve (a0: the
-// triangle's first element; the recursion splits on the 64-grid from a0)
+// inverses of the diagonal blocks of M (op(A), for a left-side solve its
+// transpose; a0: the triangle's first element; the recursion splits on the
+// 64-grid from a0)
 template <typename T>
 struct InvCtx {
   const T* a0 = nullptr;
@@ -463,35 +337,35 @@ template <typename T>
 static void leaf(bool right, bool lower, bool trans, bool unit, long nb, long nrhs, const T* a, long lda, T* b,
                  long ldb, hipStream_t s, const int* abort_flag, const InvCtx<T>& ic) {
   if (nb <= 0 || nrhs <= 0) return;
-  const bool eT = trans, elower = lower != eT;   // left: E = op(A)
-  if (right) {
+  if (right || ic.inv) {
     const T* inv = ic.inv + (long)(a - ic.a0) / (ic.lda + 1) / TRSM_NB * TRSM_NB * TRSM_NB;
-    const bool upper = lower == trans;   // op(A)
-#define OBA_TR(RB, MT)                                                                                             \
-  trsm_right_kernel<T, RB, MT><<<(unsigned)((nrhs + RB - 1) / RB), 256, 0, s>>>((int)nb, nrhs, a, lda, upper, inv, b, \
-                                                                                ldb, abort_flag)
-    // 32 rows per workgroup halve the reads of M: FP32 from two 16-row
+    const bool upper = right ? lower == trans : lower != trans;   // M
+#define OBA_TR(RB, MT, LEFT)                                                                                          \
+  trsm_block_kernel<T, RB, MT, LEFT><<<(unsigned)((nrhs + RB - 1) / RB), 256, 0, s>>>((int)nb, nrhs, a, lda, upper, inv, \
+                                                                                      b, ldb, abort_flag)
+    // 32 vectors per workgroup halve the reads of M: FP32 from two 16-vector
     // workgroups per CU on (16000 x 256: 54.5 us with 16 rows, 49.9 with 32);
     // FP64 is bound by its MFMAs (71.9 / 74.8)
-    if (sizeof(T) == 4 && nrhs >= 16 * 2 * (long)rt().num_cu) {
-      if (trans) OBA_TR(32, true); else OBA_TR(32, false);
+    const bool wide = sizeof(T) == 4 && nrhs >= 16 * 2 * (long)rt().num_cu;
+    if (!right) {
+      if (wide) { if (trans) OBA_TR(32, false, true); else OBA_TR(32, true, true); }
+      else { if (trans) OBA_TR(16, false, true); else OBA_TR(16, true, true); }
+    } else if (wide) {
+      if (trans) OBA_TR(32, true, false); else OBA_TR(32, false, false);
     } else {
-      if (trans) OBA_TR(16, true); else OBA_TR(16, false);
+      if (trans) OBA_TR(16, true, false); else OBA_TR(16, false, false);
     }
 #undef OBA_TR
     OBA_HIP(hipGetLastError());
     return;
   }
-  const long inc_e = 1, inc_v = ldb;
+  // a left-side triangle of one block: no inverse, one launch
+  const bool eT = trans, elower = lower != eT;   // E = op(A)
   const int waves = 4;
   const long per_block = (long)waves * TRSM_VPW;
   long blocks = (nrhs + per_block - 1) / per_block;
-  if (nb > TRSM_NB)
-    trsm_leafb_kernel<T><<<(unsigned)blocks, 64 * waves, 0, s>>>((int)nb, nrhs, a, lda, b, inc_e, inc_v, eT, elower,
-                                                                 unit, abort_flag);
-  else
-    trsm_leaf_kernel<T><<<(unsigned)blocks, 64 * waves, 0, s>>>((int)nb, nrhs, a, lda, b, inc_e, inc_v, eT, elower,
-                                                                unit, abort_flag);
+  trsm_leaf_kernel<T><<<(unsigned)blocks, 64 * waves, 0, s>>>((int)nb, nrhs, a, lda, b, 1, ldb, eT, elower, unit,
+                                                              abort_flag);
   OBA_HIP(hipGetLastError());
 }
 
@@ -500,9 +374,7 @@ template <typename T>
 static void rec(bool right, bool lower, bool trans, bool unit, long m, long n, const T* a, long lda, T* b,
                 long ldb, hipStream_t s, const int* abort_flag, const InvCtx<T>& ic) {
   const long na = right ? n : m;   // order of the triangle
-  // leaves: trsm_leafb_kernel (left), trsm_right_kernel (right; on the 64-grid
-  // of the diagonal inverses)
-  if (na <= (right ? TRSM_RN : TRSM_LEAF_MAX)) {
+  if (na <= TRSM_RN) {   // on the 64-grid of the diagonal inverses
     leaf<T>(right, lower, trans, unit, na, right ? m : n, a, lda, b, ldb, s, abort_flag, ic);
     return;
   }
@@ -556,11 +428,14 @@ void trsm(bool right, bool lower, bool trans, bool unit, long m, long n, T alpha
   if (alpha == T(0)) return;
   InvCtx<T> ic;
   DevBuf invb;
-  if (right) {
-    // M = op(A): upper when (upper, no transpose) or (lower, transpose)
-    const long nblk = (n + TRSM_NB - 1) / TRSM_NB;
+  const long na = right ? n : m;
+  if (right || na > TRSM_NB) {
+    // M = op(A) (right): upper when (upper, no transpose) or (lower,
+    // transpose); M = op(A)^T (left): the other two
+    const long nblk = (na + TRSM_NB - 1) / TRSM_NB;
     invb = DevBuf(sizeof(T) * (size_t)nblk * TRSM_NB * TRSM_NB);
-    trsm_inv_diag_kernel<T><<<(unsigned)nblk, 256, 0, s>>>(n, a, lda, trans, lower == trans, unit, invb.as<T>(),
+    trsm_inv_diag_kernel<T><<<(unsigned)nblk, 256, 0, s>>>(na, a, lda, right ? trans : !trans,
+                                                           right ? lower == trans : lower != trans, unit, invb.as<T>(),
                                                            abort_flag);
     OBA_HIP(hipGetLastError());
     ic.a0 = a;
