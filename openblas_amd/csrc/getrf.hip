@@ -1029,8 +1029,9 @@ struct LuLeaf {
   int* mv;
 };
 
-// the leaves of one block, in order, for lu_swap_block_kernel
-constexpr int LU_MAXL = 16;
+// the leaves of one block, in order, for lu_swap_block_kernel (slabs of
+// LU_SB_ROWS rows)
+constexpr int LU_MAXL = 16, LU_SB_ROWS = 16;
 struct LuLeafSet {
   long j0[LU_MAXL];
   const int* mv[LU_MAXL];
@@ -1039,40 +1040,50 @@ struct LuLeafSet {
 
 // The interchanges of all leaves of a block, in order, on the At rows in
 // [lo, hi) outside [ex_lo, ex_hi): lu_swap_kernel's gather/scatter once per
-// leaf inside one launch (each workgroup owns its 64-row slab throughout).
+// leaf inside one launch (each workgroup owns its slab of rows throughout).
+// The bound is the chain of a load and a store per leaf, so all leaves' moves
+// come to LDS first and slabs are 16 rows (one 128-byte line of a column in
+// FP64): 5001 rows, 16 leaves 24.7 us FP64; 143 with 64-row slabs (79
+// workgroups), the moves read leaf by leaf and the values passed through LDS.
 template <typename T, int W>
 __global__ __launch_bounds__(256) void lu_swap_block_kernel(T* __restrict__ At, long ldt, long lo, long hi, long ex_lo,
                                                             long ex_hi, long m, LuLeafSet ls) {
-  constexpr int RB = 64;
-  __shared__ int sd[2 * W], ss[2 * W];
-  __shared__ int s_cnt;
-  __shared__ T vals[2 * W][RB];
-  const long r0 = lo + (long)blockIdx.x * RB;
-  for (int l = 0; l < ls.n; l++) {
-    const long j0 = ls.j0[l], mp = m - j0;
+  constexpr int RB = LU_SB_ROWS, MU = 2 * W * RB / 256;
+  __shared__ int sd[LU_MAXL][2 * W], ss[LU_MAXL][2 * W];
+  __shared__ int s_cnt[LU_MAXL];
+  const int t = threadIdx.x;
+  for (int i = t; i < ls.n * 2 * W; i += 256) {
+    const int l = i / (2 * W), k = i % (2 * W);
     const int* moves = ls.mv[l];
-    if (threadIdx.x == 0) s_cnt = min(max(moves[0], 0), 2 * W);
-    __syncthreads();
-    const int cnt = s_cnt;
-    if ((int)threadIdx.x < cnt) {
-      int d = moves[1 + 2 * threadIdx.x], sr = moves[2 + 2 * threadIdx.x];
+    const long mp = m - ls.j0[l];
+    const int cnt = min(max(moves[0], 0), 2 * W);
+    if (k == 0) s_cnt[l] = cnt;
+    if (k < cnt) {
+      int d = moves[1 + 2 * k], sr = moves[2 + 2 * k];
       if (d < 0 || d >= mp || sr < 0 || sr >= mp) d = sr = 0;   // never index outside the panel rows
-      sd[threadIdx.x] = d;
-      ss[threadIdx.x] = sr;
+      sd[l][k] = d;
+      ss[l][k] = sr;
     }
-    __syncthreads();
-    for (int idx = threadIdx.x; idx < cnt * RB; idx += blockDim.x) {
-      const int k = idx / RB, rr = idx % RB;
-      const long r = r0 + rr;
-      if (r < hi && !(r >= ex_lo && r < ex_hi)) vals[k][rr] = At[r + (j0 + ss[k]) * ldt];
+  }
+  __syncthreads();
+  const long r = lo + (long)blockIdx.x * RB + t % RB;
+  const bool in = r < hi && !(r >= ex_lo && r < ex_hi);
+  for (int l = 0; l < ls.n; l++) {
+    T* const col = At + r + ls.j0[l] * ldt;
+    const int cnt = s_cnt[l];
+    T v[MU];
+#pragma unroll
+    for (int u = 0; u < MU; u++) {
+      const int k = t / RB + u * (256 / RB);
+      v[u] = in && k < cnt ? col[ss[l][k] * ldt] : T(0);
     }
-    __syncthreads();
-    for (int idx = threadIdx.x; idx < cnt * RB; idx += blockDim.x) {
-      const int k = idx / RB, rr = idx % RB;
-      const long r = r0 + rr;
-      if (r < hi && !(r >= ex_lo && r < ex_hi)) At[r + (j0 + sd[k]) * ldt] = vals[k][rr];
+    __syncthreads();   // every read before any write: a move's destination can be another's source
+#pragma unroll
+    for (int u = 0; u < MU; u++) {
+      const int k = t / RB + u * (256 / RB);
+      if (in && k < cnt) col[sd[l][k] * ldt] = v[u];
     }
-    __syncthreads();   // before the next leaf's moves overwrite s_cnt, sd, ss and vals
+    __syncthreads();   // and every write before the next leaf's reads
   }
 }
 
@@ -1249,8 +1260,8 @@ static void lu_blocked(LuCtx<T>& c, long mn, long nb) {
       LuLeafSet ls;
       ls.n = (int)std::min<size_t>(LU_MAXL, c.leaves.size() - l);
       for (int i = 0; i < ls.n; i++) { ls.j0[i] = c.leaves[l + i].j0; ls.mv[i] = c.leaves[l + i].mv; }
-      lu_swap_block_kernel<T, LU_W><<<(unsigned)((c.nrows_t + 63) / 64), 256, 0, M>>>(At, ldt, 0, c.nrows_t, jb, jn,
-                                                                                    c.m, ls);
+      lu_swap_block_kernel<T, LU_W><<<(unsigned)((c.nrows_t + LU_SB_ROWS - 1) / LU_SB_ROWS), 256, 0, M>>>(
+          At, ldt, 0, c.nrows_t, jb, jn, c.m, ls);
       OBA_HIP(hipGetLastError());
     }
     if (jn >= mn) break;
