@@ -375,9 +375,14 @@ void gemm(bool ta, bool tb, long m, long n, long k, T alpha, const T* a, long ld
   }
   // FP32 (16-cycle steps) needs the LDS reuse of 128x128 tiles once there are
   // enough of them: 8192^3 7883 us against 8414 with 64x64; 3000^3 574 / 468
+  // FP64 gains from them at the largest sizes only, where 64x64 tiles read A and
+  // B 40 times over (normal random data, 64x64x8 / 128x128x8 / 128x128x4, ms):
+  // 8192^3 16.43 (17.7 on a card whose memory is slower) / 15.63 / 15.82, 6000^3
+  // 6.78 / 6.56 / 6.58, 4000^3 1.97 / 1.98 / 1.94, 6144^2 x 2048 2.25 / 2.28 /
+  // 2.30, 12000^2 x 448 2.00 / 2.20 / 2.12
   const long m128 = (m + 127) / 128, t128 = tri ? m128 * (m128 + 1) / 2 : m128 * ((n + 127) / 128);
   if (t64 <= 2 * cu && k >= 256) launch_cfg<T, 64, 64, BK64, 2, 2>(OBA_GEMM_ARGS);
-  else if (!D && t128 >= 8 * cu) launch_cfg<T, 128, 128, 16, 1, 2>(OBA_GEMM_ARGS);
+  else if (t128 >= 8 * cu && (!D || (tri == 0 && k >= 4096))) launch_cfg<T, 128, 128, D ? 8 : 16, 1, 2>(OBA_GEMM_ARGS);
   else launch_cfg<T, 64, 64, BK64, 1, 4>(OBA_GEMM_ARGS);
 #undef OBA_GEMM_ARGS
 }
