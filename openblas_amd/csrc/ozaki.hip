@@ -490,7 +490,6 @@ constexpr int CRT_PIECES = 14;   // 18-bit pieces of a scaled operand: t <= 252 
 constexpr int CRT_L16 = 2 * CRT_LIMBS;   // 16-bit limbs of the CRT sums
 struct CrtTab {
   int p[CRT_NMAX];
-  double invp[CRT_NMAX];
   float invpf[CRT_NMAX];
   int c18[CRT_NMAX][CRT_PIECES];                     // 2^(18 i) mod p, balanced
   unsigned q[CRT_NMAX + 1][CRT_NMAX][CRT_LIMBS];     // Q_m for the first NM moduli (32-bit limbs)
@@ -532,7 +531,6 @@ static const CrtTab& crt_host_tab() {
   for (int m = 0; m < CRT_NMAX; m++) {
     const int p = kCrtModuli[m];
     T.p[m] = p;
-    T.invp[m] = 1.0 / p;
     T.invpf[m] = 1.0f / (float)p;
     long v = 1 % p;
     for (int i = 0; i < CRT_PIECES; i++) { T.c18[m][i] = (int)(v > p / 2 ? v - p : v); v = (v * (1L << 18)) % p; }
