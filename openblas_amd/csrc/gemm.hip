@@ -320,7 +320,8 @@ void gemm(bool ta, bool tb, long m, long n, long k, T alpha, const T* a, long ld
   // per synchronous call (launch and completion about 10 us of it), NN unless
   // said; the last column is the kernel before this table (128x128 or 64x64
   // tiles, per-element loads at odd leading dimensions, fragments read in
-  // front of their own MFMAs):
+  // front of their own MFMAs; 8192^3 on data that draw little power, normal
+  // random data further down):
   //   FP64            64x64x8 KS1  KS2  64x32x16 KS2  32x32x16 KS1  KS2   before
   //   8192^3                15009  15300        16224         17668  18713  16400
   //   2047x3001x1501 TN       320    327          370           430    488    617
