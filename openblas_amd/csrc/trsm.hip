@@ -8,11 +8,12 @@
 //
 // Design: recursive blocking on the triangle (split in halves on a 64-row
 // grid) so that almost all flops land in large MFMA GEMM updates.  Leaves (up
-// to 256 rows or columns of the triangle) multiply by explicit inverses of the
-// 64x64 diagonal blocks; a left-side triangle of a single block is solved by
-// wavefronts of right-hand-side vectors: lane i owns x_i and row i of the
-// triangle, and x_k is broadcast with v_readlane after it is final (forward or
-// backward column-oriented substitution).
+// to 256 rows or columns of the triangle) are substitutions on the left side
+// and multiply by explicit inverses of the 64x64 diagonal blocks on the right.
+// A left-side triangle of a single block is solved by wavefronts of
+// right-hand-side vectors: lane i owns x_i and row i of the triangle, and x_k is
+// broadcast with v_readlane after it is final (forward or backward
+// column-oriented substitution).
 #include "kernels.h"
 #include "tri_inv.h"
 
@@ -121,13 +122,11 @@ __global__ __launch_bounds__(256) void trsm_leaf_kernel(int nb, long nvec, const
   }
 }
 
-// Leaves through explicit inverses of the 64x64 diagonal blocks, on either
-// side: a left-side solve op(A) X = B is X^T op(A)^T = B^T, the right-side
-// kernel with M = op(A)^T and B's two strides exchanged.  A fully unrolled
-// per-row substitution is ~4000 straight-line instructions run once per
-// wavefront and measured at 40-65 us per right-side leaf whatever its size
-// (instruction fetch); the left side's, a wavefront per vector with 64x64 tiles
-// of the triangle through LDS, took 32.3 us per 256 x 1024 FP64 leaf.
+// Leaves of up to TRSM_RN rows or columns of the triangle in one launch: the
+// right side through explicit inverses of the 64x64 diagonal blocks, the left
+// side by substitution.  (A fully unrolled per-row substitution on the right
+// side is ~4000 straight-line instructions run once per wavefront and measured
+// at 40-65 us per leaf whatever its size, instruction fetch.)
 //
 // (1) One workgroup per diagonal block b of M = op(A) (upper or lower,
 //     unit or not) computes M_bb^{-1} by doubling, as the lower triangle L =
@@ -191,7 +190,7 @@ __global__ __launch_bounds__(256) void trsm_inv_diag_kernel(long na, const T* __
 
 // (2) One launch solves X M = B for up to TRSM_RN columns, in place: a
 //     workgroup owns RB rows of B in LDS and takes the 64-column blocks in
-//     dependency order, X_b = (B_b - sum_k X_k M_kb) M_bb^{-1}, both products
+//     dependency order, X_b = (B_b - sum_k X_k M_kb) M_bb^{-1}, the products
 //     on the matrix cores (wavefront w: columns 16w..16w+15 of the block).
 //     The tiles of M and of the inverses come straight from L2 as fragments,
 //     the next tile's loads in flight behind the current one's MFMAs; step s
@@ -217,9 +216,8 @@ template <> struct TrMf<float> {
   __device__ static inline int orow(int l, int r) { return 4 * (l >> 4) + r; }
 };
 
-// LEFT: element (r, c) of the solve's B lies at B[c + r*ldb].
-template <typename T, int RB, bool MT, bool LEFT>
-__global__ __launch_bounds__(256) void trsm_block_kernel(int n, long nvec, const T* __restrict__ A, long lda,
+template <typename T, int RB, bool MT>
+__global__ __launch_bounds__(256) void trsm_right_kernel(int n, long nvec, const T* __restrict__ A, long lda,
                                                          bool upper, const T* __restrict__ inv, T* __restrict__ B,
                                                          long ldb, const int* abort_flag) {
   constexpr int LDX = RB + 2, RT = RB / 16, NB = TRSM_NB;
@@ -260,13 +258,13 @@ __global__ __launch_bounds__(256) void trsm_block_kernel(int n, long nvec, const
     T v[16];
 #pragma unroll
     for (int u = 0; u < 16; u++) {
-      const int i = i0 + t + 256 * u, r = LEFT ? i / np : i % RB, c = LEFT ? i % np : i / RB;
-      v[u] = LEFT ? B[min(c, n - 1) + (v0 + min(r, rows - 1)) * ldb] : B[v0 + min(r, rows - 1) + (long)min(c, n - 1) * ldb];
+      const int i = i0 + t + 256 * u, r = i % RB, c = i / RB;
+      v[u] = B[v0 + min(r, rows - 1) + (long)min(c, n - 1) * ldb];
     }
 #pragma unroll
     for (int u = 0; u < 16; u++) {
-      const int i = i0 + t + 256 * u, r = LEFT ? i / np : i % RB, c = LEFT ? i % np : i / RB;
-      if (LEFT ? r < RB : c < np) Xs[c * LDX + r] = c < n && r < rows ? v[u] : T(0);
+      const int i = i0 + t + 256 * u, r = i % RB, c = i / RB;
+      if (c < np) Xs[c * LDX + r] = c < n && r < rows ? v[u] : T(0);
     }
   }
   __syncthreads();
@@ -305,7 +303,7 @@ __global__ __launch_bounds__(256) void trsm_block_kernel(int n, long nvec, const
         for (int x = 0; x < 4; x++) {
           const int c = 16 * w + mf::orow(lane, x), r = 16 * i + lr;
           xb[c * LDX + r] = acc[i][x];
-          if (!LEFT && r < rows && b * NB + c < n) B[v0 + r + (long)(b * NB + c) * ldb] = acc[i][x];
+          if (r < rows && b * NB + c < n) B[v0 + r + (long)(b * NB + c) * ldb] = acc[i][x];
           acc[i][x] = T(0);
         }
       if (nq >= nblk) break;
@@ -314,18 +312,268 @@ __global__ __launch_bounds__(256) void trsm_block_kernel(int n, long nvec, const
     q = nq;
     p = np2;
   }
-  if constexpr (LEFT) {   // consecutive elements of a column of B to consecutive lanes
-    __syncthreads();
-    for (int i = t; i < np * RB; i += 256) {
-      const int r = i / np, c = i % np;
-      if (c < n && r < rows) B[c + (v0 + r) * ldb] = Xs[c * LDX + r];
-    }
-  }
 }
 
-// inverses of the diagonal blocks of M (op(A), for a left-side solve its
-// transpose; a0: the triangle's first element; the recursion splits on the
-// 64-grid from a0)
+// x[0..N-1] += (y of lane K of each 16-lane row) * e[0..N-1], the broadcast
+// taken by the FMA itself; the leading s_nop covers the wait states between a
+// VALU write of y and its DPP read
+#define TRSM_DPP(T, D, Y, E, K) "v_fmac_" T "_dpp %" #D ", %" #Y ", %" #E " row_newbcast:%" #K " row_mask:0xf bank_mask:0xf\n\t"
+#define TRSM_AXPY(TY, T)                                                                                              \
+  template <int K, int N>                                                                                             \
+  __device__ __attribute__((always_inline)) inline void trsm_axpy(TY* x, TY y, const TY* e) {                         \
+    if constexpr (N == 4)                                                                                             \
+      asm("s_nop 1\n\t" TRSM_DPP(T, 0, 4, 5, 9) TRSM_DPP(T, 1, 4, 6, 9) TRSM_DPP(T, 2, 4, 7, 9) TRSM_DPP(T, 3, 4, 8, 9) \
+          : "+&v"(x[0]), "+&v"(x[1]), "+&v"(x[2]), "+&v"(x[3])                                                        \
+          : "v"(y), "v"(e[0]), "v"(e[1]), "v"(e[2]), "v"(e[3]), "n"(K));                                              \
+    else if constexpr (N == 3)                                                                                        \
+      asm("s_nop 1\n\t" TRSM_DPP(T, 0, 3, 4, 7) TRSM_DPP(T, 1, 3, 5, 7) TRSM_DPP(T, 2, 3, 6, 7)                       \
+          : "+&v"(x[0]), "+&v"(x[1]), "+&v"(x[2]) : "v"(y), "v"(e[0]), "v"(e[1]), "v"(e[2]), "n"(K));                  \
+    else if constexpr (N == 2)                                                                                        \
+      asm("s_nop 1\n\t" TRSM_DPP(T, 0, 2, 3, 5) TRSM_DPP(T, 1, 2, 4, 5)                                               \
+          : "+&v"(x[0]), "+&v"(x[1]) : "v"(y), "v"(e[0]), "v"(e[1]), "n"(K));                                          \
+    else if constexpr (N == 1)                                                                                        \
+      asm("s_nop 1\n\t" TRSM_DPP(T, 0, 1, 2, 3) : "+&v"(x[0]) : "v"(y), "v"(e[0]), "n"(K));                           \
+  }
+TRSM_AXPY(double, "f64")
+TRSM_AXPY(float, "f32")
+#undef TRSM_AXPY
+#undef TRSM_DPP
+
+// rows i, 16+i, ... of columns TRSM_SG*G.. of a 64x64 lower triangle E (E + i given)
+constexpr int TRSM_SG = 4;
+template <int G, typename T>
+__device__ __attribute__((always_inline)) inline void trsm_subst_read(T (&ec)[TRSM_SG][4], const T* e) {
+#pragma unroll
+  for (int c = 0; c < TRSM_SG; c++)
+#pragma unroll
+    for (int s = TRSM_SG * G / 16; s < 4; s++) ec[c][s] = e[(TRSM_SG * G + c) * (TRSM_NB + 1) + 16 * s];
+}
+// column C and the later ones of its group; x[v][s]: rows 16s+i less the
+// columns so far, nr[s] the negative reciprocals of their diagonal
+template <int C, int NV, typename T>
+__device__ __attribute__((always_inline)) inline void trsm_subst_col(T (&x)[NV][4], T (&sol)[NV][4], const T (&nr)[4],
+                                                                     const T (&ec)[TRSM_SG][4], int i) {
+  constexpr int S = C / 16, K = C % 16, S1 = K == 15 ? S + 1 : S;   // the last row of a step has none below it there
+#pragma unroll
+  for (int v = 0; v < NV; v++) {
+    // solved rows of the step take the column too: their solution is kept
+    // apart, and nothing reads x of a solved row
+    const T y = x[v][S] * nr[S];
+    sol[v][S] = i == K ? y : sol[v][S];
+    trsm_axpy<K, 4 - S1>(x[v] + S1, y, ec[C % TRSM_SG] + S1);
+  }
+  if constexpr ((C + 1) % TRSM_SG != 0) trsm_subst_col<C + 1>(x, sol, nr, ec, i);
+}
+template <int G, int NV, typename T>
+__device__ __attribute__((always_inline)) inline void trsm_subst_group(T (&x)[NV][4], T (&sol)[NV][4], const T (&nr)[4],
+                                                                       const T (&ec)[TRSM_SG][4], const T* e, int i) {
+  if constexpr (G + 1 < TRSM_NB / TRSM_SG) {
+    T en[TRSM_SG][4];
+    trsm_subst_read<G + 1>(en, e);
+    __builtin_amdgcn_sched_barrier(0);   // the next group's reads run behind this one's chain
+    trsm_subst_col<TRSM_SG * G>(x, sol, nr, ec, i);
+    __builtin_amdgcn_sched_barrier(0);
+    trsm_subst_group<G + 1>(x, sol, nr, en, e, i);
+  } else {
+    trsm_subst_col<TRSM_SG * G>(x, sol, nr, ec, i);
+  }
+}
+// One wavefront solves the 64x64 lower triangle E (E(i, k) at E[k*65 + i], its
+// diagonal's reciprocals apart in rinv) for 4 NV vectors in place: lane (i, g)
+// = (lane % 16, lane / 16) holds rows i, 16+i, 32+i and 48+i of vectors g, g+4,
+// ...  A row, once final, reaches the later ones by DPP inside the FMAs, so no
+// row leaves its wavefront and there is no barrier inside; an Inf or NaN stays
+// with the rows that depend on it.  The element (k, v) lies at xm[k*si + v] and
+// the reciprocal k at rinv[k*ri] (both strides negative: the rows of an upper
+// triangle, counted from its end).  The bound is the chain of 64 columns, a
+// multiplication and an FMA each.
+template <int NV, typename T>
+__device__ __attribute__((always_inline)) inline void trsm_subst64(const T* E, const T* rinv, int ri, T* xm, int si) {
+  int lane = threadIdx.x & 63;
+  asm volatile("" : "+v"(lane));   // the addresses and masks are made here, not kept from before the caller's loop
+  const int i = lane & 15, g = lane >> 4;
+  xm += i * si + g;
+  T x[NV][4], sol[NV][4], nr[4], ec[TRSM_SG][4];
+  trsm_subst_read<0>(ec, E + i);
+#pragma unroll
+  for (int s = 0; s < 4; s++) {
+    nr[s] = -rinv[(16 * s + i) * ri];
+#pragma unroll
+    for (int v = 0; v < NV; v++) {
+      x[v][s] = xm[16 * s * si + 4 * v];
+      sol[v][s] = T(0);
+    }
+  }
+  trsm_subst_group<0>(x, sol, nr, ec, E + i, i);
+#pragma unroll
+  for (int s = 0; s < 4; s++)
+#pragma unroll
+    for (int v = 0; v < NV; v++) xm[16 * s * si + 4 * v] = -sol[v][s];
+}
+
+// (3) One launch solves op(A) X = B for up to TRSM_RN rows, in place: a
+//     workgroup owns RB columns of B in LDS and takes the 64-row blocks in
+//     dependency order.  X_b = B_b - sum_k E_bk X_k on the matrix cores (E =
+//     op(A), the fragments straight from L2 as on the right side), then the
+//     diagonal block by substitution, every wavefront its own vectors: backward
+//     stable whatever the block's condition, and an Inf or NaN of B or A
+//     reaches only the rows that depend on it, as in the reference.  All tiles
+//     of the next block row are on their way from memory during a block's
+//     substitution.  The bound is that chain: per block 3700 cycles of
+//     substitution (58 a column), 600 to 1200 before it and about 1100 per tile
+//     product.  A synchronous call with 256 x 1024 FP64 takes 45.4 us (55.0 with
+//     a wavefront per vector and every tile through LDS; 49.9 with the right
+//     side's inverses, which lost up to the block's condition in backward error
+//     and sent an Inf or NaN to rows that do not depend on it), 8192 x 1024
+//     1.93 ms (2.92, 1.86).
+//     MT: the columns of M = E^T are rows of A as stored (E(i, k) = A(i, k)).
+template <typename T, int RB, bool MT>
+__global__ __launch_bounds__(256, 2) void trsm_left_kernel(int n, long nvec, const T* __restrict__ A, long lda,
+                                                           bool lower, bool unit, T* __restrict__ B, long ldb,
+                                                           const int* abort_flag) {
+  constexpr int LDX = RB + 2, RT = RB / 16, NB = TRSM_NB;
+  typedef TrMf<T> mf;
+  __shared__ T Xs[TRSM_RN * LDX];   // X(k, v) at Xs[k*LDX + v]
+  __shared__ T Es[NB * (NB + 1)];   // the diagonal block, an upper one reversed
+  __shared__ T s_rinv[TRSM_RN];     // reciprocals of the diagonal
+  if (abort_flag && *abort_flag) return;
+  const long v0 = (long)blockIdx.x * RB;
+  const int t = threadIdx.x, w = __builtin_amdgcn_readfirstlane(t >> 6);
+  int lane = t & 63;
+  const int nblk = (n + NB - 1) / NB;
+  const int vecs = (int)min((long)RB, nvec - v0);
+  auto blk_of = [&](int q) { return lower ? q : nblk - 1 - q; };   // lower: E is lower triangular
+  // rows and columns past n repeat one that is there: taken out where it
+  // matters.  Addresses step from load to load (a product of 64 bits each took
+  // longer than the loads).
+  auto fetch_diag = [&](int q, T (&f)[16]) __attribute__((always_inline)) {
+    const int o = blk_of(q) * NB, c0 = min(o + w, n - 1);
+    const T* src = A + (long)c0 * lda;
+    const int r = min(o + lane, n - 1);
+#pragma unroll
+    for (int u = 0; u < 16; u++) {
+      f[u] = src[r];
+      src += c0 + 4 * u + 4 < n ? 4 * lda : 0;
+    }
+  };
+  // step s of a product takes k = kof(s) + KL*(lane/16) of the tile: rows of A
+  // in pieces of 128 bytes (MT), columns in pieces of 64, 16 per lane
+  constexpr int V = 16 / (int)sizeof(T), KL = MT ? 1 : V;
+  auto kof = [](int s) { return MT ? 4 * s : s / V * (4 * V) + s % V; };
+  auto fetch = [&](int q, int p, T (&f)[16]) __attribute__((always_inline)) {
+    const int i = min(blk_of(q) * NB + 16 * w + (lane & 15), n - 1), k0 = blk_of(p) * NB + KL * (lane >> 4);
+    const bool whole = (blk_of(p) + 1) * NB <= n;
+    if constexpr (MT) {
+      const T* src = A + i + (long)min(k0, n - 1) * lda;
+      if (whole) {
+#pragma unroll
+        for (int s = 0; s < 16; s++) {
+          f[s] = *src;
+          src += 4 * lda;
+        }
+      } else {
+#pragma unroll
+        for (int s = 0; s < 16; s++) {
+          f[s] = *src;
+          src += k0 + kof(s + 1) < n ? 4 * lda : 0;
+        }
+      }
+    } else {
+      const T* src = A + (long)i * lda;
+      if (whole) {
+        typedef T vec __attribute__((ext_vector_type(16 / sizeof(T)), aligned(sizeof(T))));
+#pragma unroll
+        for (int s = 0; s < 16; s += V) {
+          const vec x = *(const vec*)(src + k0 + kof(s));
+#pragma unroll
+          for (int e = 0; e < V; e++) f[s + e] = x[e];
+        }
+      } else {
+#pragma unroll
+        for (int s = 0; s < 16; s++) f[s] = src[min(k0 + kof(s), n - 1)];
+      }
+    }
+  };
+  T fd[16], f0[16], f1[16], f2[16];
+  fetch_diag(0, fd);
+  s_rinv[t] = t < n && !unit ? T(1) / A[t + (long)t * lda] : T(1);   // TRSM_RN threads
+#pragma unroll
+  for (int r0 = 0; r0 < RB; r0 += 16) {   // a thread per row of X
+    T v[16];
+#pragma unroll
+    for (int u = 0; u < 16; u++) v[u] = B[min(t, n - 1) + (v0 + min(r0 + u, vecs - 1)) * ldb];
+#pragma unroll
+    for (int u = 0; u < 16; u++) Xs[t * LDX + r0 + u] = t < n && r0 + u < vecs ? v[u] : T(0);
+  }
+  __syncthreads();
+#pragma unroll 1
+  for (int q = 0; q < nblk; q++) {
+    const int b = blk_of(q);
+    T* const xb = Xs + b * NB * LDX;
+    asm volatile("" : "+v"(lane));   // a block's addresses are made in its turn: all kept from before the loop they spill
+    const int lr = lane & 15, lg = lane >> 4;
+    {
+      // Of E(r, c) only r > c counts (r < c of an upper one): the other entries
+      // meet rows that are solved already.  But columns past n come first in
+      // an upper one and have to be zero.
+      if (!lower && (b + 1) * NB > n) {
+#pragma unroll
+        for (int u = 0; u < 16; u++) fd[u] = b * NB + (MT ? w + 4 * u : lane) < n ? fd[u] : T(0);
+      }
+      const int r = MT ? lane : w, c = MT ? w : lane, dir = lower ? 1 : -1, step = dir * (MT ? 4 * (NB + 1) : 4);
+      T* dst = Es + (lower ? c * (NB + 1) + r : (NB - 1 - c) * (NB + 1) + NB - 1 - r);
+#pragma unroll
+      for (int u = 0; u < 16; u++) {
+        *dst = fd[u];
+        dst += step;
+      }
+    }
+    if (q > 0) {   // less the products of the solved blocks, in place, every wavefront its 16 rows
+      typename mf::acc acc[RT];
+#pragma unroll
+      for (int i = 0; i < RT; i++) acc[i] = typename mf::acc{};
+      auto product = [&](int p, const T (&f)[16]) __attribute__((always_inline)) {
+        const T* src = Xs + (blk_of(p) * NB + KL * lg) * LDX + lr;
+#pragma unroll
+        for (int s = 0; s < 16; s++)
+#pragma unroll
+          for (int i = 0; i < RT; i++) acc[i] = mf::mma(f[s], src[kof(s) * LDX + 16 * i], acc[i]);
+      };
+      if (blk_of(0) == nblk - 1) {   // its rows past n
+#pragma unroll
+        for (int s = 0; s < 16; s++) f0[s] = (nblk - 1) * NB + KL * lg + kof(s) < n ? f0[s] : T(0);
+      }
+      product(0, f0);
+      if (q > 1) product(1, f1);
+      if (q > 2) product(2, f2);
+#pragma unroll
+      for (int i = 0; i < RT; i++)
+#pragma unroll
+        for (int x = 0; x < 4; x++) xb[(16 * w + mf::orow(lane, x)) * LDX + 16 * i + lr] -= acc[i][x];
+    }
+    if (q + 1 < nblk) {
+      fetch_diag(q + 1, fd);
+      fetch(q + 1, 0, f0);
+      if (q > 0) fetch(q + 1, 1, f1);
+      if (q > 1) fetch(q + 1, 2, f2);
+    }
+    __syncthreads();
+    const int first = lower ? 0 : NB - 1, dir = lower ? 1 : -1;
+    trsm_subst64<RT>(Es, s_rinv + b * NB + first, dir, xb + w * (RB / 4) + first * LDX, dir * LDX);
+    __syncthreads();
+  }
+  int nv = vecs;
+  asm volatile("" : "+s"(nv));   // nor the comparisons made for the loads
+  if (t < n) {   // consecutive rows of a column of B to consecutive lanes
+#pragma unroll
+    for (int r = 0; r < RB; r++)
+      if (r < nv) B[t + (v0 + r) * ldb] = Xs[t * LDX + r];
+  }
+}
+static_assert(TRSM_RN == 4 * TRSM_NB, "a row per thread; at most three solved blocks before the last");
+
+// right side: inverses of op(A)'s diagonal blocks (a0: the triangle's first
+// element; the recursion splits on the 64-grid from a0)
 template <typename T>
 struct InvCtx {
   const T* a0 = nullptr;
@@ -337,34 +585,42 @@ template <typename T>
 static void leaf(bool right, bool lower, bool trans, bool unit, long nb, long nrhs, const T* a, long lda, T* b,
                  long ldb, hipStream_t s, const int* abort_flag, const InvCtx<T>& ic) {
   if (nb <= 0 || nrhs <= 0) return;
-  if (right || ic.inv) {
+  // 32 vectors per workgroup halve the reads of the triangle: FP32 from two
+  // 16-vector workgroups per CU on (right, 16000 x 256: 54.5 us with 16 rows,
+  // 49.9 with 32); FP64 is bound by its MFMAs (71.9 / 74.8)
+  [[maybe_unused]] const bool wide = nrhs >= 16 * 2 * (long)rt().num_cu;
+  if (right) {
     const T* inv = ic.inv + (long)(a - ic.a0) / (ic.lda + 1) / TRSM_NB * TRSM_NB * TRSM_NB;
-    const bool upper = right ? lower == trans : lower != trans;   // M
-#define OBA_TR(RB, MT, LEFT)                                                                                          \
-  trsm_block_kernel<T, RB, MT, LEFT><<<(unsigned)((nrhs + RB - 1) / RB), 256, 0, s>>>((int)nb, nrhs, a, lda, upper, inv, \
-                                                                                      b, ldb, abort_flag)
-    // 32 vectors per workgroup halve the reads of M: FP32 from two 16-vector
-    // workgroups per CU on (16000 x 256: 54.5 us with 16 rows, 49.9 with 32);
-    // FP64 is bound by its MFMAs (71.9 / 74.8)
-    const bool wide = sizeof(T) == 4 && nrhs >= 16 * 2 * (long)rt().num_cu;
-    if (!right) {
-      if (wide) { if (trans) OBA_TR(32, false, true); else OBA_TR(32, true, true); }
-      else { if (trans) OBA_TR(16, false, true); else OBA_TR(16, true, true); }
-    } else if (wide) {
-      if (trans) OBA_TR(32, true, false); else OBA_TR(32, false, false);
-    } else {
-      if (trans) OBA_TR(16, true, false); else OBA_TR(16, false, false);
-    }
-#undef OBA_TR
+    const bool upper = lower == trans;   // op(A)
+    auto launch = [&](auto rb) {
+      constexpr int RB = decltype(rb)::value;
+      const unsigned g = (unsigned)((nrhs + RB - 1) / RB);
+      if (trans) trsm_right_kernel<T, RB, true><<<g, 256, 0, s>>>((int)nb, nrhs, a, lda, upper, inv, b, ldb, abort_flag);
+      else trsm_right_kernel<T, RB, false><<<g, 256, 0, s>>>((int)nb, nrhs, a, lda, upper, inv, b, ldb, abort_flag);
+    };
+    if constexpr (sizeof(T) == 4) wide ? launch(std::integral_constant<int, 32>{}) : launch(std::integral_constant<int, 16>{});
+    else launch(std::integral_constant<int, 16>{});
     OBA_HIP(hipGetLastError());
     return;
   }
-  // a left-side triangle of one block: no inverse, one launch
-  const bool eT = trans, elower = lower != eT;   // E = op(A)
+  const bool elower = lower != trans;   // E = op(A)
+  if (nb > TRSM_NB) {
+    auto launch = [&](auto rb) {
+      constexpr int RB = decltype(rb)::value;
+      const unsigned g = (unsigned)((nrhs + RB - 1) / RB);
+      if (trans) trsm_left_kernel<T, RB, false><<<g, 256, 0, s>>>((int)nb, nrhs, a, lda, elower, unit, b, ldb, abort_flag);
+      else trsm_left_kernel<T, RB, true><<<g, 256, 0, s>>>((int)nb, nrhs, a, lda, elower, unit, b, ldb, abort_flag);
+    };
+    if constexpr (sizeof(T) == 4) wide ? launch(std::integral_constant<int, 32>{}) : launch(std::integral_constant<int, 16>{});
+    else launch(std::integral_constant<int, 16>{});
+    OBA_HIP(hipGetLastError());
+    return;
+  }
+  // a left-side triangle of one block
   const int waves = 4;
   const long per_block = (long)waves * TRSM_VPW;
   long blocks = (nrhs + per_block - 1) / per_block;
-  trsm_leaf_kernel<T><<<(unsigned)blocks, 64 * waves, 0, s>>>((int)nb, nrhs, a, lda, b, 1, ldb, eT, elower, unit,
+  trsm_leaf_kernel<T><<<(unsigned)blocks, 64 * waves, 0, s>>>((int)nb, nrhs, a, lda, b, 1, ldb, trans, elower, unit,
                                                               abort_flag);
   OBA_HIP(hipGetLastError());
 }
@@ -428,14 +684,11 @@ void trsm(bool right, bool lower, bool trans, bool unit, long m, long n, T alpha
   if (alpha == T(0)) return;
   InvCtx<T> ic;
   DevBuf invb;
-  const long na = right ? n : m;
-  if (right || na > TRSM_NB) {
-    // M = op(A) (right): upper when (upper, no transpose) or (lower,
-    // transpose); M = op(A)^T (left): the other two
-    const long nblk = (na + TRSM_NB - 1) / TRSM_NB;
+  if (right) {
+    // op(A) is upper when (upper, no transpose) or (lower, transpose)
+    const long nblk = (n + TRSM_NB - 1) / TRSM_NB;
     invb = DevBuf(sizeof(T) * (size_t)nblk * TRSM_NB * TRSM_NB);
-    trsm_inv_diag_kernel<T><<<(unsigned)nblk, 256, 0, s>>>(na, a, lda, right ? trans : !trans,
-                                                           right ? lower == trans : lower != trans, unit, invb.as<T>(),
+    trsm_inv_diag_kernel<T><<<(unsigned)nblk, 256, 0, s>>>(n, a, lda, trans, lower == trans, unit, invb.as<T>(),
                                                            abort_flag);
     OBA_HIP(hipGetLastError());
     ic.a0 = a;
