@@ -117,21 +117,27 @@ double cost(const BDesc& d) { return (double)std::max(d.m, 1) * std::max(d.n, 1)
 
 // Largest first: a counting sort on the exponent and the leading 4 mantissa
 // bits of the cost, which is as fine as the work queues need (a comparison sort
-// of the 80-byte descriptors took half the host time of a call).
+// of the 80-byte descriptors took half the host time of a call with 10^4
+// problems).  Only the keys that occur are counted: a pass over all 4096 was
+// 2 us of a 40 us call.
 void order_largest_first(std::vector<BDesc>& p) {
-  constexpr int NB = 1 << 12;
-  std::vector<int> at(NB + 1, 0);
   std::vector<unsigned short> key(p.size());
+  unsigned lo = 0xffff, hi = 0;
   for (size_t i = 0; i < p.size(); i++) {
     const float c = (float)cost(p[i]);
     unsigned b;
     memcpy(&b, &c, sizeof b);
-    key[i] = (unsigned short)(NB - 1 - (b >> 19));   // cost >= 1: the sign bit is clear
-    at[key[i] + 1]++;
+    b >>= 19;   // cost >= 1: the sign bit is clear
+    key[i] = (unsigned short)b;
+    lo = std::min(lo, b);
+    hi = std::max(hi, b);
   }
-  for (int b = 0; b < NB; b++) at[b + 1] += at[b];
+  if (lo >= hi) return;   // one size class, or nothing
+  std::vector<int> at(hi - lo + 2, 0);
+  for (auto k : key) at[hi - k + 1]++;
+  for (size_t b = 1; b < at.size(); b++) at[b] += at[b - 1];
   std::vector<BDesc> out(p.size());
-  for (size_t i = 0; i < p.size(); i++) out[at[key[i]]++] = p[i];
+  for (size_t i = 0; i < p.size(); i++) out[at[hi - key[i]]++] = p[i];
   p.swap(out);
 }
 
