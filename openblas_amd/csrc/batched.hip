@@ -507,6 +507,8 @@ __global__ __launch_bounds__(256) void bgetrs_kernel(const BDesc* __restrict__ d
 // ---- host side: plans, graphs, tuning -------------------------------------------
 namespace {
 
+constexpr int BCTR = 8 * BG_CTR;   // words of a plan's queue counters
+
 struct Cfg {
   int var = 0;    // kernel variant
   int grid = 2;   // persistent workgroups per CU
@@ -543,7 +545,7 @@ typedef void (*Launcher)(const Cfg& c, const void* ctx, const BDesc* tab, const 
 
 void enqueue(Launcher L, const Cfg& c, const void* ctx, const BDesc* tab, const void* extra, int nitems, int count,
              unsigned* ctr, int* info, hipStream_t s) {
-  bzero_kernel<<<1, 64, 0, s>>>(ctr, 8);
+  bzero_kernel<<<1, BCTR, 0, s>>>(ctr, BCTR);
   L(c, ctx, tab, extra, nitems, count, ctr, info, s);
 }
 
@@ -573,7 +575,7 @@ int* run_plan(int slot, Launcher L, const Cfg& c, const void* ctx, size_t ctx_by
   if (P.exec) { OBA_HIP(hipGraphExecDestroy(P.exec)); P.exec = nullptr; }
   P.probs.clear();
   P.tab = DevBuf(tb + extra.size() + 16);
-  P.ctr = DevBuf(256);
+  P.ctr = DevBuf(sizeof(unsigned) * BCTR);
   P.info = DevBuf(sizeof(int) * (size_t)std::max(count, 1));
   OBA_HIP(hipMemcpyAsync(P.tab.p, probs.data(), tb, hipMemcpyHostToDevice, r.stream));
   if (!extra.empty())
@@ -617,7 +619,7 @@ Cfg tune(const std::string& sig, const std::vector<Cfg>& cands, Launcher L, cons
     total += elem * (size_t)std::max(fs[rows_field], 1) * (size_t)std::max(fs[cols_field], 1);
   }
   DevBuf sbuf(total + 256), tsrc(sizeof(BDesc) * count), tdst(sizeof(BDesc) * count + extra.size() + 16),
-      ctr(256), info(sizeof(int) * (size_t)std::max(count, 1));
+      ctr(sizeof(unsigned) * BCTR), info(sizeof(int) * (size_t)std::max(count, 1));
   size_t off = 0;
   for (auto& d : scr) {
     const int* fs = &d.m;
@@ -683,6 +685,7 @@ std::vector<char> no_extra() { return {}; }
 int grid_of(const Cfg& c) { return std::max(1, rt().num_cu * c.grid); }
 
 // ---- launchers ---------------------------------------------------------------
+// nitems: the items of the longest segment
 template <typename T, bool TA, bool TB>
 void launch_gemm_form(const BDesc* tab, const void* extra, int nitems, unsigned* ctr, hipStream_t s) {
   static const int per_cu = [] {
@@ -691,7 +694,8 @@ void launch_gemm_form(const BDesc* tab, const void* extra, int nitems, unsigned*
     return std::max(n, 1);
   }();
   const BSeg* seg = (const BSeg*)extra;
-  bgemm_kernel<T, TA, TB><<<std::min(nitems, rt().num_cu * per_cu), 256, 0, s>>>(tab, seg, (const int2*)(seg + 1), ctr);
+  bgemm_kernel<T, TA, TB><<<8 * std::min(nitems, std::max(rt().num_cu * per_cu / 8, 1)), 256, 0, s>>>(
+      tab, seg, (const int2*)(seg + 1), ctr);
   OBA_HIP(hipGetLastError());
 }
 
@@ -803,7 +807,7 @@ void gemm_batched(int ta, int tb, std::vector<BDesc>& probs) {
     by += sizeof(T) * ((double)d.m * d.k + (double)d.k * d.n + (d.beta != 0.0 ? 2.0 : 1.0) * d.m * d.n);
   }
   KTimer kt("batched_gemm", rt().stream, fl, by);
-  run_plan(tslot<T>(BK_GEMM), launch_gemm<T>, c, ctx, sizeof ctx, probs, nw, work);
+  run_plan(tslot<T>(BK_GEMM), launch_gemm<T>, c, ctx, sizeof ctx, probs, *std::max_element(len, len + 8), work);
 }
 
 template <typename T>
