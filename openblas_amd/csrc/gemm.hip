@@ -343,23 +343,71 @@ void gemm(bool ta, bool tb, long m, long n, long k, T alpha, const T* a, long ld
   constexpr int BK32 = D ? 16 : 32, BK64 = D ? 8 : 16;
 #define OBA_GEMM_ARGS ta, tb, m, n, k, alpha, a, lda, b, ldb, beta, c, ldc, s, tri, abort_flag
   if (8 * t64 < 7 * cu) {
-    // a deep K of few tiles is split over workgroups too (256x256x8192 FP64:
-    // 95 us with four groups in one workgroup, 33 in 16 parts)
-    const long parts_w = std::min<long>({8L, cu / std::max(t32, 1L), k / 512});
-    if (ws_ok && tri == 0 && abort_flag == nullptr && k >= 1024 && parts_w > 1) {
-      const long kc = ((k + parts_w - 1) / parts_w + 15) / 16 * 16;
-      const int parts = (int)((k + kc - 1) / kc);
-      DevBuf w(sizeof(T) * (size_t)parts * m * n);
-      launch_cfg<T, 32, 32, BK32, 4, 2>(ta, tb, m, n, k, alpha, a, lda, b, ldb, T(0), w.as<T>(), m, s, 0, nullptr,
-                                        parts, kc, m * n);
-      const long total = m * n;
-      gemm_ksum_kernel<T><<<(unsigned)std::min<long>((total + 255) / 256, 4096), 256, 0, s>>>(m, n, parts, w.as<T>(),
-                                                                                             beta, c, ldc);
-      OBA_HIP(hipGetLastError());
-      return;
+    // A deep K of few tiles is split over workgroups too: 32x32 tiles with four
+    // groups while two parts of them fit the CUs (256x256x8192 FP64: 95 us
+    // unsplit, 33 in 16 parts), above that the tile and the parts that the
+    // measured rates below make fastest: us per unit of k and tile (32x32 tiles
+    // read both operands along k when op(A) is transposed and op(B) is not),
+    // per round of two workgroups on a CU, for the sum and per byte of a part.
+    // us per call, unsplit 32x32 / so split: FP64 640x256x4096 54 / 44,
+    // 512x640x4096 83 / 65, 1280x400x2048 74 / 61, 640x1280x8192 308 / 231, FP32
+    // 512x640x8192 114 / 64, 640x1280x1500 58 / 44; 512x1024x1024 stays at 32.
+    // A C of at most 32 columns (rows) takes 64x32 (32x32) tiles, whose clamped
+    // loads want two workgroups on a CU: 8192x28x4096 FP64 107 / 78, 16x5440x6528
+    // FP32 92 / 63; below k = 2048 nothing is gained.
+    if (ws_ok && tri == 0 && abort_flag == nullptr && k >= 1024) {
+      const long parts_w = std::min<long>({8L, cu / std::max(t32, 1L), k / 512});
+      long parts = 1, bm = 32, bn = 32;
+      if (parts_w > 1) {
+        parts = parts_w;
+      } else if (std::min(m, n) <= 32) {
+        if (n <= 32) bm = 64;
+        double best = 1e300;
+        for (long p = 1, t = n <= 32 ? t6432 : t32; p <= 12 && (p == 1 || (k >= 2048 && k >= 256 * p)); p++) {
+          const double c = (double)((p * t + cu - 1) / cu), v = c / (double)p * (c == 1.0 ? 1.5 : 1.0);
+          if (v < 0.97 * best) { best = v; parts = p; }
+        }
+      } else {
+        const bool clamped = std::min(m, n) < 64;
+        const double us64 = (D ? 0.033 : 0.0165) * (clamped ? 1.4 : 1.0);
+        const double us32 = D ? (ta && !tb ? 0.0127 : 0.0095) : (ta && !tb ? 0.0071 : 0.0060);
+        double best = 1e300;
+        auto tile = [&](long w, long t, double us, double alone) {   // alone: the factor of one workgroup on its CU
+          for (long p = 1; p <= 12 && (p == 1 || k >= 256 * p); p++) {
+            const long c = (p * t + cu - 1) / cu;
+            const double v = (double)(c * k) / (double)p * us * (c == 1 ? alone : 1.0) + 3.0 * (double)((c + 1) / 2) +
+                             (p == 1 ? 0.0 : 4.5 + 3e-7 * (double)(p * m * n) * sizeof(T));
+            if (v < best) { best = v; parts = p; bm = bn = w; }
+          }
+        };
+        tile(32, t32, us32, D ? 1.1 : 1.0);   // unsplit: four groups
+        tile(64, t64, us64, clamped ? 1.5 : 1.05);
+      }
+      if (parts > 1 || bm == 64) {
+        if (parts > 1) {
+          const long kc = ((k + parts - 1) / parts + 15) / 16 * 16;
+          const int np = (int)((k + kc - 1) / kc);
+          DevBuf w(sizeof(T) * (size_t)np * m * n);
+#define OBA_GEMM_SPLIT ta, tb, m, n, k, alpha, a, lda, b, ldb, T(0), w.as<T>(), m, s, 0, nullptr, np, kc, m * n
+          if (parts_w > 1) launch_cfg<T, 32, 32, BK32, 4, 2>(OBA_GEMM_SPLIT);
+          else if (bm == 32) launch_cfg<T, 32, 32, BK32, 2, 2>(OBA_GEMM_SPLIT);
+          else if (bn == 32) launch_cfg<T, 64, 32, BK32, 2, 2>(OBA_GEMM_SPLIT);
+          else launch_cfg<T, 64, 64, BK64, 2, 2>(OBA_GEMM_SPLIT);
+#undef OBA_GEMM_SPLIT
+          const long total = m * n;
+          gemm_ksum_kernel<T><<<(unsigned)std::min<long>((total + 255) / 256, 4096), 256, 0, s>>>(m, n, np, w.as<T>(), beta,
+                                                                                                 c, ldc);
+          OBA_HIP(hipGetLastError());
+          return;
+        }
+        if (bn == 64) {
+          launch_cfg<T, 64, 64, BK64, 2, 2>(OBA_GEMM_ARGS);
+          return;
+        }
+      }
     }
     if (k >= 1024 && t32 <= cu) launch_cfg<T, 32, 32, BK32, 4, 2>(OBA_GEMM_ARGS);
-    else if (k >= 1024 || (D && k >= 256 && t32 <= 2 * cu)) launch_cfg<T, 32, 32, BK32, 2, 2>(OBA_GEMM_ARGS);
+    else if (k >= 1024 || (k >= (D ? 256 : 512) && t32 <= 2 * cu)) launch_cfg<T, 32, 32, BK32, 2, 2>(OBA_GEMM_ARGS);
     else launch_cfg<T, 32, 32, BK32, 1, 4>(OBA_GEMM_ARGS);
     return;
   }
