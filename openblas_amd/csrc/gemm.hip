@@ -423,15 +423,22 @@ void gemm(bool ta, bool tb, long m, long n, long k, T alpha, const T* a, long ld
     }
   }
   // FP32 (16-cycle steps) needs the LDS reuse of 128x128 tiles once there are
-  // enough of them: 8192^3 7883 us against 8414 with 64x64; 3000^3 574 / 468
+  // enough of them: 8192^3 7883 us against 8414 with 64x64; 3000^3 574 / 468.
+  // With fewer they pay where their rounds of two per CU come out full (128x128
+  // / 64x64, us): NN 4096^3 1018 / 1069, 4096x2048x1000 141 / 149, TT 4096^3 1006
+  // / 1155, 8192x2048x200 74 / 78, 5440x4096x1000 (0.90 full) 390 / 403; not NN
+  // 5440x4096x1000 392 / 376, 5000^3 (0.78) 2140 / 2051, TT 3500^3 (0.77) 865 / 753.
+  // Nor below k = 128, where the tail's clamped loads show: 8192x5440x24 65 / 56.
   // FP64 gains from them at the largest sizes only, where 64x64 tiles read A and
   // B 40 times over (normal random data, 64x64x8 / 128x128x8 / 128x128x4, ms):
   // 8192^3 16.43 (17.7 on a card whose memory is slower) / 15.63 / 15.82, 6000^3
   // 6.78 / 6.56 / 6.58, 4000^3 1.97 / 1.98 / 1.94, 6144^2 x 2048 2.25 / 2.28 /
   // 2.30, 12000^2 x 448 2.00 / 2.20 / 2.12
   const long m128 = (m + 127) / 128, t128 = tri ? m128 * (m128 + 1) / 2 : m128 * ((n + 127) / 128);
+  const long slots = 2 * cu, rounds = (t128 + slots - 1) / slots;
+  const bool full128 = !D && tri == 0 && k >= 128 && t128 >= slots && t128 >= (ta && tb ? 0.85 : 0.95) * (double)(rounds * slots);
   if (t64 <= 2 * cu && k >= 256) launch_cfg<T, 64, 64, BK64, 2, 2>(OBA_GEMM_ARGS);
-  else if (t128 >= 8 * cu && (!D || (tri == 0 && k >= 4096))) launch_cfg<T, 128, 128, D ? 8 : 16, 1, 2>(OBA_GEMM_ARGS);
+  else if (full128 || (t128 >= 8 * cu && (D ? tri == 0 && k >= 4096 : k >= 128))) launch_cfg<T, 128, 128, D ? 8 : 16, 1, 2>(OBA_GEMM_ARGS);
   else launch_cfg<T, 64, 64, BK64, 1, 4>(OBA_GEMM_ARGS);
 #undef OBA_GEMM_ARGS
 }
