@@ -30,6 +30,7 @@
 #include "lu_internal.h"
 #include "lu_device.h"
 #include "lu_key.h"
+#include "wave.h"
 #include <cfloat>
 #include <climits>
 #include <cmath>

@@ -137,6 +137,7 @@ __global__ __launch_bounds__(L3_NT) void lu_panel3_kernel(T* __restrict__ At, lo
     vec v[RPT][4][NB];
     load_rows(j0, v);
     rows_to_lds(v);   // rows of this wavefront only
+    wave_fence();
 #pragma unroll
     for (int q = 0; q < RPT; q++) {
       y0[q] = s_l[wr0 + q * 64 + lane];
@@ -194,6 +195,7 @@ __global__ __launch_bounds__(L3_NT) void lu_panel3_kernel(T* __restrict__ At, lo
     }
     __syncthreads();
     rows_to_lds(v);
+    wave_fence();
     // 16-row tiles of this wavefront: the multipliers are replaced by the
     // products, which every thread then subtracts from its own rows
     const int lr = lane & 15, lk = lane >> 4;
@@ -218,6 +220,7 @@ __global__ __launch_bounds__(L3_NT) void lu_panel3_kernel(T* __restrict__ At, lo
 #pragma unroll
         for (int x = 0; x < 4; x++) tile[(16 * n + LuMf<T>::orow(lane, x)) * LDL] = acc[n][x];
     }
+    wave_fence();
 #pragma unroll
     for (int q = 0; q < RPT; q++) {
       y0[q] -= s_l[wr0 + q * 64 + lane];
@@ -310,6 +313,7 @@ __global__ __launch_bounds__(L3_NT) void lu_panel3_kernel(T* __restrict__ At, lo
         lb = l3_rlf(l[0], win);
         if (lane == win) put(y[0], y0[0]);
       }
+      wave_fence();
       rinv = l3_rlf(rinv, win);
       if constexpr (MULTI) {
         unsigned long long* dst = recs + (size_t)g * R::N;

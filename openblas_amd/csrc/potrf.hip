@@ -136,7 +136,9 @@ __global__ __launch_bounds__(256) void potrf_leaf_kernel(int nb, T* a, long lda,
       if (w == 3 && q > 0) {
         tri_inv16(S, Y, s_rinv, 16 * (q - 1));
         if (!(q & 1)) {   // join with the block before
+          wave_fence();
           tri_prod<1>(U, S, Y, q - 1, q - 2, q - 2, T(1));
+          wave_fence();
           tri_prod<1>(Y, Y, U, q - 1, q - 2, q - 1, T(-1));
         }
       }

@@ -1,7 +1,9 @@
 // Inverse of a 64x64 lower triangle in LDS: 16x16 blocks by substitution, joins
-// on the matrix cores.  A matrix element (i, k) is at k*(TRI_NB + 1) + i.
+// on the matrix cores.  A matrix element (i, k) is at k*(TRI_NB + 1) + i.  What a
+// wavefront leaves in LDS other lanes of it may read after a wave_fence().
 #pragma once
 #include <hip/hip_runtime.h>
+#include "wave.h"
 
 namespace oba {
 

@@ -174,6 +174,7 @@ __global__ __launch_bounds__(256) void trsm_inv_diag_kernel(long na, const T* __
   __syncthreads();
   if (w < 2) {
     tri_prod<1>(U, S, Y, 2 * w + 1, 2 * w, 2 * w, T(1));
+    wave_fence();
     tri_prod<1>(Y, Y, U, 2 * w + 1, 2 * w, 2 * w + 1, T(-1));
   }
   __syncthreads();
