@@ -77,42 +77,25 @@ __global__ void bzero_kernel(unsigned* p, int n) {
   if (i < n) p[i] = 0u;
 }
 
-// copies operand `which` (0: a, 1: b, 2: c) of every problem from src to dst
-// descriptors (rows x cols, each with its own leading dimension); used to
-// give the tuner scratch copies of in/out operands
+// copies operand a or b of every problem from src to dst descriptors (rows x
+// cols, each with its own leading dimension): scratch copies of in/out operands
+// for the tuner
 template <typename T>
-__global__ void bcopy_kernel(const BDesc* __restrict__ src, const BDesc* __restrict__ dst, int which, int rows_field,
+__global__ void bcopy_kernel(const BDesc* __restrict__ src, const BDesc* __restrict__ dst, bool b_operand, int rows_field,
                              int cols_field) {
   const BDesc& s = src[blockIdx.y];
   const BDesc& d = dst[blockIdx.y];
   const int* fs = &s.m;
   const long rows = fs[rows_field], cols = fs[cols_field];
-  const long lds = which == 2 ? s.ldc : which ? s.ldb : s.lda, ldd = which == 2 ? d.ldc : which ? d.ldb : d.lda;
-  gptr<const T> a = (gptr<const T>)(which == 2 ? s.c : which ? s.b : s.a);
-  gptr<T> b = (gptr<T>)(which == 2 ? d.c : which ? d.b : d.a);
+  const long lds = b_operand ? s.ldb : s.lda, ldd = b_operand ? d.ldb : d.lda;
+  gptr<const T> a = (gptr<const T>)(b_operand ? s.b : s.a);
+  gptr<T> b = (gptr<T>)(b_operand ? d.b : d.a);
   const long total = rows * cols;
   for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < total; e += (long)gridDim.x * blockDim.x) {
     const long i = e % rows, j = e / rows;
     b[i + j * ldd] = a[i + j * lds];
   }
 }
-
-// ---- batched GEMM --------------------------------------------------------------
-template <typename T> struct BMF;
-template <> struct BMF<double> {
-  typedef double acc __attribute__((ext_vector_type(4)));
-  __device__ static inline acc mma(double a, double b, acc c) {
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-  }
-  __device__ static inline int orow(int l, int r) { return 4 * r + (l >> 4); }
-};
-template <> struct BMF<float> {
-  typedef float acc __attribute__((ext_vector_type(4)));
-  __device__ static inline acc mma(float a, float b, acc c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-  }
-  __device__ static inline int orow(int l, int r) { return 4 * (l >> 4) + r; }
-};
 
 // ---- batched Cholesky (n <= 256*RPT) -------------------------------------------
 // LOWER: A = L*L^T with L(i,c) = a[i + c*lda]; upper: A = U^T*U, U = L^T,
@@ -201,7 +184,7 @@ __global__ __launch_bounds__(256) void bpotrf_kernel(const BDesc* __restrict__ d
         // trailing SYRK A22 -= L21 L21^T on MFMA 16x16 tiles of the lower
         // triangle (4 wavefronts, GT tiles each per step, their C elements
         // loaded before the products so one memory latency covers GT tiles)
-        typedef BMF<T> mf;
+        typedef MF<T> mf;
         const int c0 = j0 + w, nr = n - c0;
         if (nr > 0) {
           if (live[0] && row[0] >= c0) {
@@ -600,12 +583,11 @@ int* run_plan(int slot, Launcher L, const Cfg& c, const void* ctx, size_t ctx_by
   return P.info.as<int>();
 }
 
-// Times every candidate config on scratch copies (operand `which` of each
+// Times every candidate config on scratch copies (operand a or b of each
 // problem, rows x cols given by BDesc field indices) and keeps the fastest
-// for this batch signature.
+// for this batch signature (Cholesky and solves).
 Cfg tune(const std::string& sig, const std::vector<Cfg>& cands, Launcher L, const void* ctx,
-         const std::vector<BDesc>& probs, const std::vector<char>& extra, int nitems, int which, int rows_field,
-         int cols_field, size_t elem) {
+         const std::vector<BDesc>& probs, bool b_operand, int rows_field, int cols_field, size_t elem) {
   auto& tt = tuned();
   auto f = tt.find(sig);
   if (f != tt.end()) return f->second;
@@ -619,7 +601,7 @@ Cfg tune(const std::string& sig, const std::vector<Cfg>& cands, Launcher L, cons
     const int* fs = &d.m;
     total += elem * (size_t)std::max(fs[rows_field], 1) * (size_t)std::max(fs[cols_field], 1);
   }
-  DevBuf sbuf(total + 256), tsrc(sizeof(BDesc) * count), tdst(sizeof(BDesc) * count + extra.size() + 16),
+  DevBuf sbuf(total + 256), tsrc(sizeof(BDesc) * count), tdst(sizeof(BDesc) * count),
       ctr(sizeof(unsigned) * BCTR), info(sizeof(int) * (size_t)std::max(count, 1));
   size_t off = 0;
   for (auto& d : scr) {
@@ -627,33 +609,28 @@ Cfg tune(const std::string& sig, const std::vector<Cfg>& cands, Launcher L, cons
     const int rows = std::max(fs[rows_field], 1);
     void* p = sbuf.as<char>() + off;
     off += elem * (size_t)rows * (size_t)std::max(fs[cols_field], 1);
-    if (which == 0) { d.a = p; d.lda = rows; }
-    else if (which == 1) { d.b = p; d.ldb = rows; }
-    else { d.c = p; d.ldc = rows; }
+    if (b_operand) { d.b = p; d.ldb = rows; }
+    else { d.a = p; d.lda = rows; }
   }
   OBA_HIP(hipMemcpyAsync(tsrc.p, probs.data(), sizeof(BDesc) * count, hipMemcpyHostToDevice, r.stream));
   OBA_HIP(hipMemcpyAsync(tdst.p, scr.data(), sizeof(BDesc) * count, hipMemcpyHostToDevice, r.stream));
-  if (!extra.empty())
-    OBA_HIP(hipMemcpyAsync(tdst.as<char>() + sizeof(BDesc) * count, extra.data(), extra.size(), hipMemcpyHostToDevice,
-                           r.stream));
-  const void* dx = extra.empty() ? nullptr : (const void*)(tdst.as<char>() + sizeof(BDesc) * count);
   auto refresh = [&]() {
     if (count == 0) return;
     dim3 g(64, (unsigned)count);
-    if (elem == 8) bcopy_kernel<double><<<g, 256, 0, r.stream>>>(tsrc.as<BDesc>(), tdst.as<BDesc>(), which, rows_field, cols_field);
-    else bcopy_kernel<float><<<g, 256, 0, r.stream>>>(tsrc.as<BDesc>(), tdst.as<BDesc>(), which, rows_field, cols_field);
+    if (elem == 8) bcopy_kernel<double><<<g, 256, 0, r.stream>>>(tsrc.as<BDesc>(), tdst.as<BDesc>(), b_operand, rows_field, cols_field);
+    else bcopy_kernel<float><<<g, 256, 0, r.stream>>>(tsrc.as<BDesc>(), tdst.as<BDesc>(), b_operand, rows_field, cols_field);
   };
   hipEvent_t e0, e1;
   OBA_HIP(hipEventCreate(&e0));
   OBA_HIP(hipEventCreate(&e1));
   refresh();
-  enqueue(L, cands[0], ctx, tdst.as<BDesc>(), dx, nitems, count, ctr.as<unsigned>(), info.as<int>(), r.stream);
+  enqueue(L, cands[0], ctx, tdst.as<BDesc>(), nullptr, 0, count, ctr.as<unsigned>(), info.as<int>(), r.stream);
   float best = 1e30f;
   Cfg bc = cands[0];
   for (const Cfg& c : cands) {
     refresh();
     OBA_HIP(hipEventRecord(e0, r.stream));
-    enqueue(L, c, ctx, tdst.as<BDesc>(), dx, nitems, count, ctr.as<unsigned>(), info.as<int>(), r.stream);
+    enqueue(L, c, ctx, tdst.as<BDesc>(), nullptr, 0, count, ctr.as<unsigned>(), info.as<int>(), r.stream);
     OBA_HIP(hipEventRecord(e1, r.stream));
     OBA_HIP(hipEventSynchronize(e1));
     float ms = 0.f;
@@ -893,9 +870,8 @@ void potrf_batched(bool lower, std::vector<BDesc>& probs, int* info_host) {
     std::vector<Cfg> cands;
     for (int v = 0; v < 2; v++)
       for (int g : {1, 2, 4}) cands.push_back(Cfg{v, g});
-    const std::vector<char> none;
-    Cfg c = tune(signature(BK_POTRF, sizeof(T), ctx[0] * 2 + ctx[1], small), cands, launch_potrf<T>, ctx, small, none,
-                 0, 0, 1, 1, sizeof(T));
+    Cfg c = tune(signature(BK_POTRF, sizeof(T), ctx[0] * 2 + ctx[1], small), cands, launch_potrf<T>, ctx, small, false, 1,
+                 1, sizeof(T));
     double fl = 0, by = 0;
     for (auto& d : small) {
       fl += (double)d.n * d.n * d.n / 3.0;
@@ -923,9 +899,8 @@ void getrs_batched(bool trans, std::vector<BDesc>& probs, int* info_host) {
     const int ctx[2] = {S, trans ? 1 : 0};
     std::vector<Cfg> cands;
     for (int g : {2, 4, 8, 16}) cands.push_back(Cfg{0, g});
-    const std::vector<char> none;
-    Cfg c = tune(signature(BK_GETRS, sizeof(T), ctx[0] * 2 + ctx[1], small), cands, launch_getrs<T>, ctx, small, none,
-                 0, 1, 1, 2, sizeof(T));
+    Cfg c = tune(signature(BK_GETRS, sizeof(T), ctx[0] * 2 + ctx[1], small), cands, launch_getrs<T>, ctx, small, true, 1,
+                 2, sizeof(T));
     double fl = 0, by = 0;
     for (auto& d : small) {
       fl += 2.0 * d.n * d.n * std::max(d.k, 0);

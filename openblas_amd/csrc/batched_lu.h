@@ -26,22 +26,11 @@
 // the trailing matrix), a fourth workgroup per CU 4.0 (spills).
 #pragma once
 #include "lu_key.h"
+#include "wave.h"
 
 namespace oba {
 
 constexpr int BLU_W = 32;
-
-template <typename T> struct BLuMf;
-template <> struct BLuMf<double> {
-  typedef double acc __attribute__((ext_vector_type(4)));
-  __device__ static inline acc mma(double a, double b, acc c) { return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0); }
-  __device__ static inline int orow(int l, int r) { return 4 * r + (l >> 4); }
-};
-template <> struct BLuMf<float> {
-  typedef float acc __attribute__((ext_vector_type(4)));
-  __device__ static inline acc mma(float a, float b, acc c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
-  __device__ static inline int orow(int l, int r) { return 4 * (l >> 4) + r; }
-};
 
 // x[0..N-1] += (u of lanes L0.. of each 16-lane row) * l, the broadcast taken
 // by the FMA itself (DPP row_newbcast): no LDS read and no move per element.
@@ -177,7 +166,7 @@ __global__ __launch_bounds__(64 * NWV, NWV <= 2 ? 2 : 3) void bgetrf_kernel(cons
                                                              int* __restrict__ info_out) {
   constexpr int W = BLU_W, NT = 64 * NWV, LDU = W + 4, CC = NWV < 4 ? 32 * NWV : 128, LDC = CC + 1;
   constexpr int LDD = W + 1, MAXP = NT / W, G = 8;
-  typedef BLuMf<T> mf;
+  typedef MF<T> mf;
   __shared__ T s_c[W * LDC];                // U12 of a column chunk
   __shared__ T s_l[W * LDD];                // strictly lower part of the diagonal block
   __shared__ __attribute__((aligned(16))) T s_u[W * LDU];   // pivot row j, element c: column (j & ~7) + c of the panel

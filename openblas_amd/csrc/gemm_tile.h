@@ -4,29 +4,9 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <type_traits>
+#include "wave.h"
 
 namespace oba {
-
-typedef double d4 __attribute__((ext_vector_type(4)));
-typedef float f4 __attribute__((ext_vector_type(4)));
-
-template <typename T> struct MF;
-template <> struct MF<double> {
-  typedef d4 acc;
-  __device__ static inline acc mma(double a, double b, acc c) {
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-  }
-  // accumulator element r of lane l holds output row 4r + l/16 (measured
-  // lane layout of the f64 16x16x4 instruction), column l%16.
-  __device__ static inline int orow(int l, int r) { return 4 * r + (l >> 4); }
-};
-template <> struct MF<float> {
-  typedef f4 acc;
-  __device__ static inline acc mma(float a, float b, acc c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-  }
-  __device__ static inline int orow(int l, int r) { return 4 * (l >> 4) + r; }
-};
 
 // A vector of V elements at an element-aligned (not 16-byte-aligned) address:
 // global loads and stores of 16 bytes only need 4-byte alignment, so odd

@@ -36,19 +36,6 @@
 //    one XCD was measured no faster (P = 16: 104 against 100 us).
 #pragma once
 
-// the MFMA of the node update inside the panel (lane layouts as in gemm.hip)
-template <typename T> struct LuMf;
-template <> struct LuMf<double> {
-  typedef double acc __attribute__((ext_vector_type(4)));
-  __device__ static inline acc mma(double a, double b, acc c) { return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0); }
-  __device__ static inline int orow(int l, int r) { return 4 * r + (l >> 4); }
-};
-template <> struct LuMf<float> {
-  typedef float acc __attribute__((ext_vector_type(4)));
-  __device__ static inline acc mma(float a, float b, acc c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
-  __device__ static inline int orow(int l, int r) { return 4 * (l >> 4) + r; }
-};
-
 constexpr int L3_NT = 256, L3_NW = 4, L3_RPT = 2, L3_ROWS = L3_NT * L3_RPT;
 constexpr int L3_PMAX = 32;   // workgroups; a wavefront polls up to L3_PMAX / L3_NW records at once
 constexpr unsigned long long L3_EMPTY = ~0ull;
@@ -210,15 +197,15 @@ __global__ __launch_bounds__(L3_NT) void lu_panel3_kernel(T* __restrict__ At, lo
       T fa[W / 4];
 #pragma unroll
       for (int k = 0; k < W / 4; k++) fa[k] = tile[(4 * k + lk) * LDL];
-      typename LuMf<T>::acc acc[2] = {};
+      typename MF<T>::acc acc[2] = {};
 #pragma unroll
       for (int k = 0; k < W / 4; k++)
 #pragma unroll
-        for (int n = 0; n < 2; n++) acc[n] = LuMf<T>::mma(fb[n][k], fa[k], acc[n]);
+        for (int n = 0; n < 2; n++) acc[n] = MF<T>::mma(fb[n][k], fa[k], acc[n]);
 #pragma unroll
       for (int n = 0; n < 2; n++)
 #pragma unroll
-        for (int x = 0; x < 4; x++) tile[(16 * n + LuMf<T>::orow(lane, x)) * LDL] = acc[n][x];
+        for (int x = 0; x < 4; x++) tile[(16 * n + MF<T>::orow(lane, x)) * LDL] = acc[n][x];
     }
     wave_fence();
 #pragma unroll

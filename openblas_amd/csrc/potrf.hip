@@ -56,7 +56,7 @@ template <typename T>
 __global__ __launch_bounds__(256) void potrf_leaf_kernel(int nb, T* a, long lda, bool upper, long j0, int* info,
                                                          T* inv) {
   constexpr int NB = PO_NB, LD = NB + 1;
-  typedef TriMf<T> mf;
+  typedef MF<T> mf;
   __shared__ T S[NB * LD];   // E(i, c) at S[c*LD + i]
   __shared__ T Y[NB * LD];   // L^{-1}(i, c) at Y[c*LD + i]
   __shared__ T U[NB * LD];   // products of the joins

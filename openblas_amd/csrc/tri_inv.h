@@ -9,18 +9,6 @@ namespace oba {
 
 constexpr int TRI_NB = 64;
 
-template <typename T> struct TriMf;
-template <> struct TriMf<double> {
-  typedef double acc __attribute__((ext_vector_type(4)));
-  __device__ static inline acc mma(double a, double b, acc c) { return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0); }
-  __device__ static inline int orow(int l, int r) { return 4 * r + (l >> 4); }
-};
-template <> struct TriMf<float> {
-  typedef float acc __attribute__((ext_vector_type(4)));
-  __device__ static inline acc mma(float a, float b, acc c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
-  __device__ static inline int orow(int l, int r) { return 4 * (l >> 4) + r; }
-};
-
 // lane K of each row of 16 lanes, to all of the row
 template <int K>
 __device__ inline float tri_bcast16(float v) {
@@ -69,7 +57,7 @@ template <int NK, typename T>
 __device__ __attribute__((always_inline)) inline void tri_prod(T* o, const T* x, const T* y, int ri, int ci, int k0,
                                                                  T sign) {
   constexpr int LD = TRI_NB + 1;
-  typedef TriMf<T> mf;
+  typedef MF<T> mf;
   const int lane = threadIdx.x & 63, lr = lane & 15, lg = lane >> 4;
   typename mf::acc acc[2] = {};
 #pragma unroll

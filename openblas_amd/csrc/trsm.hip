@@ -30,17 +30,14 @@ __device__ inline float bcast_lane(float v, int k) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), k));
 }
 
-// Solves E x = b for nvec vectors, E = op(A) (left) or op(A)^T (right),
-// nb <= 64.  Vector v, element i lives at B[i*inc_e + v*inc_v].
-// eT: E(i,k) = A(k,i) (else A(i,k)); elower: E is lower triangular.
-// right-hand-side vectors per wavefront (more workgroups beat interleaved
-// chains: DTRSM 8192 x 1024 3.52 ms with 2, 3.21 ms with 1)
-constexpr int TRSM_VPW = 1;
-
+// Solves E x = b for nvec vectors, E = op(A), nb <= 64.  Element i of vector v
+// lies at B[i + v*ldb].  eT: E(i,k) = A(k,i) (else A(i,k)); elower: E is lower
+// triangular.  A wavefront per vector (two, interleaved, halve the workgroups:
+// DTRSM 8192 x 1024 3.52 ms against 3.21 when its leaves were these).
 template <typename T>
 __global__ __launch_bounds__(256) void trsm_leaf_kernel(int nb, long nvec, const T* __restrict__ A, long lda,
-                                                        T* __restrict__ B, long inc_e, long inc_v, bool eT,
-                                                        bool elower, bool unit, const int* abort_flag) {
+                                                        T* __restrict__ B, long ldb, bool eT, bool elower, bool unit,
+                                                        const int* abort_flag) {
   constexpr int LDE = TRSM_NB + 1;     // padded: conflict-free transposed stores
   __shared__ T E[TRSM_NB * LDE];       // E(i,k) at E[k*LDE + i]
   __shared__ T dinv[TRSM_NB];
@@ -69,57 +66,35 @@ __global__ __launch_bounds__(256) void trsm_leaf_kernel(int nb, long nvec, const
   }
   __syncthreads();
   const int lane = threadIdx.x & 63;
-  const long v0 = ((long)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) * TRSM_VPW;
-  // lane i holds row i of E and its reciprocal pivot in registers; the
-  // wavefront's TRSM_VPW vectors (interleaved chains when more than one)
-  // run through fully unrolled steps (static register indices; a runtime step loop reading E
-  // from LDS inside the chain took ~36 us per 64 x 1024 leaf)
+  const long v = (long)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+  // lane i holds row i of E and its reciprocal pivot in registers; the steps
+  // are unrolled (static register indices; a runtime step loop reading E from
+  // LDS inside the chain took ~36 us per 64 x 1024 leaf)
   T e[TRSM_NB];
 #pragma unroll
   for (int k = 0; k < TRSM_NB; k++) e[k] = E[k * LDE + lane];
   const T di = dinv[lane];
-  T x[TRSM_VPW];
-#pragma unroll
-  for (int vv = 0; vv < TRSM_VPW; vv++) {
-    const long v = v0 + vv;
-    x[vv] = (v < nvec && lane < nb) ? B[v * inc_v + lane * inc_e] : T(0);
-  }
+  T x = (v < nvec && lane < nb) ? B[v * ldb + lane] : T(0);
   if (elower) {
 #pragma unroll
     for (int k = 0; k < TRSM_NB; k++) {
       if (k < nb) {
-        T xk[TRSM_VPW];
-#pragma unroll
-        for (int vv = 0; vv < TRSM_VPW; vv++) {
-          if (lane == k) x[vv] *= di;
-          xk[vv] = bcast_lane(x[vv], k);
-        }
-#pragma unroll
-        for (int vv = 0; vv < TRSM_VPW; vv++)
-          if (lane > k) x[vv] -= e[k] * xk[vv];
+        if (lane == k) x *= di;
+        const T xk = bcast_lane(x, k);
+        if (lane > k) x -= e[k] * xk;
       }
     }
   } else {
 #pragma unroll
     for (int k = TRSM_NB - 1; k >= 0; k--) {
       if (k < nb) {
-        T xk[TRSM_VPW];
-#pragma unroll
-        for (int vv = 0; vv < TRSM_VPW; vv++) {
-          if (lane == k) x[vv] *= di;
-          xk[vv] = bcast_lane(x[vv], k);
-        }
-#pragma unroll
-        for (int vv = 0; vv < TRSM_VPW; vv++)
-          if (lane < k) x[vv] -= e[k] * xk[vv];
+        if (lane == k) x *= di;
+        const T xk = bcast_lane(x, k);
+        if (lane < k) x -= e[k] * xk;
       }
     }
   }
-#pragma unroll
-  for (int vv = 0; vv < TRSM_VPW; vv++) {
-    const long v = v0 + vv;
-    if (v < nvec && lane < nb) B[v * inc_v + lane * inc_e] = x[vv];
-  }
+  if (v < nvec && lane < nb) B[v * ldb + lane] = x;
 }
 
 // Leaves of up to TRSM_RN rows or columns of the triangle in one launch: the
@@ -205,24 +180,12 @@ __global__ __launch_bounds__(256) void trsm_inv_diag_kernel(long na, const T* __
 //     4000 x 2000 1056 -> 461, 739 -> 322.
 constexpr int TRSM_RN = 256;
 
-template <typename T> struct TrMf;
-template <> struct TrMf<double> {
-  typedef double acc __attribute__((ext_vector_type(4)));
-  __device__ static inline acc mma(double a, double b, acc c) { return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0); }
-  __device__ static inline int orow(int l, int r) { return 4 * r + (l >> 4); }
-};
-template <> struct TrMf<float> {
-  typedef float acc __attribute__((ext_vector_type(4)));
-  __device__ static inline acc mma(float a, float b, acc c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
-  __device__ static inline int orow(int l, int r) { return 4 * (l >> 4) + r; }
-};
-
 template <typename T, int RB, bool MT>
 __global__ __launch_bounds__(256) void trsm_right_kernel(int n, long nvec, const T* __restrict__ A, long lda,
                                                          bool upper, const T* __restrict__ inv, T* __restrict__ B,
                                                          long ldb, const int* abort_flag) {
   constexpr int LDX = RB + 2, RT = RB / 16, NB = TRSM_NB;
-  typedef TrMf<T> mf;
+  typedef MF<T> mf;
   __shared__ T Xs[TRSM_RN * LDX];   // X(r, c) at Xs[c*LDX + r]
   __shared__ T Ts[NB * LDX];        // B_b less the products of the solved blocks
   if (abort_flag && *abort_flag) return;
@@ -433,7 +396,7 @@ __global__ __launch_bounds__(256, 2) void trsm_left_kernel(int n, long nvec, con
                                                            bool lower, bool unit, T* __restrict__ B, long ldb,
                                                            const int* abort_flag) {
   constexpr int LDX = RB + 2, RT = RB / 16, NB = TRSM_NB;
-  typedef TrMf<T> mf;
+  typedef MF<T> mf;
   __shared__ T Xs[TRSM_RN * LDX];   // X(k, v) at Xs[k*LDX + v]
   __shared__ T Es[NB * (NB + 1)];   // the diagonal block, an upper one reversed
   __shared__ T s_rinv[TRSM_RN];     // reciprocals of the diagonal
@@ -618,11 +581,8 @@ static void leaf(bool right, bool lower, bool trans, bool unit, long nb, long nr
     return;
   }
   // a left-side triangle of one block
-  const int waves = 4;
-  const long per_block = (long)waves * TRSM_VPW;
-  long blocks = (nrhs + per_block - 1) / per_block;
-  trsm_leaf_kernel<T><<<(unsigned)blocks, 64 * waves, 0, s>>>((int)nb, nrhs, a, lda, b, 1, ldb, trans, elower, unit,
-                                                              abort_flag);
+  trsm_leaf_kernel<T><<<(unsigned)((nrhs + 3) / 4), 256, 0, s>>>((int)nb, nrhs, a, lda, b, ldb, trans, elower, unit,
+                                                                 abort_flag);
   OBA_HIP(hipGetLastError());
 }
 
