@@ -433,7 +433,8 @@ void gemm(bool ta, bool tb, long m, long n, long k, T alpha, const T* a, long ld
   // B 40 times over (normal random data, 64x64x8 / 128x128x8 / 128x128x4, ms):
   // 8192^3 16.43 (17.7 on a card whose memory is slower) / 15.63 / 15.82, 6000^3
   // 6.78 / 6.56 / 6.58, 4000^3 1.97 / 1.98 / 1.94, 6144^2 x 2048 2.25 / 2.28 /
-  // 2.30, 12000^2 x 448 2.00 / 2.20 / 2.12
+  // 2.30, 12000^2 x 448 2.00 / 2.20 / 2.12.  The FP64 form spills 194 to 256
+  // VGPRs around its tail and its stores; the main loop reads none of them back.
   const long m128 = (m + 127) / 128, t128 = tri ? m128 * (m128 + 1) / 2 : m128 * ((n + 127) / 128);
   const long slots = 2 * cu, rounds = (t128 + slots - 1) / slots;
   const bool full128 = !D && tri == 0 && k >= 128 && t128 >= slots && t128 >= (ta && tb ? 0.85 : 0.95) * (double)(rounds * slots);
