@@ -24,7 +24,7 @@
 // alone), the trailing update 25 %, the gathers 13 %.  16-column panels take
 // 5.8 ms instead of 3.9 for the problems above 128 rows (twice the passes over
 // the trailing matrix), a fourth workgroup per CU 4.0 (the FP64 forms of 4 and 8
-// wavefronts spill 5 VGPRs with three, many more with four).
+// wavefronts spill 5 VGPRs with three, more with four).
 #pragma once
 #include "lu_key.h"
 #include "wave.h"
